@@ -117,6 +117,7 @@ struct Request {
   // the caller's or laid out tightly in `yuv` (pinned).
   PinnedBlock yuv;
   bool caller = false;
+  bool row_kernel = false;  // caller planes written by copy_rows (else 2D copies)
   nes_frame_planes planes[kMaxViews] = {}, dplanes[kMaxViews] = {};
   uint64_t rays = 0, samples = 0, batch = 0;
   uint32_t batch_requests = 0, batch_passes = 0;
@@ -124,6 +125,23 @@ struct Request {
 
 static size_t yuv_bytes(const nes_camera &c) {
   return (size_t)c.width * c.height + 2 * (size_t)(c.width / 2) * (c.height / 2);
+}
+
+// Staged planes of a request whose frames go to caller memory: rows 16-byte
+// aligned, as encoder frames are, so that they are copied in 16-byte stores.
+static size_t pitch16(size_t w) { return (w + 15) & ~(size_t)15; }
+static size_t padded_bytes(const nes_camera &c) {
+  return pitch16(c.width) * c.height + 2 * pitch16(c.width / 2) * (c.height / 2);
+}
+static nes_frame_planes padded_planes(uint8_t *p, const nes_camera &c) {
+  nes_frame_planes f;
+  const size_t yp = pitch16(c.width), cp = pitch16(c.width / 2);
+  f.data[0] = p;
+  f.data[1] = p + yp * c.height;
+  f.data[2] = f.data[1] + cp * (c.height / 2);
+  f.linesize[0] = (int32_t)yp;
+  f.linesize[1] = f.linesize[2] = (int32_t)cp;
+  return f;
 }
 
 // Tight YUV420P planes of a w x h frame starting at p.
@@ -206,17 +224,124 @@ static size_t slot_bytes(uint32_t max_rays, int precision, bool depth) {
   return (r * per_ray + cap * per_sample) / 8 * 9 + ((size_t)1 << 20);
 }
 
-// Device-to-host copy of one view's YUV420P planes (tight on the device)
-// into the request's planes.
-static int copy_planes(const nes_frame_planes &dst, const uint8_t *src, const nes_camera &c,
-                       hipStream_t stream) {
-  const nes_frame_planes s = tight_planes(const_cast<uint8_t *>(src), c);
+// Device-to-host copy of one view's staged YUV420P planes into the request's
+// planes, for caller memory the device cannot write.
+static int copy_planes(const nes_frame_planes &dst, const nes_frame_planes &src,
+                       const nes_camera &c, hipStream_t stream) {
   const size_t w[3] = {c.width, c.width / 2, c.width / 2};
   const size_t h[3] = {c.height, c.height / 2, c.height / 2};
   for (int p = 0; p < 3; ++p)
-    NES_HIP_TRY(hipMemcpy2DAsync(dst.data[p], (size_t)dst.linesize[p], s.data[p],
-                                 (size_t)s.linesize[p], w[p], h[p], hipMemcpyDeviceToHost,
+    NES_HIP_TRY(hipMemcpy2DAsync(dst.data[p], (size_t)dst.linesize[p], src.data[p],
+                                 (size_t)src.linesize[p], w[p], h[p], hipMemcpyDeviceToHost,
                                  stream));
+  return NES_OK;
+}
+
+// ------------------------------------------------- rows into pinned memory
+// Caller planes are padded frames whose padding must survive, so they are
+// written row by row.  The runtime's 2D copy (copy engines, no CU) does that
+// well where widths, pitches and addresses are multiples of 4 bytes, but with
+// one transfer per row elsewhere: a 1548x1656 stereo request with its depth
+// stream (chroma rows of 774 bytes) took 60 to 336 ms.  Such requests go
+// through one kernel that stores all their planes straight into the pinned
+// memory (that request: 3.0 ms in all).  It is bound by the PCIe link (56 GB/s),
+// which a few workgroups keep full, so it takes few and leaves the rest of
+// the chip to the next batch's render.  It is not used for aligned requests:
+// eight clients of 640x480 to 2064x2208 took 15.7 ms with it and 15.3 ms with
+// the copy engines, the render running beside it.
+struct RowCopy {
+  const uint8_t *src;
+  uint8_t *dst;
+  uint32_t src_pitch, dst_pitch, width, rows;
+  uint32_t unit;  // bytes per store: 16, 4 or 1, what every row start is aligned to
+};
+constexpr int kRowCopies = 48;  // planes per launch, passed as kernel arguments
+constexpr int kRowCopyBlocks = 4;
+struct RowCopyArgs {
+  RowCopy plane[kRowCopies];
+};
+
+// Elements of `unit` bytes of every row, then the row's last width % unit
+// bytes one by one.
+template <class T>
+__device__ __forceinline__ void copy_row_units(const RowCopy &c) {
+  const uint32_t whole = c.width / (uint32_t)sizeof(T);
+  const uint32_t per_row = whole + c.width % (uint32_t)sizeof(T);
+  const uint32_t step = gridDim.x * blockDim.x;
+  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t row = i / per_row, at = i % per_row;
+  const uint32_t row_step = step / per_row, at_step = step % per_row;
+  while (row < c.rows) {
+    const uint8_t *s = c.src + (size_t)row * c.src_pitch;
+    uint8_t *d = c.dst + (size_t)row * c.dst_pitch;
+    if (at < whole) {
+      reinterpret_cast<T *>(d)[at] = reinterpret_cast<const T *>(s)[at];
+    } else {
+      const uint32_t b = whole * (uint32_t)sizeof(T) + (at - whole);
+      d[b] = s[b];
+    }
+    row += row_step;
+    at += at_step;
+    if (at >= per_row) {
+      at -= per_row;
+      ++row;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void copy_rows(RowCopyArgs a) {
+  const RowCopy c = a.plane[blockIdx.y];
+  if (c.unit == 16)
+    copy_row_units<uint4>(c);
+  else if (c.unit == 4)
+    copy_row_units<uint32_t>(c);
+  else
+    copy_row_units<uint8_t>(c);
+}
+
+// Whether the device can write `rows` rows of `width` bytes, `pitch` apart,
+// at p: all of it inside one pinned allocation that has the same address on
+// both sides (as hipHostMalloc gives it).
+static bool device_writable(const uint8_t *p, size_t width, size_t rows, size_t pitch) {
+  hipPointerAttribute_t at;
+  void *start = nullptr;
+  size_t size = 0;
+  hipDeviceptr_t q = const_cast<uint8_t *>(p);
+  const bool ok = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeHost &&
+                  at.devicePointer == p &&
+                  hipPointerGetAttribute(&start, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, q) == hipSuccess &&
+                  hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, q) == hipSuccess && start;
+  if (!ok) {
+    (void)hipGetLastError();  // an ordinary host pointer is not an error
+    return false;
+  }
+  const uintptr_t a = (uintptr_t)p, lo = (uintptr_t)start;
+  const size_t span = (rows - 1) * pitch + width;
+  return a >= lo && a - lo <= size && size - (a - lo) >= span;
+}
+
+// Whether the runtime's 2D copy takes a plane in whole-word rows.
+static bool rows_word_aligned(const nes_frame_planes &f, const nes_camera &c) {
+  uintptr_t al = c.width | c.width / 2;
+  for (int p = 0; p < 3; ++p) al |= (uintptr_t)f.data[p] | (uintptr_t)f.linesize[p];
+  return al % 4 == 0;
+}
+
+static RowCopy row_copy(const uint8_t *src, size_t src_pitch, uint8_t *dst, size_t dst_pitch,
+                        size_t width, size_t rows) {
+  const uintptr_t al = (uintptr_t)src | (uintptr_t)dst | src_pitch | dst_pitch;
+  return RowCopy{src, dst, (uint32_t)src_pitch, (uint32_t)dst_pitch, (uint32_t)width, (uint32_t)rows,
+                 al % 16 == 0 ? 16u : al % 4 == 0 ? 4u : 1u};
+}
+
+static int launch_row_copies(const std::vector<RowCopy> &copies, hipStream_t stream) {
+  for (size_t i = 0; i < copies.size(); i += kRowCopies) {
+    RowCopyArgs a{};
+    const size_t n = std::min<size_t>(kRowCopies, copies.size() - i);
+    std::copy(copies.begin() + i, copies.begin() + i + n, a.plane);
+    copy_rows<<<dim3(kRowCopyBlocks, (unsigned)n), 256, 0, stream>>>(a);
+    NES_HIP_TRY(hipGetLastError());
+  }
   return NES_OK;
 }
 
@@ -225,8 +350,12 @@ static int launch_output(nes_server *s, Slot &sl) {
   RenderWork &w = sl.work;
   const OutLayout L = out_layout(w.out_px);
   const bool depth = s->cfg.depth_stream != 0;
+  // where each request's staged planes start: tight, as its own planes are
+  // laid out, or with padded rows for caller planes
   size_t yuv_total = 0;
-  for (const nes_camera &c : sl.views) yuv_total += yuv_bytes(c) * (depth ? 2 : 1);
+  for (auto &rq : sl.reqs)
+    for (int v = 0; v < rq->n_views; ++v)
+      yuv_total = pitch16(yuv_total) + (rq->caller ? padded_bytes(rq->views[v]) : yuv_bytes(rq->views[v])) * (depth ? 2 : 1);
   NES_TRY(sl.yuv.reserve(yuv_total + 256));
   if (s->cfg.font && s->cfg.overlay_flags) {
     // the strings of every view, stamped by one launch before frame prep
@@ -247,51 +376,59 @@ static int launch_output(nes_server *s, Slot &sl) {
   const float scale = depth_scale(s->cfg.depth_far);
   size_t off = 0;
   size_t vi = 0;
+  uint8_t *const yuv = sl.yuv.as<uint8_t>();
   for (auto &rq : sl.reqs) {
     for (int v = 0; v < rq->n_views; ++v, ++vi) {
       const nes_camera &c = sl.views[vi];
       const ViewDesc &vd = w.host_views[vi];
       const int cw = (int)c.width, ch = (int)c.height;
       const uint8_t *rgb = w.out.as<uint8_t>() + L.rgb24 + 3 * (size_t)vd.px_base;
-      const nes_frame_planes d = tight_planes(sl.yuv.as<uint8_t>() + off, c);
-      NES_TRY(launch_frameprep(rgb, nullptr, nullptr, nullptr, cw, ch, 1, 0, 0, d.data[0], cw, 0,
-                               d.data[1], cw / 2, 0, d.data[2], cw / 2, 0, s->cfg.sws_mode,
-                               sl.stream));
-      off += yuv_bytes(c);
-      if (depth) {
-        const float *dep = reinterpret_cast<const float *>(w.out.as<uint8_t>() + L.depth) +
-                           vd.px_base;
-        const nes_frame_planes dd = tight_planes(sl.yuv.as<uint8_t>() + off, c);
-        NES_TRY(launch_depth_yuv(dep, cw, ch, scale, nullptr, dd.data[0], cw, dd.data[1], cw / 2,
-                                 dd.data[2], cw / 2, s->cfg.sws_mode, sl.stream));
-        off += yuv_bytes(c);
+      if (rq->caller || v == 0) off = pitch16(off);
+      for (int st = 0; st < (depth ? 2 : 1); ++st) {
+        const nes_frame_planes d = rq->caller ? padded_planes(yuv + off, c) : tight_planes(yuv + off, c);
+        if (st == 0)
+          NES_TRY(launch_frameprep(rgb, nullptr, nullptr, nullptr, cw, ch, 1, 0, 0, d.data[0],
+                                   d.linesize[0], 0, d.data[1], d.linesize[1], 0, d.data[2],
+                                   d.linesize[2], 0, s->cfg.sws_mode, sl.stream));
+        else
+          NES_TRY(launch_depth_yuv(reinterpret_cast<const float *>(w.out.as<uint8_t>() + L.depth) + vd.px_base,
+                                   cw, ch, scale, nullptr, d.data[0], d.linesize[0], d.data[1],
+                                   d.linesize[1], d.data[2], d.linesize[2], s->cfg.sws_mode, sl.stream));
+        off += rq->caller ? padded_bytes(c) : yuv_bytes(c);
       }
     }
   }
   // The server's own planes of a request are laid out exactly as its part
   // of the staging (scene, then depth, per view): one copy per request.
+  // Planes for copy_rows go out in one launch for the whole batch.
   off = 0;
+  std::vector<RowCopy> rows;
   for (auto &rq : sl.reqs) {
-    size_t bytes = 0;
-    for (int v = 0; v < rq->n_views; ++v) bytes += yuv_bytes(rq->views[v]) * (depth ? 2 : 1);
+    off = pitch16(off);
     if (!rq->caller) {
-      NES_HIP_TRY(hipMemcpyAsync(rq->yuv.ptr, sl.yuv.as<uint8_t>() + off, bytes,
-                                 hipMemcpyDeviceToHost, sl.stream));
-    } else {
-      size_t o = off;
-      for (int v = 0; v < rq->n_views; ++v) {
-        const nes_camera &c = rq->views[v];
-        NES_TRY(copy_planes(rq->planes[v], sl.yuv.as<uint8_t>() + o, c, sl.stream));
-        o += yuv_bytes(c);
-        if (depth) {
-          NES_TRY(copy_planes(rq->dplanes[v], sl.yuv.as<uint8_t>() + o, c, sl.stream));
-          o += yuv_bytes(c);
-        }
+      size_t bytes = 0;
+      for (int v = 0; v < rq->n_views; ++v) bytes += yuv_bytes(rq->views[v]) * (depth ? 2 : 1);
+      NES_HIP_TRY(hipMemcpyAsync(rq->yuv.ptr, yuv + off, bytes, hipMemcpyDeviceToHost, sl.stream));
+      off += bytes;
+      continue;
+    }
+    for (int v = 0; v < rq->n_views; ++v) {
+      const nes_camera &c = rq->views[v];
+      for (int st = 0; st < (depth ? 2 : 1); ++st) {
+        const nes_frame_planes src = padded_planes(yuv + off, c);
+        const nes_frame_planes &dst = st ? rq->dplanes[v] : rq->planes[v];
+        if (rq->row_kernel)
+          for (int p = 0; p < 3; ++p)
+            rows.push_back(row_copy(src.data[p], (size_t)src.linesize[p], dst.data[p],
+                                    (size_t)dst.linesize[p], p ? c.width / 2 : c.width,
+                                    p ? c.height / 2 : c.height));
+        else
+          NES_TRY(copy_planes(dst, src, c, sl.stream));
+        off += padded_bytes(c);
       }
     }
-    off += bytes;
   }
-  return NES_OK;
+  return launch_row_copies(rows, sl.stream);
 }
 
 // Take waiting requests (FIFO) that fit one batch.
@@ -495,6 +632,20 @@ static int submit(nes_server *s, uint32_t client, const nes_camera *views, int n
       rq->planes[v] = planes[v];
       if (depth) rq->dplanes[v] = dplanes[v];
     }
+    // rows that are not whole words go through copy_rows where all of them are
+    // pinned memory
+    bool words = true, pinned = true;
+    for (int v = 0; v < n_views; ++v)
+      for (int st = 0; st < (depth ? 2 : 1); ++st)
+        words = words && rows_word_aligned(st ? rq->dplanes[v] : rq->planes[v], views[v]);
+    for (int v = 0; v < n_views && !words && pinned; ++v)
+      for (int st = 0; st < (depth ? 2 : 1) && pinned; ++st)
+        for (int p = 0; p < 3 && pinned; ++p) {
+          const nes_frame_planes &f = st ? rq->dplanes[v] : rq->planes[v];
+          pinned = device_writable(f.data[p], p ? views[v].width / 2 : views[v].width,
+                                   p ? views[v].height / 2 : views[v].height, (size_t)f.linesize[p]);
+        }
+    rq->row_kernel = !words && pinned;
   }
   rq->arrival = Clock::now();
   {

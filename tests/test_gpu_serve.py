@@ -234,3 +234,55 @@ def test_scene_update_under_load_never_mixes_scenes(nes):
         assert same["A"] or same["B"], i
         if i in after:
             assert same[after[i]], (i, after[i])
+
+
+class _Pageable:
+    """Encoder planes in ordinary host memory (the interface of HostPlanes)."""
+
+    def __init__(self, nes, w, h, align):
+        import ctypes as C
+        a = lambda x: (x + align - 1) // align * align
+        self.arrays = [np.full(s, 0xA5, np.uint8)
+                       for s in ((h, a(w)), (h // 2, a(w // 2)), (h // 2, a(w // 2)))]
+        self.widths = (w, w // 2, w // 2)
+        self.planes = nes.FramePlanes()
+        for i, x in enumerate(self.arrays):
+            self.planes.data[i] = x.ctypes.data_as(C.POINTER(C.c_uint8))
+            self.planes.linesize[i] = x.shape[1]
+
+    def yuv(self):
+        return tuple(x[:, :w].copy() for x, w in zip(self.arrays, self.widths))
+
+    def padding_intact(self):
+        return all((x[:, w:] == 0xA5).all() for x, w in zip(self.arrays, self.widths))
+
+    def free(self):
+        pass
+
+
+@pytest.mark.parametrize("w,h,align,pageable", [
+    (258, 66, 32, False),   # rows of 258 and 129 bytes: 16-byte stores and tails
+    (62, 34, 32, False),    # chroma rows shorter than two stores
+    (2, 2, 32, False),      # the smallest frame: one chroma byte
+    (258, 66, 4, False),    # 4-byte stores
+    (258, 66, 2, False),    # single bytes, planes at odd addresses
+    (258, 66, 32, True),    # memory that the device cannot write
+])
+def test_caller_planes_of_any_alignment_match_server_planes(nes, gpu_ctx, w, h, align, pageable):
+    """Frames written into caller planes equal the server's own planes of the
+    same request, for row lengths and alignments of every store width, and the
+    row padding stays as it was."""
+    make = (lambda: _Pageable(nes, w, h, align)) if pageable else (lambda: nes.HostPlanes(w, h, align))
+    with nes.Server(gpu_ctx, max_batch_rays=1 << 16, depth_stream=True) as srv:
+        views = stereo(nes, w, h, 40.0)
+        rc, want, want_d, _ = srv.wait(srv.submit(0, views), depth=True)
+        assert rc == 0
+        planes, dplanes = [make() for _ in views], [make() for _ in views]
+        rc, _, _, _ = srv.wait(srv.submit_into(1, views, planes, dplanes), depth=True)
+        assert rc == 0
+        for got, ref in list(zip(planes, want)) + list(zip(dplanes, want_d)):
+            for g, r in zip(got.yuv(), ref):
+                assert np.array_equal(g, r)
+            assert got.padding_intact()
+        for p in planes + dplanes:
+            p.free()
