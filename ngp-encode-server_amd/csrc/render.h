@@ -51,10 +51,15 @@ constexpr uint32_t kCountMask = 0xffffu;
 //   T < 1e-4 in the pass): [+0] rays that reached T < 1e-4, [+1] samples
 //   those rays composited, [+2] samples evaluated behind that point, [+3]
 //   rays that stopped before the last pass with steps left.
-// The host copy of a pass is one transfer: word 0 or 1 after a pass that is
-// not the last, words [0 or 1, kTotWords) after the last.
-constexpr int kTotCursor = 0, kTotCursorLater = 1, kTotEvaluated = 2, kTotTermBase = 32,
+// Words 4.. hold 64-bit device clock stamps (100 MHz): kStampBegin and
+// kStampEnd of the frame, and per pass (the last pass written for passes
+// beyond two) the starts of its march, encode, MLP and composite.
+// frame_begin clears every word on the device and frame_end stores them all
+// into the host copy.
+constexpr int kTotCursor = 0, kTotCursorLater = 1, kTotEvaluated = 2, kTotStamps = 4, kTotTermBase = 32,
               kTotTermSlots = 32, kTotTermStride = 32;
+constexpr int kStampBegin = 0, kStampEnd = 1, kStampPass = 2, kStampPasses = 2, kStampStages = 4;
+static_assert(kTotStamps + 2 * (kStampPass + kStampPasses * kStampStages) <= kTotTermBase, "stamps");
 constexpr int kTotWords = kTotTermBase + kTotTermSlots * kTotTermStride;
 constexpr size_t kTotBytes = sizeof(uint32_t) * kTotWords;
 
@@ -64,7 +69,6 @@ struct RenderWork {
   DevBuf tinfo;                   // single-pass renders: per ray slot t_start, pixel
   DevBuf gray;                    // GRAY8 depth staging of nes_render_fetch
   uint32_t *total_host = nullptr;  // pinned
-  hipEvent_t ev[12] = {};
   uint32_t n_views = 0, n_slots = 0;
   uint32_t capacity = 0;          // samples the sample buffers hold
   int capacity_precision = -1;    // feature layout the buffers were sized for
@@ -81,6 +85,9 @@ struct RenderWork {
   // samples the first pass gives each ray (kMaxSteps = one single pass).
   uint32_t first_pass_cap = kMaxSteps;
   uint32_t frame_passes = 1;      // passes the last frame launched
+  // Samples of the work area's last frame, first and later pass (0: none yet):
+  // sizes the launches of the next one, whose own count stays on the device.
+  uint32_t last_total[2] = {0, 0};
 };
 
 // What one frame evaluated and composited (for early-termination stats).
@@ -131,12 +138,17 @@ OutLayout out_layout(size_t px);
 int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_t stream);
 int render_prepare_capacity(RenderWork &w, int precision);
 int render_reserve_samples(RenderWork &w, int precision, size_t capacity);
+// Clears the frame counters and uploads the view descriptors of render_setup;
+// precedes the first pass of a frame.
+int render_begin(RenderWork &w, hipStream_t stream);
+// Stores the frame counters and stamps into total_host; follows the last pass
+// (or any pass whose counters the host reads).
+int render_end(RenderWork &w, hipStream_t stream);
 // One pass: march steps [k0, k1) (or, with resume, from where the ray's
 // previous pass stopped), at most `cap` samples per ray, then encode, MLPs
 // and composite.
 int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int k0, int k1,
-                       bool first, bool last, hipStream_t stream, hipEvent_t ev_eval_begin,
-                       hipEvent_t ev_eval_end, hipEvent_t ev_encode_end, uint32_t cap = kMaxSteps,
+                       bool first, bool last, hipStream_t stream, uint32_t cap = kMaxSteps,
                        bool resume = false);
 // A whole frame without a host round trip: one pass when the work area's
 // previous frame composited (almost) every sample it evaluated, else two:
@@ -145,10 +157,7 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
 // The pass totals and composite counters land in total_host (read them after
 // the stream has passed the launches).  Results are bit-identical to a single
 // pass.
-// ev (optional): 8 events recorded per pass p at [4p]: pass start, [4p+1]
-// encode start, [4p+2] encode end, [4p+3] MLP end.
-int render_launch_frame(const SceneDev &scene, RenderWork &w, int precision, hipStream_t stream,
-                        const hipEvent_t *ev = nullptr);
+int render_launch_frame(const SceneDev &scene, RenderWork &w, int precision, hipStream_t stream);
 // After the frame's stream work is complete: the largest pass total (a value
 // above w.capacity means the frame must be launched again after growth) and
 // the counts; updates first_pass_cap for the next frame.
@@ -165,22 +174,25 @@ bool render_growth_fits(const RenderWork &w, int precision, size_t capacity);
 // previous one stopped (bit-identical to one pass; no overflow possible).
 int render_launch_bounded(const SceneDev &scene, RenderWork &w, int precision, hipStream_t stream);
 
-// Workgroups per XCD part of the encode (and of the training scatter) for a
-// sample buffer of `capacity`: about one sample per thread, since the
-// sample count itself stays on the device.  Measured on the stereo 1080p
-// frame: 512 workgroups per part (grid-stride) 2.59 ms, 32768 (about one
-// sample per thread) 2.20 ms.
-inline uint32_t part_blocks(size_t capacity) {
-  const size_t b = (capacity + 255) / 256;
-  return (uint32_t)(b < 512 ? 512 : b > 49152 ? 49152 : b);
+// Workgroups per XCD part of the encode for about `samples` samples: one
+// sample per thread (the kernel strides over the grid where there are more).
+// Measured on the stereo 1080p frame: 512 workgroups per part 2.59 ms, 32768
+// (about one sample per thread) 2.20 ms.  An empty workgroup costs 0.2 ns of
+// dispatch (393216 of them 83 us, 32768 7 us), so the grid follows the
+// expected samples and not the capacity of the buffers.
+inline uint32_t part_blocks(size_t samples) {
+  const size_t b = (samples + 255) / 256;
+  return (uint32_t)(b < 16 ? 16 : b > 49152 ? 49152 : b);
 }
 
 // Single-stage launchers (training step): march_emit over prepared rays,
 // FP32 encode_parts, composite (which always stores the final per-ray state
 // in work.acc for the backward).
 int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStream_t stream);
-int launch_encode_f32(const float *table, RenderWork &w, hipStream_t stream);
-int launch_mlp_f32(const float *weights, RenderWork &w, const uint32_t *n_ptr, hipStream_t stream);
+// (n: the host's sample count, for the launch size.)
+int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t stream);
+int launch_mlp_f32(const float *weights, RenderWork &w, const uint32_t *n_ptr, hipStream_t stream,
+                   uint64_t *stamp = nullptr);
 int launch_composite(RenderWork &w, bool last, hipStream_t stream);
 
 // Enqueue a full render of views on stream; returns after the sample count

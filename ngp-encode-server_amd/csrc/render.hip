@@ -57,9 +57,19 @@ struct MarchArgs {
   int k_begin, k_end, first, packed, resume;
   uint2 *ray_sh;
   uint2 *tinfo;
+  uint64_t *stamp;  // device clock at the kernel's start (optional)
 };
 
+// The device's 100 MHz clock at the start of a kernel, from its first
+// workgroup.  Stage times come from these stamps: hipEventRecord between the
+// kernels costs about 5 us of idle device time each (six of them in a chain of
+// five empty launches: 20 -> 52 us).
+__device__ __forceinline__ void stamp_start(uint64_t *stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+
 __global__ __launch_bounds__(256) void march_emit(MarchArgs m) {
+  stamp_start(m.stamp);
   const ViewDesc *__restrict__ views = m.views;
   const uint32_t n_views = m.n_views, n_slots = m.n_slots;
   const uint32_t *__restrict__ occ = m.occ;
@@ -225,7 +235,8 @@ __device__ __forceinline__ void dense_f32(const float *w, const float *in, float
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mlp_fp32_valu(
     const float4 *__restrict__ pos, const float4 *__restrict__ feat,
     const uint32_t *__restrict__ n_ptr, uint32_t stride, const RayData *__restrict__ rays,
-    const float *__restrict__ Wg, float4 *__restrict__ out) {
+    const float *__restrict__ Wg, float4 *__restrict__ out, uint64_t *stamp) {
+  stamp_start(stamp);
   const uint32_t n = min(*n_ptr, stride);
   __shared__ __attribute__((aligned(16))) float W[kWeights];
   for (int i = (int)threadIdx.x; i < kWeights / 4; i += (int)blockDim.x)
@@ -325,7 +336,8 @@ __global__ __launch_bounds__(256) void encode_parts(const typename PosIn<Tab>::t
                                                     const uint32_t *__restrict__ n_ptr,
                                                     uint32_t stride, const Tab *__restrict__ table,
                                                     typename PartOut<Tab>::type *__restrict__ feat,
-                                                    uint32_t blocks_per_part) {
+                                                    uint32_t blocks_per_part, uint64_t *stamp) {
+  stamp_start(stamp);
   __shared__ uint32_t xch_all[4][256];  // per-wavefront gather exchange (FP16 hashed levels)
   uint32_t *xch = xch_all[threadIdx.x >> 6];
   const uint32_t n = min(*n_ptr, stride);
@@ -354,8 +366,10 @@ __global__ __launch_bounds__(256) void mlp_mixed(const uint32_t *__restrict__ sa
                                                  uint32_t stride,
                                                  const uint2 *__restrict__ ray_sh,
                                                  const half8 *__restrict__ wfrag,
-                                                 uint2 *__restrict__ out) {
+                                                 uint2 *__restrict__ out, uint64_t *stamp) {
+  stamp_start(stamp);
   const uint32_t n = min(*n_ptr, stride);
+  if (blockIdx.x * kEvalWaves * 16 >= n) return;  // no tile for any wave of this workgroup
   __shared__ half8 wl[20 * 64];
   for (int i = (int)threadIdx.x; i < 20 * 64; i += (int)blockDim.x) wl[i] = wfrag[i];
   __syncthreads();
@@ -460,7 +474,8 @@ __global__ __launch_bounds__(256) void composite(
     const uint32_t *__restrict__ counts, const uint32_t *__restrict__ offsets,
     const uint32_t *__restrict__ samples, const SampleOut *__restrict__ sout,
     const uint32_t *__restrict__ n_ptr, uint32_t capacity, int keep, int last, OutPtrs o,
-    const uint2 *__restrict__ tinfo, uint32_t *stats) {
+    const uint2 *__restrict__ tinfo, uint32_t *stats, uint64_t *stamp) {
+  stamp_start(stamp);
   if (*n_ptr > capacity) return;  // overflowed pass: the host re-renders
   const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = lane_id();
@@ -572,6 +587,35 @@ __global__ void zero_u32(uint32_t *p, int n) {
   if (i < n) p[i] = 0u;
 }
 
+// The start of a frame: every counter cleared and up to kArgViews view
+// descriptors stored from the kernel's arguments (a copy from host memory
+// costs 14 us before the first kernel of a small frame).
+constexpr uint32_t kArgViews = 8;
+struct ArgViews {
+  ViewDesc v[kArgViews];
+};
+constexpr int kViewWords = (int)(sizeof(ViewDesc) / sizeof(uint32_t));
+static_assert(sizeof(ViewDesc) % sizeof(uint32_t) == 0, "whole words");
+constexpr int kFrameThreads = 1024;
+
+__global__ __launch_bounds__(kFrameThreads) void frame_begin(uint32_t *total, ArgViews views,
+                                                             uint32_t n_views, ViewDesc *dst) {
+  const int t = (int)threadIdx.x;
+  for (int i = t; i < kTotWords; i += kFrameThreads)
+    if (i != kTotStamps + 2 * kStampBegin && i != kTotStamps + 2 * kStampBegin + 1) total[i] = 0u;
+  if (t < (int)n_views * kViewWords)
+    reinterpret_cast<uint32_t *>(dst)[t] = reinterpret_cast<const uint32_t *>(&views)[t];
+  if (t == 0) reinterpret_cast<uint64_t *>(total + kTotStamps)[kStampBegin] = wall_clock64();
+}
+
+// The end of a frame: the counters and stamps into pinned host memory.
+__global__ __launch_bounds__(kFrameThreads) void frame_end(const uint32_t *total, uint32_t *host) {
+  constexpr int kEnd = kTotStamps + 2 * kStampEnd;
+  for (int i = (int)threadIdx.x; i < kTotWords; i += kFrameThreads)
+    if (i != kEnd && i != kEnd + 1) host[i] = total[i];
+  if (threadIdx.x == 0) reinterpret_cast<uint64_t *>(host + kTotStamps)[kStampEnd] = wall_clock64();
+}
+
 // FP32 expected depth -> the GRAY8 depth plane of the response.
 __global__ void depth_gray8_kernel(const float *__restrict__ depth, size_t n, float scale,
                                    uint8_t *__restrict__ gray) {
@@ -663,11 +707,6 @@ void render_work_free(RenderWork &w) {
   if (w.views_pinned) hipHostFree(w.views_pinned);
   w.views_pinned = nullptr;
   w.views_pinned_cap = 0;
-  for (hipEvent_t &e : w.ev)
-    if (e) {
-      hipEventDestroy(e);
-      e = nullptr;
-    }
 }
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -739,8 +778,7 @@ int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_
   NES_TRY(w.out.reserve(out_layout(px).total));
   NES_TRY(w.total.reserve(kTotBytes));
   if (!w.total_host) NES_HIP_TRY(hipHostMalloc((void **)&w.total_host, kTotBytes));
-  for (hipEvent_t &e : w.ev)
-    if (!e) NES_HIP_TRY(hipEventCreate(&e));
+  if ((uint32_t)n_views <= kArgViews) return NES_OK;  // uploaded by frame_begin
   if (!w.ev_views) NES_HIP_TRY(hipEventCreateWithFlags(&w.ev_views, hipEventDisableTiming));
   NES_HIP_TRY(hipEventSynchronize(w.ev_views));  // the previous upload has read the staging
   if ((uint32_t)n_views > w.views_pinned_cap) {
@@ -808,101 +846,119 @@ static MarchArgs march_args(RenderWork &w, const uint32_t *occ, int k0, int k1, 
   m.resume = resume ? 1 : 0;
   m.ray_sh = nullptr;
   m.tinfo = nullptr;
+  m.stamp = nullptr;
   return m;
 }
 
+int render_begin(RenderWork &w, hipStream_t stream) {
+  ArgViews av{};
+  const uint32_t n = w.n_views <= kArgViews ? w.n_views : 0u;
+  std::copy(w.host_views.begin(), w.host_views.begin() + n, av.v);
+  frame_begin<<<1, kFrameThreads, 0, stream>>>(w.total.as<uint32_t>(), av, n, w.views.as<ViewDesc>());
+  NES_HIP_TRY(hipGetLastError());
+  return NES_OK;
+}
+
+int render_end(RenderWork &w, hipStream_t stream) {
+  frame_end<<<1, kFrameThreads, 0, stream>>>(w.total.as<uint32_t>(), w.total_host);
+  NES_HIP_TRY(hipGetLastError());
+  return NES_OK;
+}
+
+// Samples a pass is expected to have: a little more than the work area's last
+// frame had, at least one per other ray (a view that comes back into sight
+// must not run on a handful of workgroups), and about three per ray slot when
+// nothing is known.  Only launch sizes follow it.
+static size_t expected_samples(const RenderWork &w, int pass) {
+  const size_t last = w.last_total[pass];
+  const size_t est = last ? std::max<size_t>(last + last / 8, w.n_slots / 2) : (size_t)w.n_slots * 3;
+  return std::min<size_t>(est, w.capacity);
+}
+
 int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int k0, int k1,
-                       bool first, bool last, hipStream_t stream, hipEvent_t ev_eval_begin,
-                       hipEvent_t ev_eval_end, hipEvent_t ev_encode_end, uint32_t ray_cap,
-                       bool resume) {
+                       bool first, bool last, hipStream_t stream, uint32_t ray_cap, bool resume) {
   const unsigned blocks = (unsigned)((w.n_slots + 255) / 256);
   uint32_t *const total = w.total.as<uint32_t>();
   uint32_t *cursor = total + (first ? kTotCursor : kTotCursorLater);
   const uint32_t cap = w.capacity;
   // a render in one pass keeps no per-ray state between march and composite
   uint2 *tinfo = first && last ? w.tinfo.as<uint2>() : nullptr;
-  // the frame counters start with the first pass, a later pass's cursor with
-  // that pass
-  zero_u32<<<(kTotWords + 255) / 256, 256, 0, stream>>>(first ? total : cursor, first ? kTotWords : 1);
+  uint64_t *stamp = reinterpret_cast<uint64_t *>(total + kTotStamps) + kStampPass + (first ? 0 : kStampStages);
   MarchArgs m = march_args(w, scene.occ, k0, k1, first, ray_cap, resume);
   m.cursor = cursor;
   m.packed = precision == NES_PRECISION_MIXED ? 1 : 0;
   m.ray_sh = precision == NES_PRECISION_MIXED ? w.ray_sh.as<uint2>() : nullptr;
   m.tinfo = tinfo;
+  m.stamp = stamp;
   march_emit<<<blocks, 256, 0, stream>>>(m);
   NES_HIP_TRY(hipGetLastError());
-  if (ev_eval_begin) NES_HIP_TRY(hipEventRecord(ev_eval_begin, stream));
-  // fixed grids with grid-stride loops: the sample count stays on the device
-  const uint32_t bpp = part_blocks(cap);
+  // grids for the expected samples, with grid-stride loops: the sample count
+  // stays on the device
+  const size_t expect = expected_samples(w, first ? 0 : 1);
+  const uint32_t bpp = part_blocks(expect);
   const bool f32 = precision != NES_PRECISION_MIXED;
   if (f32) {
     encode_parts<float><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<float4>(), cursor, cap,
                                                            scene.table_f32, w.feat.as<float4>(),
-                                                           bpp);
+                                                           bpp, stamp + 1);
     NES_HIP_TRY(hipGetLastError());
-    if (ev_encode_end) NES_HIP_TRY(hipEventRecord(ev_encode_end, stream));
     if (precision == NES_PRECISION_FP32_VALU)
       mlp_fp32_valu<<<256 * 4, 256, 0, stream>>>(w.sample_pos.as<float4>(), w.feat.as<float4>(),
                                                  cursor, cap, w.rays.as<RayData>(),
-                                                 scene.weights_f32, w.sample_out.as<float4>());
+                                                 scene.weights_f32, w.sample_out.as<float4>(),
+                                                 stamp + 2);
     else
-      NES_TRY(launch_mlp_f32(scene.weights_f32, w, cursor, stream));
+      NES_TRY(launch_mlp_f32(scene.weights_f32, w, cursor, stream, stamp + 2));
   } else {
     encode_parts<_Float16><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<uint2>(), cursor,
                                                               cap, scene.table_f16,
-                                                              w.feat.as<uint2>(), bpp);
+                                                              w.feat.as<uint2>(), bpp, stamp + 1);
     NES_HIP_TRY(hipGetLastError());
-    if (ev_encode_end) NES_HIP_TRY(hipEventRecord(ev_encode_end, stream));
-    mlp_mixed<<<256 * 8, 256, 0, stream>>>(w.samples.as<uint32_t>(), w.feat.as<uint2>(), cursor,
+    const unsigned mlp_blocks =
+        (unsigned)std::min<size_t>(256 * 8, std::max<size_t>(expect / (16 * kEvalWaves), 64));
+    mlp_mixed<<<mlp_blocks, 256, 0, stream>>>(w.samples.as<uint32_t>(), w.feat.as<uint2>(), cursor,
                                            cap, w.ray_sh.as<uint2>(),
                                            reinterpret_cast<const half8 *>(scene.wfrag),
-                                           w.sample_out.as<uint2>());
+                                           w.sample_out.as<uint2>(), stamp + 2);
   }
   NES_HIP_TRY(hipGetLastError());
-  if (ev_eval_end) NES_HIP_TRY(hipEventRecord(ev_eval_end, stream));
   const OutPtrs optr = out_ptrs(w);
   uint32_t *stats = w.total.as<uint32_t>();
   if (f32)
     composite<float4><<<blocks, 256, 0, stream>>>(
         w.n_slots, w.rays.as<RayData>(), w.acc.as<RayAcc>(), w.counts.as<uint32_t>(),
         w.offsets.as<uint32_t>(), w.samples.as<uint32_t>(), w.sample_out.as<float4>(), cursor, cap,
-        0, last ? 1 : 0, optr, tinfo, stats);
+        0, last ? 1 : 0, optr, tinfo, stats, stamp + 3);
   else
     composite<uint2><<<blocks, 256, 0, stream>>>(
         w.n_slots, w.rays.as<RayData>(), w.acc.as<RayAcc>(), w.counts.as<uint32_t>(),
         w.offsets.as<uint32_t>(), w.samples.as<uint32_t>(), w.sample_out.as<uint2>(), cursor, cap,
-        0, last ? 1 : 0, optr, tinfo, stats);
+        0, last ? 1 : 0, optr, tinfo, stats, stamp + 3);
   NES_HIP_TRY(hipGetLastError());
-  // one transfer per pass: its cursor, and after the last pass every word
-  // from there on (a copy costs the same few microseconds at any of these
-  // sizes)
-  const size_t at = (size_t)(cursor - total);
-  NES_HIP_TRY(hipMemcpyAsync(w.total_host + at, cursor, last ? 4 * (kTotWords - at) : 4,
-                             hipMemcpyDeviceToHost, stream));
   return NES_OK;
 }
 
-int render_launch_frame(const SceneDev &scene, RenderWork &w, int precision, hipStream_t stream,
-                        const hipEvent_t *ev) {
-  w.total_host[1] = 0;  // no second pass unless launched below
+int render_launch_frame(const SceneDev &scene, RenderWork &w, int precision, hipStream_t stream) {
+  NES_TRY(render_begin(w, stream));
   const uint32_t cap1 = w.first_pass_cap;
-  auto rec = [&](int i) { return ev ? hipEventRecord(ev[i], stream) : hipSuccess; };
-  NES_HIP_TRY(rec(0));
   if (cap1 >= (uint32_t)kMaxSteps) {
     w.frame_passes = 1;
-    return render_launch_pass(scene, w, precision, 0, kMaxSteps, true, true, stream,
-                              ev ? ev[1] : nullptr, ev ? ev[3] : nullptr, ev ? ev[2] : nullptr);
+    NES_TRY(render_launch_pass(scene, w, precision, 0, kMaxSteps, true, true, stream));
+  } else {
+    // two passes, no host round trip between them: the second resumes every
+    // ray the first left above T = 1e-4 at the step after its last sample
+    w.frame_passes = 2;
+    NES_TRY(render_launch_pass(scene, w, precision, 0, kMaxSteps, true, false, stream, cap1, false));
+    NES_TRY(render_launch_pass(scene, w, precision, 0, kMaxSteps, false, true, stream, kMaxSteps, true));
   }
-  // two passes, no host round trip between them: the second resumes every
-  // ray the first left above T = 1e-4 at the step after its last sample
-  w.frame_passes = 2;
-  NES_TRY(render_launch_pass(scene, w, precision, 0, kMaxSteps, true, false, stream,
-                             ev ? ev[1] : nullptr, ev ? ev[3] : nullptr, ev ? ev[2] : nullptr,
-                             cap1, false));
-  NES_HIP_TRY(rec(4));
-  return render_launch_pass(scene, w, precision, 0, kMaxSteps, false, true, stream,
-                            ev ? ev[5] : nullptr, ev ? ev[7] : nullptr, ev ? ev[6] : nullptr,
-                            kMaxSteps, true);
+  return render_end(w, stream);
+}
+
+// A third or later pass counts its samples on the second one's cursor again.
+static int clear_later_cursor(RenderWork &w, hipStream_t stream) {
+  zero_u32<<<1, 64, 0, stream>>>(w.total.as<uint32_t>() + kTotCursorLater, 1);
+  NES_HIP_TRY(hipGetLastError());
+  return NES_OK;
 }
 
 uint32_t render_frame_max_total(const RenderWork &w) {
@@ -919,12 +975,13 @@ int render_launch_bounded(const SceneDev &scene, RenderWork &w, int precision,
   const uint32_t cap = std::min<uint32_t>(w.capacity / std::max<uint32_t>(w.n_slots, 1u),
                                           kMaxSteps);
   const int passes = (int)((kMaxSteps + cap - 1) / cap);
-  w.total_host[1] = 0;
   w.frame_passes = (uint32_t)passes;
-  for (int p = 0; p < passes; ++p)
-    NES_TRY(render_launch_pass(scene, w, precision, 0, kMaxSteps, p == 0, p == passes - 1, stream,
-                               nullptr, nullptr, nullptr, cap, p > 0));
-  return NES_OK;
+  NES_TRY(render_begin(w, stream));
+  for (int p = 0; p < passes; ++p) {
+    if (p > 1) NES_TRY(clear_later_cursor(w, stream));
+    NES_TRY(render_launch_pass(scene, w, precision, 0, kMaxSteps, p == 0, p == passes - 1, stream, cap, p > 0));
+  }
+  return render_end(w, stream);
 }
 
 bool render_growth_fits(const RenderWork &w, int precision, size_t capacity) {
@@ -951,6 +1008,9 @@ size_t sample_buffer_bytes(size_t capacity, int precision) {
 FrameCounts render_frame_finish(RenderWork &w) {
   FrameCounts c;
   c.passes = w.frame_passes;
+  // frames in more passes (bounded, windows) say nothing about a whole one
+  w.last_total[0] = c.passes <= 2 ? w.total_host[kTotCursor] : 0u;
+  w.last_total[1] = c.passes == 2 ? w.total_host[kTotCursorLater] : 0u;
   c.evaluated = w.total_host[2];
   for (int s = 0; s < kTotTermSlots; ++s) {
     const uint32_t *t = w.total_host + kTotTermBase + kTotTermStride * s;
@@ -984,11 +1044,11 @@ int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStr
   return NES_OK;
 }
 
-int launch_encode_f32(const float *table, RenderWork &w, hipStream_t stream) {
-  const uint32_t bpp = part_blocks(w.capacity);
+int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t stream) {
+  const uint32_t bpp = part_blocks(n);
   encode_parts<float><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<float4>(),
                                                          w.total.as<uint32_t>(), w.capacity,
-                                                         table, w.feat.as<float4>(), bpp);
+                                                         table, w.feat.as<float4>(), bpp, nullptr);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }
@@ -999,7 +1059,7 @@ int launch_composite(RenderWork &w, bool last, hipStream_t stream) {
                                                w.counts.as<uint32_t>(), w.offsets.as<uint32_t>(),
                                                w.samples.as<uint32_t>(), w.sample_out.as<float4>(),
                                                w.total.as<uint32_t>(), w.capacity, 1, last ? 1 : 0,
-                                               out_ptrs(w), nullptr, nullptr);
+                                               out_ptrs(w), nullptr, nullptr, nullptr);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }
@@ -1058,17 +1118,27 @@ static bool valid_precision(int p) {
   return p == NES_PRECISION_FP32 || p == NES_PRECISION_MIXED || p == NES_PRECISION_FP32_VALU;
 }
 
-// Stage times of one pass from its four events and the event that follows it.
-static void add_pass_times(const hipEvent_t *ev, hipEvent_t next, double t[4]) {
-  float a = 0, b = 0, c = 0, d = 0;
-  hipEventElapsedTime(&a, ev[0], ev[1]);
-  hipEventElapsedTime(&b, ev[1], ev[2]);
-  hipEventElapsedTime(&c, ev[2], ev[3]);
-  hipEventElapsedTime(&d, ev[3], next);
-  t[0] += a;  // march
-  t[1] += b;  // encode
-  t[2] += c;  // MLPs
-  t[3] += d;  // composite
+// Milliseconds per tick of the device clock.
+static double tick_ms() {
+  static const double ms = [] {
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, 0) != hipSuccess || khz <= 0) khz = 100000;
+    return 1.0 / khz;
+  }();
+  return ms;
+}
+
+// Stage times of `passes` passes from the stamps of the last frame_end:
+// t[0..3] += march, encode, MLPs, composite; returns begin to end.
+static double add_stage_times(const RenderWork &w, int first_pass, int passes, double t[4]) {
+  const uint64_t *st = reinterpret_cast<const uint64_t *>(w.total_host + kTotStamps);
+  auto ms = [](uint64_t a, uint64_t b) { return b > a ? (double)(b - a) * tick_ms() : 0.0; };
+  for (int p = first_pass; p < first_pass + passes; ++p) {
+    const uint64_t *s = st + kStampPass + p * kStampStages;
+    const uint64_t next = p + 1 < first_pass + passes ? s[kStampStages] : st[kStampEnd];
+    for (int k = 0; k < kStampStages; ++k) t[k] += ms(s[k], k + 1 < kStampStages ? s[k + 1] : next);
+  }
+  return ms(st[kStampBegin], st[kStampEnd]);
 }
 
 static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precision,
@@ -1079,23 +1149,19 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
   NES_TRY(render_prepare_capacity(w, precision));
   NES_TRY(check_budget(w));
   double t[4] = {0, 0, 0, 0};  // march, encode, MLPs, composite
+  double total = 0;
   FrameCounts fc;
-  hipEvent_t *ev = w.ev + 1, end = w.ev[9];
-  NES_HIP_TRY(hipEventRecord(w.ev[0], stream));
   if (steps_per_pass == 0 || steps_per_pass >= kMaxSteps) {
     // whole frame: one pass, or two when the previous frame of this work area
     // evaluated samples behind terminated rays (steps_per_pass 0)
     if (steps_per_pass) w.first_pass_cap = kMaxSteps;
     bool bounded = false;
     for (int attempt = 0;; ++attempt) {
-      if (bounded) {
-        NES_HIP_TRY(hipEventRecord(ev[0], stream));
+      if (bounded)
         NES_TRY(render_launch_bounded(scene, w, precision, stream));
-      } else {
-        NES_TRY(render_launch_frame(scene, w, precision, stream, ev));
-      }
-      NES_HIP_TRY(hipEventRecord(end, stream));
-      NES_HIP_TRY(hipEventSynchronize(end));
+      else
+        NES_TRY(render_launch_frame(scene, w, precision, stream));
+      NES_HIP_TRY(hipStreamSynchronize(stream));
       const uint32_t n = render_frame_max_total(w);
       if (bounded || n <= w.capacity) break;
       if (attempt > 0) {
@@ -1110,12 +1176,10 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
         bounded = true;
     }
     if (bounded) {
-      float a = 0;
-      hipEventElapsedTime(&a, ev[0], end);
-      t[1] += a;  // no per-stage events over bounded passes
+      double unused[4] = {0, 0, 0, 0};
+      total = t[1] = add_stage_times(w, 0, 1, unused);  // no per-stage times over bounded passes
     } else {
-      add_pass_times(ev, w.frame_passes > 1 ? ev[4] : end, t);
-      if (w.frame_passes > 1) add_pass_times(ev + 4, end, t);
+      total = add_stage_times(w, 0, (int)w.frame_passes, t);
     }
     fc = render_frame_finish(w);
   } else {
@@ -1127,11 +1191,13 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
       const int k0 = p * spp, k1 = std::min(kMaxSteps, k0 + spp);
       uint32_t n = 0;
       for (int attempt = 0;; ++attempt) {
-        NES_HIP_TRY(hipEventRecord(ev[0], stream));
-        NES_TRY(render_launch_pass(scene, w, precision, k0, k1, p == 0, p == passes - 1, stream,
-                                   ev[1], ev[3], ev[2]));
-        NES_HIP_TRY(hipEventRecord(end, stream));
-        NES_HIP_TRY(hipEventSynchronize(end));
+        if (p == 0)
+          NES_TRY(render_begin(w, stream));
+        else
+          NES_TRY(clear_later_cursor(w, stream));
+        NES_TRY(render_launch_pass(scene, w, precision, k0, k1, p == 0, p == passes - 1, stream));
+        NES_TRY(render_end(w, stream));
+        NES_HIP_TRY(hipStreamSynchronize(stream));
         n = w.total_host[p == 0 ? 0 : 1];
         if (n <= w.capacity) break;
         if (attempt > 0) {
@@ -1145,14 +1211,12 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
         }
         NES_TRY(render_reserve_samples(w, precision, want));
       }
-      add_pass_times(ev, end, t);
+      total = add_stage_times(w, p == 0 ? 0 : 1, 1, t);
     }
     w.frame_passes = (uint32_t)passes;
     fc = render_frame_finish(w);
     w.first_pass_cap = kMaxSteps;  // windows are the caller's choice, not learned from
   }
-  float total = 0;
-  hipEventElapsedTime(&total, w.ev[0], end);
   if (stats) {
     stats->rays = w.out_px;
     stats->samples = fc.evaluated;

@@ -66,6 +66,7 @@ struct TrainMlpArgs {
   const float4 *dout;       // bwd: (dL/dlogsigma, dL/dpre_r, _g, _b)
   float4 *dfeat;            // bwd: [8][stride] records of 2 float4: (position, 0), dL/dfeature
   float *grad_w;            // bwd: 9344
+  uint64_t *stamp;          // fwd: device clock at the start (optional)
 };
 
 // LDS copy of the weights: row strides S1..S5 words, matrices at P1..P5.
@@ -99,6 +100,7 @@ __global__ __launch_bounds__(256) void mlp_train(TrainMlpArgs a) {
   using WL = WLayout<kBwd>;
   constexpr int kS1 = WL::S1, kS2 = WL::S2, kS3 = WL::S3, kS4 = WL::S4, kS5 = WL::S5;
   constexpr int kP1 = WL::P1, kP2 = WL::P2, kP3 = WL::P3, kP4 = WL::P4, kP5 = WL::P5;
+  if (!kBwd && a.stamp && blockIdx.x == 0 && threadIdx.x == 0) *a.stamp = wall_clock64();
   __shared__ float W[WL::kSize];
   __shared__ float dW[kBwd ? kWeights : 1];
   __shared__ float tr_d[kBwd ? kTrainWaves : 1][64][17];
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(256) void mlp_train(TrainMlpArgs a) {
 // FP32 forward over the work area's sample list (the FP32 render path and the
 // training forward): density + colour MLPs on v_mfma_f32_16x16x4_f32.
 int nes::launch_mlp_f32(const float *weights, RenderWork &w, const uint32_t *n_ptr,
-                        hipStream_t stream) {
+                        hipStream_t stream, uint64_t *stamp) {
   TrainMlpArgs ma{};
   ma.pos = w.sample_pos.as<float4>();
   ma.feat = w.feat.as<float4>();
@@ -369,6 +371,7 @@ int nes::launch_mlp_f32(const float *weights, RenderWork &w, const uint32_t *n_p
   ma.rays = w.rays.as<RayData>();
   ma.weights = weights;
   ma.out = w.sample_out.as<float4>();
+  ma.stamp = stamp;
   mlp_train<false><<<256 * 2, 256, 0, stream>>>(ma);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
@@ -987,7 +990,7 @@ static int trainer_forward(nes_trainer *t, uint32_t n_rays, const TrainRayArgs &
       NES_TRY(trainer_grow(t, (size_t)n + n / 8 + 1024));
       continue;
     }
-    NES_TRY(launch_encode_f32(t->params, w, s));
+    NES_TRY(launch_encode_f32(t->params, w, n, s));
     NES_TRY(launch_mlp_f32(t->params + t->n_table, w, w.total.as<uint32_t>(), s));
     NES_TRY(launch_composite(w, true, s));
     return NES_OK;

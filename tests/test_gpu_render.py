@@ -304,3 +304,20 @@ def test_budget_renders_in_bounded_passes(nes, oracle, prec):
     assert sref.passes == 1 and st.passes > 2 and st.samples == sref.samples
     for k in ("rgb", "depth", "n_samples", "rgb24"):
         assert np.array_equal(ref[k], got[k]), k
+
+
+@pytest.mark.parametrize("n", [1, 8, 9])
+def test_view_batches_match_single_views(nes, gpu_ctx, n):
+    """Up to 8 view descriptors travel as kernel arguments, more through an
+    upload: every view of a batch equals the view rendered alone, also after a
+    frame with no samples (which sizes the next frame's launches)."""
+    views = [nes.camera(40 + 3 * i, 33 + i, nes.orbit_camera(40.0 * i, 10.0 + 2 * i)) for i in range(n)]
+    away = nes.camera(40, 33, nes.orbit_camera(0.0, 10.0, 2.0, 50.0))  # the cube is out of view
+    batch, st = gpu_ctx.render(views)
+    assert st.ms_total > 0 and st.ms_encode > 0 and st.ms_march > 0
+    for v, got in zip(views, batch):
+        empty, st = gpu_ctx.render(away)
+        assert st.samples == 0 and not empty[0]["rgb24"].any()
+        (alone,), _ = gpu_ctx.render(v)
+        for k in got:
+            assert np.array_equal(got[k], alone[k]), k
