@@ -55,22 +55,24 @@ __device__ __forceinline__ uint32_t ray_box(const float o[3], const float d[3],
   const float ts = tn > 0.0f ? tn : 0.0f;
   *t_start = ts;
   if (!(tf > ts)) return 0;
-  uint32_t n = 0;
-  while (n < (uint32_t)kMaxSteps && step_t((int)n, ts) < tf) ++n;
-  return n;
+  // The first n with step_t(n) >= tf.  step_t grows with n, so an estimate is
+  // moved to it by a step or two (counting up from 0 took a ray through the
+  // cube about 70 iterations).
+  int n = min(max((int)fmaf(tf - ts, 1.0f / kDelta, 0.5f), 0), kMaxSteps);
+  while (n < kMaxSteps && step_t(n, ts) < tf) ++n;
+  while (n > 0 && !(step_t(n - 1, ts) < tf)) --n;
+  return (uint32_t)n;
 }
 
-// Occupancy cell of a position (clamped to the grid, so any position gives
-// an index inside the bitfield).
-__device__ __forceinline__ uint32_t occ_cell(const float x[3]) {
+// Occupancy cell of a position scaled by the grid resolution (clamped to the
+// grid, so any position gives an index inside the bitfield).
+__device__ __forceinline__ uint32_t occ_cell(const float x128[3]) {
   int c[3];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const int ci = (int)floorf(x[a] * 128.0f);
-    c[a] = min(max(ci, 0), kOccRes - 1);
-  }
-  return (uint32_t)(c[0] + kOccRes * (c[1] + kOccRes * c[2]));
+  for (int a = 0; a < 3; ++a) c[a] = min(max((int)floorf(x128[a]), 0), kOccRes - 1);
+  return (uint32_t)(c[0] | (c[1] << 7) | (c[2] << 14));
 }
+static_assert(kOccRes == 1 << 7, "cell index");
 
 __device__ __forceinline__ void step_pos(const RayData &r, int k, float x[3],
                                          float *t) {
@@ -413,10 +415,11 @@ __device__ __forceinline__ const char *level_base(const Tab *table) {
 // reads every position, so this halves the encode's position stream; the
 // rounding (at most 2^-22) moves a level-15 interpolation weight by at most
 // 2048 * 2^-22 = 4.9e-4, below the FP16 table's own rounding.
-__device__ __forceinline__ uint2 pack_pos21(const float x[3]) {
+// x21: the position times 2^21, not yet clamped.
+__device__ __forceinline__ uint2 pack_pos21(const float x21[3]) {
   uint32_t q[3];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) q[a] = min(__float2uint_rn(x[a] * 2097152.0f), 2097151u);
+  for (int a = 0; a < 3; ++a) q[a] = __float2uint_rn(fminf(fmaxf(x21[a], 0.0f), 2097151.0f));
   return make_uint2(q[0] | (q[1] << 21), (q[1] >> 11) | (q[2] << 10));
 }
 

@@ -11,11 +11,13 @@ namespace nes {
 // out tile-major so that a wavefront's 64 rays are a compact screen block.
 struct ViewDesc {
   float c2w[12];
-  float focal;
+  float focal, inv_focal;
   uint32_t width, height, tiles_x;
   uint32_t slot_base, slot_count;  // global ray-slot range of the view
   uint32_t px_base;                // offset of the view in the output arrays
-  uint32_t pad;
+  // Bound on how far a pixel's unnormalised direction lies from its tile
+  // centre's (march_emit's tile test).
+  float tile_reach;
 };
 
 struct RayData {  // 32 bytes
@@ -30,16 +32,21 @@ struct RayAcc {  // 32 bytes, compositing state carried across passes
   uint32_t n_samples;
   uint32_t done;
   uint32_t pad;
-};
+};  // written for rays that have samples only
 
 // Sample record: ray slot in the high 25 bits, step index in the low 7.
 constexpr uint32_t kMaxSlots = 1u << 25;
 // View descriptors the pinned upload staging holds before it grows.
 constexpr uint32_t kPinnedViews = 64;
 
-// Per ray slot, the march writes counts[slot] = samples emitted by the pass in
-// the low 16 bits and the step the next pass resumes at in the high 16 bits.
-constexpr uint32_t kCountMask = 0xffffu;
+// Per ray slot, the march writes counts[slot]: samples emitted by the pass in
+// the low 8 bits (at most kMaxSteps), the flags of earlier passes, and the step
+// the next pass resumes at in the high 16 bits.  The composite of a pass that
+// is not the last adds kRayState for rays whose RayAcc it stored and kRayDone
+// for those that reached T < 1e-4.
+// offsets[wavefront] is the start of the wavefront's sample range.
+constexpr uint32_t kCountMask = 0xffu, kRayState = 0x100u, kRayDone = 0x200u;
+static_assert(kMaxSteps <= (int)kCountMask, "a ray's samples fit its count");
 
 // Words of RenderWork::total (device) and RenderWork::total_host (pinned),
 // the same layout on both sides:
@@ -63,10 +70,12 @@ static_assert(kTotStamps + 2 * (kStampPass + kStampPasses * kStampStages) <= kTo
 constexpr int kTotWords = kTotTermBase + kTotTermSlots * kTotTermStride;
 constexpr size_t kTotBytes = sizeof(uint32_t) * kTotWords;
 
+inline size_t wavefronts(size_t slots) { return (slots + 63) / 64; }
+
 struct RenderWork {
   DevBuf views, rays, acc, counts, offsets, samples, sample_out, sample_pos, feat, out, total;
   DevBuf ray_sh;                  // mixed path: per ray slot 16 FP16 SH values
-  DevBuf tinfo;                   // single-pass renders: per ray slot t_start, pixel
+  DevBuf t_start;                 // per ray slot that has samples: t_start
   DevBuf gray;                    // GRAY8 depth staging of nes_render_fetch
   uint32_t *total_host = nullptr;  // pinned
   uint32_t n_views = 0, n_slots = 0;
@@ -186,14 +195,14 @@ inline uint32_t part_blocks(size_t samples) {
 }
 
 // Single-stage launchers (training step): march_emit over prepared rays,
-// FP32 encode_parts, composite (which always stores the final per-ray state
-// in work.acc for the backward).
+// FP32 encode_parts, composite (which stores the final state of rays that have
+// samples in work.acc for the backward; ray slot i is output i).
 int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStream_t stream);
 // (n: the host's sample count, for the launch size.)
 int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t stream);
 int launch_mlp_f32(const float *weights, RenderWork &w, const uint32_t *n_ptr, hipStream_t stream,
                    uint64_t *stamp = nullptr);
-int launch_composite(RenderWork &w, bool last, hipStream_t stream);
+int launch_composite(RenderWork &w, hipStream_t stream);
 
 // Enqueue a full render of views on stream; returns after the sample count
 // read-backs (one host sync per pass).  Outputs land in work.out.

@@ -386,7 +386,6 @@ struct TrainRayArgs {
   uint64_t seed, step;
   const float *targets;  // [pose][H][W][3]
   RayData *rays;
-  RayAcc *acc;
   float *target;         // [ray][3]
   const float *ray_o;    // explicit rays (optional)
   const float *ray_d;
@@ -423,11 +422,6 @@ __global__ void train_rays(TrainRayArgs a) {
   }
   r.n_steps = ray_box(r.o, r.d, &r.t_start);
   a.rays[i] = r;
-  RayAcc c;
-  c.T = 1.0f; c.r = c.g = c.b = 0.0f; c.depth = 0.0f; c.n_samples = 0;
-  c.done = r.n_steps == 0;
-  c.pad = i;
-  a.acc[i] = c;
 }
 
 // Loss = mean over rays and channels of (C - target)^2; dC = dL/dC.
@@ -493,16 +487,15 @@ __global__ __launch_bounds__(256) void train_dcomposite(
   float g[3] = {0.0f, 0.0f, 0.0f};
   if (valid) {
     cnt = counts[slot] & kCountMask;
-    base = offsets[slot];
+    base = offsets[slot >> 6];  // (not written, and not used, where no lane has samples)
     if (cnt) {
-      const RayAcc a = acc[slot];
-      used = min(cnt, a.n_samples);
-      g[0] = dC[3 * a.pad + 0];
-      g[1] = dC[3 * a.pad + 1];
-      g[2] = dC[3 * a.pad + 2];
+      used = min(cnt, acc[slot].n_samples);
+      g[0] = dC[3 * slot + 0];
+      g[1] = dC[3 * slot + 1];
+      g[2] = dC[3 * slot + 2];
     }
   }
-  base = __shfl(base, 0);  // lane 0 is valid whenever any lane is
+  base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);  // lane 0 is valid whenever any lane is
   const uint32_t mx = wave_max(cnt);
   const uint64_t below = lanes_below(lane);
   // front to back over the ray's samples (rank-major positions)
@@ -947,7 +940,8 @@ static int trainer_prepare(nes_trainer *t, uint32_t n_rays) {
   NES_TRY(w.rays.reserve(sizeof(RayData) * n_rays));
   NES_TRY(w.acc.reserve(sizeof(RayAcc) * n_rays));
   NES_TRY(w.counts.reserve(sizeof(uint32_t) * n_rays));
-  NES_TRY(w.offsets.reserve(sizeof(uint32_t) * n_rays));
+  NES_TRY(w.t_start.reserve(sizeof(float) * n_rays));
+  NES_TRY(w.offsets.reserve(sizeof(uint32_t) * wavefronts(n_rays)));
   NES_TRY(w.out.reserve(out_layout(n_rays).total));
   NES_TRY(w.total.reserve(kTotBytes));
   NES_TRY(w.views.reserve(sizeof(ViewDesc)));
@@ -992,7 +986,7 @@ static int trainer_forward(nes_trainer *t, uint32_t n_rays, const TrainRayArgs &
     }
     NES_TRY(launch_encode_f32(t->params, w, n, s));
     NES_TRY(launch_mlp_f32(t->params + t->n_table, w, w.total.as<uint32_t>(), s));
-    NES_TRY(launch_composite(w, true, s));
+    NES_TRY(launch_composite(w, s));
     return NES_OK;
   }
   set_last_error("training sample buffers could not be grown");
@@ -1041,7 +1035,6 @@ static TrainRayArgs step_rays(nes_trainer *t, uint64_t step) {
   ra.step = step;
   ra.targets = t->targets;
   ra.rays = t->work.rays.as<RayData>();
-  ra.acc = t->work.acc.as<RayAcc>();
   ra.target = t->target;
   return ra;
 }
@@ -1248,7 +1241,6 @@ static int trainer_forward_rays(nes_trainer *t, const float *ray_o, const float 
   TrainRayArgs ra{};
   ra.n_rays = n;
   ra.rays = t->work.rays.as<RayData>();
-  ra.acc = t->work.acc.as<RayAcc>();
   ra.ray_o = t->xo.as<float>();
   ra.ray_d = t->xd.as<float>();
   return trainer_forward(t, n, ra);

@@ -321,3 +321,27 @@ def test_view_batches_match_single_views(nes, gpu_ctx, n):
         (alone,), _ = gpu_ctx.render(v)
         for k in got:
             assert np.array_equal(got[k], alone[k]), k
+
+
+@pytest.mark.parametrize("radius,fov", [(0.3, 100.0), (0.9, 20.0), (2.0, 5.0), (2.0, 160.0), (40.0, 3.0)])
+def test_tiles_outside_the_cube_match_oracle_sample_counts(nes, oracle, scene1, radius, fov):
+    """The march leaves out tiles that cannot see the cube: with every cell
+    occupied, each pixel's sample count equals the oracle's for eyes inside,
+    beside and far from the cube, narrow and wide views, and camera axes that
+    are not orthonormal."""
+    t, w, _ = scene1
+    occ = np.full(nes.OCC_WORDS, 0xffffffff, np.uint32)
+    w = w.copy()
+    w[2048:2048 + 64] = 0.0  # density 1: no ray ends early
+    m = np.array(nes.orbit_camera(25.0, 15.0, radius, 0.1), np.float32)
+    skew = m.copy()
+    skew[0::4] *= 1.7
+    skew[1::4] += 0.3 * skew[0::4]
+    with nes.Context(t, w, occ) as ctx:
+        for c2w in (m, skew):
+            v = nes.camera(101, 67, c2w, fov=fov)
+            (out,), _ = ctx.render(v, precision=nes.PRECISION_FP32)
+            ocam = oracle.camera(101, 67, c2w, fov=fov)
+            _, _, ns = oracle.render_pixels(t, w, occ, ocam, np.arange(101 * 67, dtype=np.uint32),
+                                            threads=8)
+            assert np.array_equal(out["n_samples"].reshape(-1), ns)
