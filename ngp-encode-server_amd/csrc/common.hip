@@ -51,6 +51,23 @@ int ensure_device() {
 
 hipStream_t library_stream() { return g_stream; }
 
+bool device_writable(const void *p, size_t bytes) {
+  if (!p || !bytes) return false;
+  unsigned type = 0;
+  void *dev = nullptr, *start = nullptr;
+  size_t size = 0;
+  hipPointer_attribute what[4] = {HIP_POINTER_ATTRIBUTE_MEMORY_TYPE, HIP_POINTER_ATTRIBUTE_DEVICE_POINTER,
+                                  HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, HIP_POINTER_ATTRIBUTE_RANGE_SIZE};
+  void *to[4] = {&type, &dev, &start, &size};
+  if (hipDrvPointerGetAttributes(4, what, to, const_cast<void *>(p)) != hipSuccess) {
+    (void)hipGetLastError();  // an ordinary host pointer is not an error
+    return false;
+  }
+  const uintptr_t a = (uintptr_t)p, lo = (uintptr_t)start;
+  return type == (unsigned)hipMemoryTypeHost && dev == p && start && a >= lo && a - lo <= size &&
+         size - (a - lo) >= bytes;
+}
+
 int DevBuf::reserve(size_t need) {
   if (need <= bytes) return NES_OK;
   release();

@@ -134,6 +134,11 @@ int get_dev_vfilter(int h, DevVFilter *out);
 
 hipStream_t library_stream();
 
+// Whether kernels can write [p, p + bytes): all of it inside one pinned host
+// allocation with the same address on both sides (as hipHostMalloc gives it).
+// Asked anew for every call: nothing is remembered about a caller's memory.
+bool device_writable(const void *p, size_t bytes);
+
 int launch_frameprep(const uint8_t *rgb_a, const float *depth_a,
                      const uint8_t *rgb_b, const float *depth_b, int w, int h,
                      int n_frames, size_t rgb_frame_bytes,

@@ -70,18 +70,42 @@ static_assert(kTotStamps + 2 * (kStampPass + kStampPasses * kStampStages) <= kTo
 constexpr int kTotWords = kTotTermBase + kTotTermSlots * kTotTermStride;
 constexpr size_t kTotBytes = sizeof(uint32_t) * kTotWords;
 
+// One output array on its way to pinned host memory: src (device, 16-byte
+// aligned) to dst, `bytes` long, bpp bytes per pixel of view `view`.  With a
+// gray_scale the source is FP32 depth, stored as the GRAY8 plane.
+struct HostArray {
+  const uint8_t *src;
+  uint8_t *dst;
+  uint64_t bytes;
+  uint32_t bpp, view;
+  uint32_t unit;  // bytes per store: 16, 4 or 1, what dst is aligned to
+  float gray_scale;
+};
+constexpr uint32_t kHostArrays = 40;  // carried to the device as kernel arguments
+
 inline size_t wavefronts(size_t slots) { return (slots + 63) / 64; }
+
+// Views start on this pixel in the output arrays, so that every array of every
+// view starts on 16 bytes.
+constexpr size_t kViewAlign = 64;
 
 struct RenderWork {
   DevBuf views, rays, acc, counts, offsets, samples, sample_out, sample_pos, feat, out, total;
   DevBuf ray_sh;                  // mixed path: per ray slot 16 FP16 SH values
   DevBuf t_start;                 // per ray slot that has samples: t_start
   DevBuf gray;                    // GRAY8 depth staging of nes_render_fetch
+  DevBuf tile_n;                  // per wavefront of ray slots: samples of the first pass
+  DevBuf host_arrays;             // device copy of host_out
+  HostArray host_out[kHostArrays];  // outputs the frame stores into host memory itself
+  uint32_t n_host_out = 0;
+  // whether pixels without samples are stored while the encode runs
+  bool store_background = false;
   uint32_t *total_host = nullptr;  // pinned
   uint32_t n_views = 0, n_slots = 0;
   uint32_t capacity = 0;          // samples the sample buffers hold
   int capacity_precision = -1;    // feature layout the buffers were sized for
-  size_t out_px = 0;
+  size_t out_px = 0;              // pixels of the output arrays (each view starts on kViewAlign)
+  size_t pixels = 0;              // pixels of the views
   std::vector<ViewDesc> host_views;
   // Pinned staging of the view descriptors: an upload from pageable memory
   // can block the host until the stream reaches it.  ev_views marks the
@@ -150,9 +174,13 @@ int render_reserve_samples(RenderWork &w, int precision, size_t capacity);
 // Clears the frame counters and uploads the view descriptors of render_setup;
 // precedes the first pass of a frame.
 int render_begin(RenderWork &w, hipStream_t stream);
-// Stores the frame counters and stamps into total_host; follows the last pass
-// (or any pass whose counters the host reads).
+// Stores the frame counters and stamps into total_host and the outputs of
+// host_out into theirs; follows the last pass (or any pass whose counters the
+// host reads).
 int render_end(RenderWork &w, hipStream_t stream);
+// Has the frame of render_setup store the requested outputs into the caller's
+// memory, if all of it is pinned; n_host_out stays 0 otherwise.
+void plan_host_outputs(RenderWork &w, const nes_view_out *outs);
 // One pass: march steps [k0, k1) (or, with resume, from where the ray's
 // previous pass stopped), at most `cap` samples per ray, then encode, MLPs
 // and composite.
@@ -206,9 +234,12 @@ int launch_composite(RenderWork &w, hipStream_t stream);
 
 // Enqueue a full render of views on stream; returns after the sample count
 // read-backs (one host sync per pass).  Outputs land in work.out.
+// With outs, the requested outputs are in the caller's memory on return if
+// *delivered is set (render_fetch gets them otherwise).
 int render_enqueue(const SceneDev &scene, RenderWork &work, int precision,
                    const nes_camera *views, int n_views, int steps_per_pass,
-                   hipStream_t stream, nes_render_stats *stats);
+                   hipStream_t stream, nes_render_stats *stats,
+                   const nes_view_out *outs = nullptr, bool *delivered = nullptr);
 int render_fetch(RenderWork &work, int view, const nes_view_out *out,
                  hipStream_t stream);
 void render_work_free(RenderWork &w);

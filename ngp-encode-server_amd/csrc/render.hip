@@ -73,6 +73,7 @@ struct MarchArgs {
   int resume;      // kMarchNext: every ray with samples left has kRayState, go on at its step
   int store_rays;  // kMarchFirst: 0 none (single pass), 1 rays with samples, 2 every ray
   uint2 *ray_sh;
+  uint32_t *tile_n;  // kMarchFirst: samples per wavefront
   uint64_t *stamp;  // device clock at the kernel's start (optional)
 };
 
@@ -228,7 +229,10 @@ __global__ __launch_bounds__(256) void march_emit(MarchArgs m) {
   }
   // the workgroup's range of the sample list, one part per wavefront
   const uint32_t wave_total = wave_sum(cnt);
-  if (lane == 0) wave_n[wave] = wave_total;
+  if (lane == 0) {
+    wave_n[wave] = wave_total;
+    if (m.mode == kMarchFirst && slot < m.n_slots) m.tile_n[slot >> 6] = wave_total;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     const uint32_t n = wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
@@ -370,6 +374,71 @@ __device__ __forceinline__ float sigmoid_fast(float v) {
   return __builtin_amdgcn_rcpf(1.0f + __expf(-v));
 }
 
+// ------------------------------------------------- outputs to host memory
+// A frame whose outputs go to pinned host memory is bound by the link for a
+// quarter of its time (stereo 1080p RGB24 and depth: 29 MB, 0.52 ms at 56
+// GB/s, against 1.4 ms of kernels).  Pixels of tiles without samples are final
+// (zero) once the march is done, so they are stored during the encode, by a
+// few extra workgroups of its launch; the rest follow the composite.  The
+// split is by 128-byte line of each output array: a line is background if all
+// of its pixels lie in tiles without samples.
+
+// Whether the 16 bytes at `unit` of the array are background.
+__device__ __forceinline__ bool unit_is_background(const HostArray &h, const ViewDesc &v,
+                                                   const uint32_t *__restrict__ tile_n, uint32_t unit) {
+  const uint32_t p0 = unit * 16 / h.bpp, p1 = min((unit * 16 + 15) / h.bpp, v.width * v.height - 1);
+  const uint32_t *tn = tile_n + (v.slot_base >> 6);
+  uint32_t y = p0 / v.width, x = p0 - y * v.width;
+  uint32_t n = 0;
+  // the tiles of the first pixel and of every pixel that starts a tile or row
+  for (uint32_t p = p0;;) {
+    n |= tn[(y >> 3) * v.tiles_x + (x >> 3)];
+    const uint32_t step = min(8u - (x & 7u), v.width - x);
+    p += step;
+    x += step;
+    if (p > p1) break;
+    if (x == v.width) {
+      x = 0;
+      ++y;
+    }
+  }
+  return n == 0;
+}
+
+// The same for the 128-byte line of this lane's unit; lanes hold consecutive
+// units from a multiple of 64 on.
+__device__ __forceinline__ bool line_is_background(const HostArray &h, const ViewDesc &v,
+                                                   const uint32_t *__restrict__ tile_n, uint32_t unit,
+                                                   uint32_t n_units) {
+  const uint64_t b = __ballot(unit < n_units && unit_is_background(h, v, tile_n, unit));
+  return ((b >> (lane_id() & ~7)) & 0xffu) == 0xffu;
+}
+
+struct BackgroundArgs {
+  const HostArray *arrays;
+  const ViewDesc *views;
+  const uint32_t *tile_n;
+  uint32_t n_arrays, groups;  // groups: workgroups that store, 0 = none
+};
+
+// One store of 1 KB per wavefront in flight: with kBackgroundGroups x 4 waves
+// that covers the link's bandwidth times its latency, and no more queues up
+// in the memory pipeline that the encode's gathers share.
+__device__ __forceinline__ void store_background(const BackgroundArgs &a, uint32_t grp) {
+  const uint32_t wave = grp * 4 + (threadIdx.x >> 6), n_waves = a.groups * 4;
+  for (uint32_t i = 0; i < a.n_arrays; ++i) {
+    const HostArray h = a.arrays[i];
+    const ViewDesc v = a.views[h.view];
+    const uint32_t n_units = (uint32_t)(h.bytes / 16);
+    for (uint32_t at = wave * 64; at < n_units; at += n_waves * 64) {
+      const uint32_t unit = at + (uint32_t)lane_id();
+      if (line_is_background(h, v, a.tile_n, unit, n_units))
+        reinterpret_cast<uint4 *>(h.dst)[unit] = make_uint4(0u, 0u, 0u, 0u);
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+  }
+}
+
 // ------------------------------------------------- XCD-partitioned encode
 // MI355X dispatches workgroup b to XCD b % 8, and each XCD has its own 4 MB
 // L2.  Part p = b % 8 encodes only levels p and 15 - p for every sample, so
@@ -402,12 +471,18 @@ __global__ __launch_bounds__(256) void encode_parts(const typename PosIn<Tab>::t
                                                     const uint32_t *__restrict__ n_ptr,
                                                     uint32_t stride, const Tab *__restrict__ table,
                                                     typename PartOut<Tab>::type *__restrict__ feat,
-                                                    uint32_t blocks_per_part, uint64_t *stamp) {
+                                                    uint32_t blocks_per_part, BackgroundArgs bg,
+                                                    uint64_t *stamp) {
   stamp_start(stamp);
   __shared__ uint32_t xch_all[4][256];  // per-wavefront gather exchange (FP16 hashed levels)
+  // the first workgroups (a multiple of kParts of them) store background pixels
+  if (blockIdx.x < bg.groups) {
+    store_background(bg, blockIdx.x);
+    return;
+  }
   uint32_t *xch = xch_all[threadIdx.x >> 6];
   const uint32_t n = min(*n_ptr, stride);
-  const uint32_t grp = blockIdx.x / kParts;
+  const uint32_t grp = (blockIdx.x - bg.groups) / kParts;
   switch (blockIdx.x % kParts) {
     case 0: encode_part_loop<Tab, 0>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
     case 1: encode_part_loop<Tab, 1>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
@@ -675,26 +750,86 @@ constexpr uint32_t kArgViews = 8;
 struct ArgViews {
   ViewDesc v[kArgViews];
 };
+struct ArgArrays {
+  HostArray a[kHostArrays];
+};
 constexpr int kViewWords = (int)(sizeof(ViewDesc) / sizeof(uint32_t));
-static_assert(sizeof(ViewDesc) % sizeof(uint32_t) == 0, "whole words");
+constexpr int kArrayWords = (int)(sizeof(HostArray) / sizeof(uint32_t));
+static_assert(sizeof(ViewDesc) % sizeof(uint32_t) == 0 && sizeof(HostArray) % sizeof(uint32_t) == 0, "whole words");
 constexpr int kFrameThreads = 1024;
 
-__global__ __launch_bounds__(kFrameThreads) void frame_begin(uint32_t *total, ArgViews views,
-                                                             uint32_t n_views, ViewDesc *dst) {
+__global__ __launch_bounds__(kFrameThreads) void frame_begin(uint32_t *total, ArgViews views, uint32_t n_views,
+                                                             ViewDesc *dst, ArgArrays arrays,
+                                                             uint32_t n_arrays, HostArray *array_dst) {
   const int t = (int)threadIdx.x;
   for (int i = t; i < kTotWords; i += kFrameThreads)
     if (i != kTotStamps + 2 * kStampBegin && i != kTotStamps + 2 * kStampBegin + 1) total[i] = 0u;
-  if (t < (int)n_views * kViewWords)
-    reinterpret_cast<uint32_t *>(dst)[t] = reinterpret_cast<const uint32_t *>(&views)[t];
+  for (int i = t; i < (int)n_views * kViewWords; i += kFrameThreads)
+    reinterpret_cast<uint32_t *>(dst)[i] = reinterpret_cast<const uint32_t *>(&views)[i];
+  for (int i = t; i < (int)n_arrays * kArrayWords; i += kFrameThreads)
+    reinterpret_cast<uint32_t *>(array_dst)[i] = reinterpret_cast<const uint32_t *>(&arrays)[i];
   if (t == 0) reinterpret_cast<uint64_t *>(total + kTotStamps)[kStampBegin] = wall_clock64();
 }
 
-// The end of a frame: the counters and stamps into pinned host memory.
-__global__ __launch_bounds__(kFrameThreads) void frame_end(const uint32_t *total, uint32_t *host) {
+// `bytes` of depth as GRAY8, or of the array as it is, from element `at` on.
+template <class T>
+__device__ __forceinline__ void store_unit(const HostArray &h, uint32_t at) {
+  T v;
+  if (h.gray_scale != 0.0f) {
+    uint8_t g[sizeof(T)];
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(T); ++i)
+      g[i] = depth_gray8(reinterpret_cast<const float *>(h.src)[(size_t)at * sizeof(T) + i], h.gray_scale);
+    __builtin_memcpy(&v, g, sizeof(T));
+  } else {
+    v = reinterpret_cast<const T *>(h.src)[at];
+  }
+  reinterpret_cast<T *>(h.dst)[at] = v;
+}
+
+template <class T>
+__device__ __forceinline__ void store_array(const HostArray &h) {
+  const uint32_t n = (uint32_t)(h.bytes / sizeof(T));
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) store_unit<T>(h, i);
+  if (blockIdx.x == 0 && threadIdx.x < h.bytes % sizeof(T))
+    store_unit<uint8_t>(h, (uint32_t)(n * sizeof(T)) + threadIdx.x);
+}
+
+// Output arrays into host memory, one per blockIdx.y; with `bg`, only what
+// store_background left.
+__device__ __forceinline__ void store_outputs(const HostArray &h, const BackgroundArgs *bg) {
+  if (bg) {
+    const ViewDesc v = bg->views[h.view];
+    const uint32_t n_units = (uint32_t)(h.bytes / 16);
+    for (uint32_t at = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 64; at < n_units; at += gridDim.x * 256) {
+      const uint32_t unit = at + (uint32_t)lane_id();
+      if (!line_is_background(h, v, bg->tile_n, unit, n_units) && unit < n_units) store_unit<uint4>(h, unit);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < h.bytes % 16) store_unit<uint8_t>(h, n_units * 16 + threadIdx.x);
+  } else if (h.unit == 16) {
+    store_array<uint4>(h);
+  } else if (h.unit == 4) {
+    store_array<uint32_t>(h);
+  } else {
+    store_array<uint8_t>(h);
+  }
+}
+
+// The end of a frame: the counters and stamps and the output arrays into
+// pinned host memory.
+__global__ __launch_bounds__(256) void frame_end(const uint32_t *total, uint32_t *host, BackgroundArgs a) {
   constexpr int kEnd = kTotStamps + 2 * kStampEnd;
-  for (int i = (int)threadIdx.x; i < kTotWords; i += kFrameThreads)
-    if (i != kEnd && i != kEnd + 1) host[i] = total[i];
-  if (threadIdx.x == 0) reinterpret_cast<uint64_t *>(host + kTotStamps)[kStampEnd] = wall_clock64();
+  if (blockIdx.x == 0 && blockIdx.y == 0) {
+    for (int i = (int)threadIdx.x; i < kTotWords; i += (int)blockDim.x)
+      if (i != kEnd && i != kEnd + 1) host[i] = total[i];
+    if (threadIdx.x == 0) reinterpret_cast<uint64_t *>(host + kTotStamps)[kStampEnd] = wall_clock64();
+  }
+  if (blockIdx.y < a.n_arrays) store_outputs(a.arrays[blockIdx.y], a.groups ? &a : nullptr);
+}
+
+// The same for arrays of a finished frame (nes_render_fetch).
+__global__ __launch_bounds__(256) void store_arrays(ArgArrays arrays) {
+  store_outputs(arrays.a[blockIdx.y], nullptr);
 }
 
 // FP32 expected depth -> the GRAY8 depth plane of the response.
@@ -775,7 +910,7 @@ void scene_free(SceneDev &s) {
 }
 
 void render_work_free(RenderWork &w) {
-  for (DevBuf *b : {&w.views, &w.rays, &w.acc, &w.counts, &w.offsets, &w.ray_sh, &w.t_start, &w.gray, &w.samples,
+  for (DevBuf *b : {&w.views, &w.rays, &w.acc, &w.counts, &w.offsets, &w.ray_sh, &w.t_start, &w.gray, &w.tile_n, &w.host_arrays, &w.samples,
                     &w.sample_out, &w.sample_pos, &w.feat, &w.out, &w.total})
     b->release();
   if (w.total_host) hipHostFree(w.total_host);
@@ -817,9 +952,11 @@ int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_
   // after a failed setup or pass is refused instead of reading stale layouts.
   w.n_views = 0;
   w.out_px = 0;
+  w.n_host_out = 0;
+  w.store_background = false;
   if (!views || n_views < 1) return NES_EINVAL;
   w.host_views.resize((size_t)n_views);
-  uint64_t slots = 0, px = 0;
+  uint64_t slots = 0, px = 0, pixels = 0;
   for (int i = 0; i < n_views; ++i) {
     const nes_camera &c = views[i];
     if (c.width < 1 || c.height < 1 || c.width > 16384 || c.height > 16384 ||
@@ -844,7 +981,8 @@ int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_
     const double down = std::sqrt((double)c.c2w[1] * c.c2w[1] + (double)c.c2w[5] * c.c2w[5] + (double)c.c2w[9] * c.c2w[9]);
     v.tile_reach = (float)(1.01 * 3.5 * (right + down) / (double)v.focal);
     slots += v.slot_count;
-    px += (uint64_t)c.width * c.height;
+    px = align_up(px + (uint64_t)c.width * c.height, kViewAlign);
+    pixels += (uint64_t)c.width * c.height;
     if (slots > kMaxSlots) {
       set_last_error("render batch exceeds 2^25 ray slots");
       return NES_ERANGE;
@@ -853,6 +991,7 @@ int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_
   w.n_views = (uint32_t)n_views;
   w.n_slots = (uint32_t)slots;
   w.out_px = px;
+  w.pixels = pixels;
   NES_TRY(w.views.reserve(sizeof(ViewDesc) * n_views));
   NES_TRY(w.rays.reserve(sizeof(RayData) * slots));
   NES_TRY(w.acc.reserve(sizeof(RayAcc) * slots));
@@ -860,6 +999,8 @@ int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_
   NES_TRY(w.offsets.reserve(sizeof(uint32_t) * wavefronts(slots)));
   NES_TRY(w.ray_sh.reserve(32 * slots));
   NES_TRY(w.t_start.reserve(sizeof(float) * slots));
+  NES_TRY(w.tile_n.reserve(sizeof(uint32_t) * wavefronts(slots)));
+  NES_TRY(w.host_arrays.reserve(sizeof(HostArray) * kHostArrays));
   NES_TRY(w.out.reserve(out_layout(px).total));
   NES_TRY(w.total.reserve(kTotBytes));
   if (!w.total_host) NES_HIP_TRY(hipHostMalloc((void **)&w.total_host, kTotBytes));
@@ -891,7 +1032,9 @@ int render_work_reserve(RenderWork &w, uint64_t max_slots, uint64_t max_px, uint
   NES_TRY(w.offsets.reserve(sizeof(uint32_t) * wavefronts(max_slots)));
   NES_TRY(w.ray_sh.reserve(32 * max_slots));
   NES_TRY(w.t_start.reserve(sizeof(float) * max_slots));
-  NES_TRY(w.out.reserve(out_layout(max_px).total));
+  NES_TRY(w.tile_n.reserve(sizeof(uint32_t) * wavefronts(max_slots)));
+  NES_TRY(w.host_arrays.reserve(sizeof(HostArray) * kHostArrays));
+  NES_TRY(w.out.reserve(out_layout(max_px + kViewAlign * max_views).total));
   NES_TRY(w.total.reserve(kTotBytes));
   return render_reserve_samples(w, precision, std::max<size_t>(max_slots * 4, (size_t)1 << 20));
 }
@@ -920,6 +1063,7 @@ static MarchArgs march_args(RenderWork &w, const uint32_t *occ, int k0, int k1, 
   m.offsets = w.offsets.as<uint32_t>();
   m.samples = w.samples.as<uint32_t>();
   m.t_start = w.t_start.as<float>();
+  m.tile_n = w.tile_n.as<uint32_t>();
   m.pos = w.sample_pos.as<float4>();
   m.cursor = w.total.as<uint32_t>();
   m.capacity = w.capacity;
@@ -948,15 +1092,84 @@ int render_begin(RenderWork &w, hipStream_t stream) {
   ArgViews av{};
   const uint32_t n = w.n_views <= kArgViews ? w.n_views : 0u;
   std::copy(w.host_views.begin(), w.host_views.begin() + n, av.v);
-  frame_begin<<<1, kFrameThreads, 0, stream>>>(w.total.as<uint32_t>(), av, n, w.views.as<ViewDesc>());
+  ArgArrays aa{};
+  std::copy(w.host_out, w.host_out + w.n_host_out, aa.a);
+  frame_begin<<<1, kFrameThreads, 0, stream>>>(w.total.as<uint32_t>(), av, n, w.views.as<ViewDesc>(), aa,
+                                               w.n_host_out, w.host_arrays.as<HostArray>());
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }
 
+// Workgroups that store background during the encode: enough in flight for
+// the link, and not so much that the encode's loads queue behind it.  Frame
+// times with 0 (everything after the composite), 8, 16, 24, 32, 64 of them:
+//   stereo 1080p           2170 1790 1721 1896 1972 2042 us
+//   solid stereo 1440x1600 2012 1987 1640 1727 1804 1886 us
+constexpr uint32_t kBackgroundGroups = 16;
+static_assert(kBackgroundGroups % kParts == 0, "the encode's parts follow blockIdx % kParts");
+
+static BackgroundArgs background_args(const RenderWork &w) {
+  return BackgroundArgs{w.host_arrays.as<HostArray>(), w.views.as<ViewDesc>(), w.tile_n.as<uint32_t>(),
+                        w.n_host_out, w.store_background ? kBackgroundGroups : 0u};
+}
+
+// Workgroups per array for stores over the link: a few dozen keep it busy.
+static unsigned store_blocks(uint64_t most_bytes) {
+  return (unsigned)std::min<uint64_t>(32, std::max<uint64_t>(1, (most_bytes + 4095) / 4096));
+}
+
 int render_end(RenderWork &w, hipStream_t stream) {
-  frame_end<<<1, kFrameThreads, 0, stream>>>(w.total.as<uint32_t>(), w.total_host);
+  uint64_t most = 0;
+  for (uint32_t i = 0; i < w.n_host_out; ++i) most = std::max(most, w.host_out[i].bytes);
+  frame_end<<<dim3(store_blocks(most), std::max(w.n_host_out, 1u)), 256, 0, stream>>>(
+      w.total.as<uint32_t>(), w.total_host, background_args(w));
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
+}
+
+// The requested arrays of one view; false if any of them is not pinned.
+static bool host_arrays_of_view(const RenderWork &w, uint32_t view, const nes_view_out &o, HostArray *a, uint32_t *n) {
+  const ViewDesc &v = w.host_views[view];
+  const size_t px = (size_t)v.width * v.height, base = v.px_base;
+  const OutLayout L = out_layout(w.out_px);
+  const uint8_t *d = w.out.as<uint8_t>();
+  const struct {
+    void *dst;
+    size_t at;
+    uint32_t bpp;
+    float scale;
+  } all[5] = {{o.rgb24, L.rgb24 + 3 * base, 3, 0.0f},
+              {o.depth, L.depth + 4 * base, 4, 0.0f},
+              {o.rgb_f32, L.rgbf + 12 * base, 12, 0.0f},
+              {o.n_samples, L.nsamp + 2 * base, 2, 0.0f},
+              {o.depth_gray8, L.depth + 4 * base, 1, depth_scale(o.depth_far)}};
+  for (const auto &x : all) {
+    if (!x.dst) continue;
+    if (*n == kHostArrays || !device_writable(x.dst, px * x.bpp)) return false;
+    const uintptr_t al = (uintptr_t)x.dst;
+    a[(*n)++] = HostArray{d + x.at, static_cast<uint8_t *>(x.dst), px * x.bpp, x.bpp, view,
+                          al % 16 == 0 ? 16u : al % 4 == 0 ? 4u : 1u, x.scale};
+  }
+  return true;
+}
+
+// Outputs below this are stored after the composite in one go: 1 MiB takes
+// the link 19 us, about what the march and an encode of such a frame leave.
+// At 640x480 (2.1 MB) the split gains 279 -> 247 us.
+constexpr uint64_t kBackgroundMinBytes = 1u << 20;
+
+void plan_host_outputs(RenderWork &w, const nes_view_out *outs) {
+  uint32_t n = 0;
+  for (uint32_t i = 0; i < w.n_views; ++i)
+    if (!host_arrays_of_view(w, i, outs[i], w.host_out, &n)) return;
+  w.n_host_out = n;
+  uint64_t bytes = 0;
+  bool split = true;
+  for (uint32_t i = 0; i < n; ++i) {
+    bytes += w.host_out[i].bytes;
+    split = split && w.host_out[i].unit == 16 && w.host_out[i].bytes < (1ull << 31);
+  }
+  w.store_background = split && bytes >= kBackgroundMinBytes;
 }
 
 // Samples a pass is expected to have: a little more than the work area's last
@@ -993,10 +1206,12 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
   // stays on the device
   const size_t expect = expected_samples(w, first ? 0 : 1);
   const uint32_t bpp = part_blocks(expect);
+  BackgroundArgs bg = background_args(w);
+  if (!first) bg.groups = 0;
   if (f32) {
-    encode_parts<float><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<float4>(), cursor, cap,
+    encode_parts<float><<<bpp * kParts + bg.groups, 256, 0, stream>>>(w.sample_pos.as<float4>(), cursor, cap,
                                                            scene.table_f32, w.feat.as<float4>(),
-                                                           bpp, stamp + 1);
+                                                           bpp, bg, stamp + 1);
     NES_HIP_TRY(hipGetLastError());
     if (precision == NES_PRECISION_FP32_VALU)
       mlp_fp32_valu<<<256 * 4, 256, 0, stream>>>(w.sample_pos.as<float4>(), w.feat.as<float4>(),
@@ -1006,9 +1221,9 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
     else
       NES_TRY(launch_mlp_f32(scene.weights_f32, w, cursor, stream, stamp + 2));
   } else {
-    encode_parts<_Float16><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<uint2>(), cursor,
+    encode_parts<_Float16><<<bpp * kParts + bg.groups, 256, 0, stream>>>(w.sample_pos.as<uint2>(), cursor,
                                                               cap, scene.table_f16,
-                                                              w.feat.as<uint2>(), bpp, stamp + 1);
+                                                              w.feat.as<uint2>(), bpp, bg, stamp + 1);
     NES_HIP_TRY(hipGetLastError());
     const unsigned mlp_blocks =
         (unsigned)std::min<size_t>(256 * 8, std::max<size_t>(expect / (16 * kEvalWaves), 64));
@@ -1120,7 +1335,7 @@ FrameCounts render_frame_finish(RenderWork &w) {
   // behind T < 1e-4; several passes: keep two while more than 1 % of the
   // pixels stopped early with steps left (the work the first pass saved)
   const bool wasteful = c.wasted * 20 > c.evaluated;
-  const bool saving = c.saved_rays * 100 > w.out_px;
+  const bool saving = c.saved_rays * 100 > w.pixels;
   if (c.terminated && ((c.passes == 1 && wasteful) || (c.passes > 1 && saving))) {
     const uint64_t m = (c.term_samples + c.terminated - 1) / c.terminated;
     w.first_pass_cap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(m, 1), kMaxSteps - 1);
@@ -1144,7 +1359,8 @@ int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t
   const uint32_t bpp = part_blocks(n);
   encode_parts<float><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<float4>(),
                                                          w.total.as<uint32_t>(), w.capacity,
-                                                         table, w.feat.as<float4>(), bpp, nullptr);
+                                                         table, w.feat.as<float4>(), bpp, BackgroundArgs{},
+                                                         nullptr);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }
@@ -1170,7 +1386,7 @@ int render_prepare_capacity(RenderWork &w, int precision) {
 
 size_t work_device_bytes(const RenderWork &w) {
   size_t b = 0;
-  for (const DevBuf *d : {&w.views, &w.rays, &w.acc, &w.counts, &w.offsets, &w.ray_sh, &w.t_start, &w.gray, &w.samples,
+  for (const DevBuf *d : {&w.views, &w.rays, &w.acc, &w.counts, &w.offsets, &w.ray_sh, &w.t_start, &w.gray, &w.tile_n, &w.host_arrays, &w.samples,
                           &w.sample_out, &w.sample_pos, &w.feat, &w.out, &w.total})
     b += d->bytes;
   return b;
@@ -1180,7 +1396,7 @@ size_t work_device_bytes(const RenderWork &w) {
 // render starts from nothing, and report NES_ENOMEM.
 static int check_budget(RenderWork &w) {
   if (w.budget && work_device_bytes(w) > w.budget) {
-    for (DevBuf *d : {&w.views, &w.rays, &w.acc, &w.counts, &w.offsets, &w.ray_sh, &w.t_start, &w.gray, &w.samples,
+    for (DevBuf *d : {&w.views, &w.rays, &w.acc, &w.counts, &w.offsets, &w.ray_sh, &w.t_start, &w.gray, &w.tile_n, &w.host_arrays, &w.samples,
                       &w.sample_out, &w.sample_pos, &w.feat, &w.out, &w.total})
       d->release();
     w.capacity = 0;
@@ -1194,13 +1410,20 @@ static int check_budget(RenderWork &w) {
 
 static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precision,
                                 const nes_camera *views, int n_views, int steps_per_pass,
-                                hipStream_t stream, nes_render_stats *stats);
+                                hipStream_t stream, nes_render_stats *stats,
+                                const nes_view_out *outs);
 
 int render_enqueue(const SceneDev &scene, RenderWork &w, int precision,
                    const nes_camera *views, int n_views, int steps_per_pass,
-                   hipStream_t stream, nes_render_stats *stats) {
+                   hipStream_t stream, nes_render_stats *stats, const nes_view_out *outs,
+                   bool *delivered) {
   const int rc = render_enqueue_inner(scene, w, precision, views, n_views, steps_per_pass, stream,
-                                      stats);
+                                      stats, outs);
+  if (delivered) *delivered = rc == NES_OK && w.n_host_out != 0;
+  // the caller's memory is not referred to after this call
+  if (rc != NES_OK && w.n_host_out) hipStreamSynchronize(stream);
+  w.n_host_out = 0;
+  w.store_background = false;
   if (rc != NES_OK) {
     // a failed render leaves nothing to fetch
     w.n_views = 0;
@@ -1238,7 +1461,8 @@ static double add_stage_times(const RenderWork &w, int first_pass, int passes, d
 
 static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precision,
                                 const nes_camera *views, int n_views, int steps_per_pass,
-                                hipStream_t stream, nes_render_stats *stats) {
+                                hipStream_t stream, nes_render_stats *stats,
+                                const nes_view_out *outs) {
   if (!valid_precision(precision) || steps_per_pass < 0) return NES_EINVAL;
   NES_TRY(render_setup(w, views, n_views, stream));
   NES_TRY(render_prepare_capacity(w, precision));
@@ -1250,6 +1474,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
     // whole frame: one pass, or two when the previous frame of this work area
     // evaluated samples behind terminated rays (steps_per_pass 0)
     if (steps_per_pass) w.first_pass_cap = kMaxSteps;
+    if (outs) plan_host_outputs(w, outs);
     bool bounded = false;
     for (int attempt = 0;; ++attempt) {
       if (bounded)
@@ -1313,7 +1538,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
     w.first_pass_cap = kMaxSteps;  // windows are the caller's choice, not learned from
   }
   if (stats) {
-    stats->rays = w.out_px;
+    stats->rays = w.pixels;
     stats->samples = fc.evaluated;
     stats->ms_total = total;
     stats->ms_march = t[0];
@@ -1335,6 +1560,15 @@ int render_fetch(RenderWork &w, int view, const nes_view_out *out, hipStream_t s
   if (base + px > w.out_px) {
     set_last_error("view lies outside the last render's outputs");
     return NES_EINVAL;
+  }
+  ArgArrays arrays{};
+  uint32_t n = 0;
+  if (host_arrays_of_view(w, (uint32_t)view, *out, arrays.a, &n)) {
+    // pinned memory: every array in one launch
+    if (n) store_arrays<<<dim3(store_blocks(12 * px), n), 256, 0, stream>>>(arrays);
+    NES_HIP_TRY(hipGetLastError());
+    NES_HIP_TRY(hipStreamSynchronize(stream));
+    return NES_OK;
   }
   const OutLayout L = out_layout(w.out_px);
   const uint8_t *o = w.out.as<uint8_t>();
@@ -1443,9 +1677,11 @@ int nes_render(nes_ctx *ctx, int precision, const nes_camera *views, int n_views
   if (!ctx || !outs) return NES_EINVAL;
   std::lock_guard<std::mutex> lk(ctx->mu);
   const std::shared_ptr<SceneDev> sc = ctx_scene(ctx);
+  bool delivered = false;
   NES_TRY(render_enqueue(*sc, ctx->work, precision, views, n_views, steps_per_pass, ctx->stream,
-                         stats));
-  for (int i = 0; i < n_views; ++i) NES_TRY(render_fetch(ctx->work, i, &outs[i], ctx->stream));
+                         stats, outs, &delivered));
+  for (int i = 0; i < n_views && !delivered; ++i)
+    NES_TRY(render_fetch(ctx->work, i, &outs[i], ctx->stream));
   return NES_OK;
 }
 

@@ -299,27 +299,6 @@ __global__ __launch_bounds__(256) void copy_rows(RowCopyArgs a) {
     copy_row_units<uint8_t>(c);
 }
 
-// Whether the device can write `rows` rows of `width` bytes, `pitch` apart,
-// at p: all of it inside one pinned allocation that has the same address on
-// both sides (as hipHostMalloc gives it).
-static bool device_writable(const uint8_t *p, size_t width, size_t rows, size_t pitch) {
-  hipPointerAttribute_t at;
-  void *start = nullptr;
-  size_t size = 0;
-  hipDeviceptr_t q = const_cast<uint8_t *>(p);
-  const bool ok = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeHost &&
-                  at.devicePointer == p &&
-                  hipPointerGetAttribute(&start, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, q) == hipSuccess &&
-                  hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, q) == hipSuccess && start;
-  if (!ok) {
-    (void)hipGetLastError();  // an ordinary host pointer is not an error
-    return false;
-  }
-  const uintptr_t a = (uintptr_t)p, lo = (uintptr_t)start;
-  const size_t span = (rows - 1) * pitch + width;
-  return a >= lo && a - lo <= size && size - (a - lo) >= span;
-}
-
 // Whether the runtime's 2D copy takes a plane in whole-word rows.
 static bool rows_word_aligned(const nes_frame_planes &f, const nes_camera &c) {
   uintptr_t al = c.width | c.width / 2;
@@ -642,8 +621,8 @@ static int submit(nes_server *s, uint32_t client, const nes_camera *views, int n
       for (int st = 0; st < (depth ? 2 : 1) && pinned; ++st)
         for (int p = 0; p < 3 && pinned; ++p) {
           const nes_frame_planes &f = st ? rq->dplanes[v] : rq->planes[v];
-          pinned = device_writable(f.data[p], p ? views[v].width / 2 : views[v].width,
-                                   p ? views[v].height / 2 : views[v].height, (size_t)f.linesize[p]);
+          const size_t w = p ? views[v].width / 2 : views[v].width, h = p ? views[v].height / 2 : views[v].height;
+          pinned = device_writable(f.data[p], (h - 1) * (size_t)f.linesize[p] + w);
         }
     rq->row_kernel = !words && pinned;
   }

@@ -345,3 +345,86 @@ def test_tiles_outside_the_cube_match_oracle_sample_counts(nes, oracle, scene1, 
             _, _, ns = oracle.render_pixels(t, w, occ, ocam, np.arange(101 * 67, dtype=np.uint32),
                                             threads=8)
             assert np.array_equal(out["n_samples"].reshape(-1), ns)
+
+
+def _pinned_render(nes, ctx, views, prec, arrays, offset=0, far=2.5):
+    """nes_render into pinned memory (nes_host_alloc), each array `offset`
+    bytes into its allocation; returns the same dicts as Context.render."""
+    import ctypes as C
+    kinds = {"rgb24": (3, np.uint8), "depth": (1, np.float32), "rgb": (3, np.float32),
+             "n_samples": (1, np.uint16), "depth_gray8": (1, np.uint8)}
+    types = {np.uint8: C.c_uint8, np.float32: C.c_float, np.uint16: C.c_uint16}
+    outs, blocks, res = (nes.ViewOut * len(views))(), [], []
+    for o, v in zip(outs, views):
+        r, ptr = {}, {}
+        for name in arrays:
+            ch, dt = kinds[name]
+            n = v.height * v.width * ch * np.dtype(dt).itemsize
+            p = C.c_void_p()
+            nes.check(nes.lib().nes_host_alloc(n + 64, C.byref(p)), "nes_host_alloc")
+            blocks.append(p)
+            raw = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_uint8)), (n + 64,))
+            raw[:] = 0xA5
+            r[name] = (raw, offset, n, dt, (v.height, v.width) + ((3,) if ch == 3 else ()))
+            ptr[name] = C.cast(C.c_void_p(p.value + offset), C.POINTER(types[dt]))
+        o.rgb24, o.depth, o.rgb_f32 = (ptr.get(k) for k in ("rgb24", "depth", "rgb"))
+        o.n_samples, o.depth_gray8, o.depth_far = ptr.get("n_samples"), ptr.get("depth_gray8"), far
+        res.append(r)
+    st = nes.RenderStats()
+    nes.check(nes.lib().nes_render(ctx.handle, prec, (nes.Camera * len(views))(*views), len(views), outs,
+                                   0, C.byref(st)), "nes_render")
+    out = []
+    for r in res:
+        got = {}
+        for name, (raw, off, n, dt, shape) in r.items():
+            assert (raw[:off] == 0xA5).all() and (raw[off + n:] == 0xA5).all(), name
+            got[name] = raw[off:off + n].copy().view(dt).reshape(shape)
+        out.append(got)
+    for p in blocks:
+        nes.check(nes.lib().nes_host_free(p), "nes_host_free")
+    return out, st
+
+
+ALL = ("rgb24", "depth", "rgb", "n_samples", "depth_gray8")
+
+
+@pytest.mark.parametrize("prec", [FP32, MIXED])
+@pytest.mark.parametrize("w,h,offset", [
+    (640, 480, 0),    # background lines stored during the encode
+    (643, 251, 0),    # rows that start inside 16-byte units, partial tiles
+    (9, 20011, 0),    # lines that span rows
+    (640, 480, 4),    # 4-byte stores
+    (640, 480, 1),    # single bytes
+    (31, 17, 0),      # small: everything after the composite
+])
+def test_outputs_into_pinned_memory_match_pageable(nes, gpu_ctx, prec, w, h, offset):
+    """Outputs that the render's own kernels store into pinned memory equal
+    the ones copied to ordinary memory, for both eyes and every array, and
+    nothing beside them is written."""
+    h = min(h, 16384)
+    views = [nes.camera(w, h, nes.orbit_camera(30.0, 20.0, 2.0, e), fov=70.0) for e in (-0.032, 0.032)]
+    want, _ = gpu_ctx.render(views, precision=prec, depth_far=2.5)
+    got, st = _pinned_render(nes, gpu_ctx, views, prec, ALL, offset)
+    assert st.rays == 2 * w * h
+    for a, b in zip(want, got):
+        for k in ALL:
+            assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("prec", [FP32, MIXED])
+def test_pinned_outputs_of_multi_pass_frames(nes, oracle, prec):
+    """The same for frames in two passes (rays that end early) and within a
+    budget that needs bounded passes, and for a frame that outgrows its
+    buffers once."""
+    t, w, o = _const_scene(1500.0)
+    views = [nes.camera(512, 400, nes.orbit_camera(30.0, 20.0), fov=40.0)]
+    for budget in (0, 1 << 28):
+        with nes.Context(t, w, o, hbm_budget=budget) as ctx:
+            for _ in range(3):
+                got, st = _pinned_render(nes, ctx, views, prec, ALL)
+            passes = st.passes
+        with nes.Context(t, w, o) as ctx:
+            want, _ = ctx.render(views, precision=prec, steps_per_pass=128, depth_far=2.5)
+        assert passes > 1
+        for k in ALL:
+            assert np.array_equal(want[0][k], got[0][k]), k
