@@ -182,11 +182,8 @@ int nes_frameprep_device(const uint8_t *rgb_a, const float *depth_a,
 /* nes_frameprep_device without device allocation.  This entry point has no
  * counterpart in the reference: it is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  Its only scratch buffer, the vertical chroma filter of
- * the frame height, lives in a fixed device array of 144 KiB per GPU, held
- * until the process ends, so h is limited to 8192 (NES_ERANGE above).  The
- * array is shared by every call on a GPU and keeps the last call's table:
- * calls that overlap on one GPU race.  The work is enqueued on `stream` (a
+ * forbid hipMalloc).  It uses no scratch memory, so calls may overlap; h is
+ * limited to 8192 (NES_ERANGE above).  The work is enqueued on `stream` (a
  * hipStream_t) and the call returns without waiting; stream NULL uses the
  * null stream and returns after completion.  Same layout and results as
  * nes_frameprep_device. */

@@ -15,11 +15,10 @@
 //          the build: x86-64 uses yuv2yuvX_sse3 (pmulhw taps) for every output
 //          row but the last two luma rows, which use yuv2planeX_8_c.
 //
-// Kernel layout: one workgroup per (256-pixel strip, 16 chroma rows) tile of
-// one frame.  Phase 1 streams the tile's source rows (plus the filter's
-// 6-row halo) once from HBM, composites A/B, writes luma and parks the 15-bit
-// chroma intermediates in LDS; phase 2 runs the vertical chroma filter out of
-// LDS.  Inputs are read once (+~19% halo), outputs written once.
+// Kernel layout: one workgroup per tile of one frame (a 256-pixel strip of some
+// chroma rows).  Phase 1 streams the tile's source rows (plus the filter's
+// 6-row halo) once, composites A/B, writes luma and parks the 15-bit chroma
+// intermediates in LDS; phase 2 runs the vertical chroma filter out of LDS.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -160,59 +159,43 @@ VFilter build_vchroma_filter(int h) {
 
 namespace {
 std::mutex g_filter_mu;
-std::map<int, DevVFilter> g_filters;
+std::map<int, VRows> g_filters;  // by frame height (at most 8192 of them)
 }  // namespace
 
-static bool filter_fits_tiles(const VFilter &f, int h);
-
-int get_dev_vfilter(int h, DevVFilter *out) {
+int get_vrows(int h, VRows *out) {
   std::lock_guard<std::mutex> lk(g_filter_mu);
   auto it = g_filters.find(h);
-  if (it != g_filters.end()) {
-    *out = it->second;
-    return NES_OK;
+  if (it == g_filters.end()) {
+    const VFilter f = build_vchroma_filter(h);
+    const int ch = (int)f.pos.size();
+    VRows r;
+    r.taps = f.taps;
+    bool ok = f.taps >= 1 && f.taps <= kVTaps && ch == h / 2;
+    for (int k = 0; ok && k < ch; ++k) {
+      const int c = row_class(k, ch);
+      int16_t coef[kVTaps] = {};
+      std::copy_n(&f.coef[(size_t)k * f.taps], f.taps, coef);
+      if (c != 2) {
+        r.pos[c] = f.pos[k];
+      } else {
+        ok = f.taps == kVTaps && f.pos[k] == 2 * k - 3 && (k == 2 || std::equal(coef, coef + kVTaps, r.coef[2]));
+      }
+      std::copy_n(coef, kVTaps, r.coef[c]);
+    }
+    if (!ok) {
+      set_last_error("unsupported vertical filter size");
+      return NES_ERANGE;
+    }
+    it = g_filters.emplace(h, r).first;
   }
-  VFilter f = build_vchroma_filter(h);
-  if (f.taps < 1 || f.taps > 16 || !filter_fits_tiles(f, h)) {
-    set_last_error("unsupported vertical filter size");
-    return NES_ERANGE;
-  }
-  DevVFilter d;
-  d.taps = f.taps;
-  NES_HIP_TRY(hipMalloc(&d.coef, f.coef.size() * sizeof(int16_t)));
-  NES_HIP_TRY(hipMalloc(&d.pos, f.pos.size() * sizeof(int32_t)));
-  NES_HIP_TRY(hipMemcpy(d.coef, f.coef.data(), f.coef.size() * sizeof(int16_t),
-                        hipMemcpyHostToDevice));
-  NES_HIP_TRY(hipMemcpy(d.pos, f.pos.data(), f.pos.size() * sizeof(int32_t),
-                        hipMemcpyHostToDevice));
-  g_filters[h] = d;
-  *out = d;
+  *out = it->second;
   return NES_OK;
 }
 
 // ---------------------------------------------------------------- device
-constexpr int kFpQuads = 64;               // 4-pixel quads per tile row
-// 16 chroma rows per tile: a tile reads its 32 source rows plus the filter's
-// 6-row halo (the most any height needs; filter_fits_tiles checks it), and
-// the 19.5 KB of LDS let 8 workgroups (32 waves) share a CU.  Measured on
-// 256 720p frames: 32 rows 0.83 ms, 16 rows 0.74 ms, 8 rows 0.75 ms -- the
-// occupancy gained outweighs the extra halo reads.
-constexpr int kFpCRows = 16;
-constexpr int kFpRows = 2 * kFpCRows + 6;   // LDS source rows
-constexpr int kFpThreads = 256;
-
-// Source rows one tile of kFpCRows chroma rows reads (the kernel's lo..hi):
-// every tile of a filter must fit the kFpRows rows of the LDS tile.
-static bool filter_fits_tiles(const VFilter &f, int h) {
-  const int ch = h >> 1;
-  for (int k0 = 0; k0 < ch; k0 += kFpCRows) {
-    const int k1 = std::min(k0 + kFpCRows, ch);
-    const int lo = std::min(f.pos[k0], 2 * k0);
-    const int hi = std::min(std::max(f.pos[k1 - 1] + f.taps - 1, 2 * k1 - 1), h - 1);
-    if (lo < 0 || hi - lo + 1 > kFpRows) return false;
-  }
-  return true;
-}
+constexpr int kFpQuads = 64;    // 4-pixel quads per tile row, one per lane
+constexpr int kFpWaves = 4;
+constexpr int kFpXcds = 8;      // workgroup b runs on XCD b % 8
 
 struct FrameprepArgs {
   const uint8_t *rgb_a;
@@ -222,146 +205,276 @@ struct FrameprepArgs {
   uint8_t *y;
   uint8_t *u;
   uint8_t *v;
-  const int16_t *coef;
-  const int32_t *pos;
   size_t rgb_fb, depth_fb, y_fb, u_fb, v_fb;  // per-frame byte offsets
-  int w, h, y_stride, u_stride, v_stride, taps, mode;
+  int w, h, y_stride, u_stride, v_stride, mode;
+  uint32_t strips, tiles, frames;  // tiles: per strip
+  uint32_t run;                    // consecutive tiles per XCD
+  VRows flt;
 };
 
-__device__ __forceinline__ int y_of(int r, int g, int b) {
-  int y14 = (8414 * r + 16519 * g + 3208 * b + 524544) >> 9;
-  int y15 = min(2 * y14, 32767);
-  return min(max((y15 + 64) >> 7, 0), 255);
+// Loads and stores at any byte alignment (gfx950 serves them in one
+// instruction), so frame widths and addresses need no case of their own.
+typedef uint32_t Word __attribute__((aligned(1)));
+typedef uint16_t Half __attribute__((aligned(1)));
+typedef uint32_t Word2 __attribute__((ext_vector_type(2), aligned(1)));
+typedef float Depth4 __attribute__((ext_vector_type(4), aligned(1)));
+typedef float Float __attribute__((aligned(1)));
+struct Rgb4 { uint32_t w[3]; };  // four RGB24 pixels
+struct RowIn {                   // one quad of a row of both inputs
+  Rgb4 a, b;
+  Depth4 da, db;
+};
+
+template <class T>
+__device__ __forceinline__ T load_from(const uint8_t *p) {
+  return *reinterpret_cast<const T *>(p);
 }
-__device__ __forceinline__ int u15_of(int rs, int gs, int bs) {
-  return min(2 * ((-4865 * rs - 9528 * gs + 14392 * bs + 8389120) >> 10), 32767);
+// kStream: past the caches (non-temporal).
+template <bool kStream, class T>
+__device__ __forceinline__ void store_to(uint8_t *p, T v) {
+  if (kStream)
+    __builtin_nontemporal_store(v, reinterpret_cast<T *>(p));
+  else
+    *reinterpret_cast<T *>(p) = v;
 }
-__device__ __forceinline__ int v15_of(int rs, int gs, int bs) {
-  return min(2 * ((14392 * rs - 12061 * gs - 2332 * bs + 8389120) >> 10), 32767);
-}
-__device__ __forceinline__ bool take_b(float da, float db) {
-  float ka = isnan(da) ? INFINITY : da;
-  float kb = isnan(db) ? INFINITY : db;
-  return !(ka <= kb);
+__device__ __forceinline__ Rgb4 load_rgb4(const uint8_t *p) {
+  const Word2 lo = load_from<Word2>(p);
+  return Rgb4{{lo.x, lo.y, load_from<Word>(p + 8)}};
 }
 
-template <bool kFast, bool kTwo>
-__global__ __launch_bounds__(kFpThreads) void frameprep_kernel(FrameprepArgs a) {
-  __shared__ int16_t su[kFpRows][2 * kFpQuads];
-  __shared__ int16_t sv[kFpRows][2 * kFpQuads];
+enum FrameClass {
+  kPlain,
+  kBulk,    // more data than the Infinity Cache holds
+  kNarrow,  // width 2
+};
 
-  const int f = blockIdx.z;
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t dot_u(uint32_t a, uint32_t c0, uint32_t c1, uint32_t acc) {
+  const u16x2 c = {(unsigned short)c0, (unsigned short)c1};
+  return __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, a), c, acc, false);
+}
+__device__ __forceinline__ int dot_i(uint32_t a, int c, int acc) {
+  const i16x2 cc = {(short)c, (short)c};
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(i16x2, a), cc, acc, false);
+}
+// Bytes i and j (0..3 of lo, 4..7 of hi) as the halves of a word.
+template <int I, int J>
+__device__ __forceinline__ uint32_t byte_pair(uint32_t hi, uint32_t lo) {
+  return __builtin_amdgcn_perm(hi, lo, 0x0c000c00u | (J << 16) | I);
+}
+
+// Depth key order with NaN as +infinity; ties keep A.
+__device__ __forceinline__ bool take_b(float da, float db) { return db < fminf(da, INFINITY); }
+
+// Luma of two pixels whose components are the halves of r, g, b.  With
+// Y14 = (8414 r + 16519 g + 3208 b + 524544) >> 9 (at most 15040, so neither
+// 2 * Y14 nor the result reaches a clamp), (2 * Y14 + 64) >> 7 is the sum
+// plus 16384 shifted by 15; the doubled sum has it in its third byte.
+__device__ __forceinline__ void luma2(uint32_t r, uint32_t g, uint32_t b, uint32_t y[2]) {
+  constexpr uint32_t kR = 2 * 8414, kG = 2 * 16519, kB = 2 * 3208, kC = 2 * (524544 + 16384);
+  y[0] = dot_u(r, kR, 0, dot_u(g, kG, 0, dot_u(b, kB, 0, kC)));
+  y[1] = dot_u(r, 0, kR, dot_u(g, 0, kG, dot_u(b, 0, kB, kC)));
+}
+// The 15-bit chroma 2 * (sum >> 10) of a pixel pair and of the next one, as
+// the halves of a word (the sums are positive and at most 30720 after it: no
+// clamp is reached).
+__device__ __forceinline__ uint32_t chroma2(int s0, int s1) {
+  const uint32_t lo = (uint32_t)s0 >> 9, hi = (uint32_t)s1 << 7;
+  return ((lo & 0xffffu) | (hi & 0xffff0000u)) & 0xfffefffeu;
+}
+__device__ __forceinline__ int usum(uint32_t r, uint32_t g, uint32_t b) {
+  return dot_i(r, -4865, dot_i(g, -9528, dot_i(b, 14392, 8389120)));
+}
+__device__ __forceinline__ int vsum(uint32_t r, uint32_t g, uint32_t b) {
+  return dot_i(r, 14392, dot_i(g, -12061, dot_i(b, -2332, 8389120)));
+}
+
+// Frame widths under four: the row's two pixels byte by byte.
+__device__ __forceinline__ Rgb4 load_two_pixels(const uint8_t *p) {
+  Rgb4 q;
+  q.w[0] = (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
+  q.w[1] = (uint32_t)p[4] | ((uint32_t)p[5] << 8);
+  q.w[2] = 0u;
+  return q;
+}
+
+// One chroma row of a quad: (u0 u1, v0 v1) in bytes.  The x86 rows (all but
+// the last) sum the high halves of the products, which no order of taps takes
+// out of 16 bits.
+template <bool kX86, class Rows>
+__device__ __forceinline__ uint2 filter_row(Rows &&rows, const int16_t *cf, int taps) {
+  const int init = kX86 ? (64 + 8 * (taps - 1)) >> 4 : 64 << 12;
+  int s[4] = {init, init, init, init};  // u0, u1, v0, v1
+#pragma unroll
+  for (int j = 0; j < kVTaps; ++j) {
+    const uint2 q = rows(j);
+    const int t[4] = {(int)(q.x & 0xffffu), (int)(q.x >> 16), (int)(q.y & 0xffffu), (int)(q.y >> 16)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int prod = __mul24((int)cf[j], t[i]);
+      s[i] += kX86 ? prod >> 16 : prod;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = min(max(s[i] >> (kX86 ? 3 : 19), 0), 255);
+  return make_uint2((uint32_t)(s[0] | (s[1] << 8)), (uint32_t)(s[2] | (s[3] << 8)));
+}
+
+template <FrameClass kClass>
+struct PlaneRow {
+  uint8_t *u, *v;
+  __device__ __forceinline__ void store(const FrameprepArgs &a, int k, uint2 s) const {
+    uint8_t *ur = u + (size_t)k * a.u_stride, *vr = v + (size_t)k * a.v_stride;
+    if (kClass == kNarrow) {
+      ur[0] = (uint8_t)s.x;
+      vr[0] = (uint8_t)s.y;
+    } else {
+      store_to<kClass == kBulk, Half>(ur, (uint16_t)s.x);
+      store_to<kClass == kBulk, Half>(vr, (uint16_t)s.y);
+    }
+  }
+};
+
+// Bound by HBM in bulk (256 720p pairs: 727 -> 706 us, 5.18 TB/s of inputs and
+// outputs, what a device copy reaches) and by its own latency for one frame
+// (720p pair with launch and wait: 24.4 -> 16.7 us, 11.1 of them an empty
+// launch and wait).  What counted: the filter's rows as kernel arguments (no
+// table in memory); byte pairs gathered by v_perm into 16-bit dot products (a
+// third fewer instructions); wide loads at any alignment, so that widths of 4k
+// + 2 need no per-pixel path (642x360 x 8: 37 -> 17 us); the next row's loads
+// ahead of this row's arithmetic.  Tiles are dealt to the XCDs in runs of
+// kFpRunRows tile rows, and neighbours meet at the rows they share (bulk: 716
+// us with single tiles, 737 with one run per XCD).  Tiles of 32 and 64 chroma
+// rows (less halo, 8 and 16 wavefronts) took 721 and 714 us, non-temporal
+// loads 820.
+template <bool kTwo, int kCRows, FrameClass kClass>
+__global__ __launch_bounds__(64 * kFpWaves) void frameprep_kernel(FrameprepArgs a) {
+  __shared__ uint2 uv[2 * kCRows + 6][kFpQuads];  // (u0 u1, v0 v1) of each quad
+  __shared__ int16_t edge_coef[kVClasses * kVTaps];
+  const uint32_t total = a.strips * a.tiles * a.frames;
+  // runs of a.run tiles, dealt to the XCDs in turn
+  const uint32_t turn = blockIdx.x / kFpXcds;
+  const uint32_t id = (turn / a.run * kFpXcds + blockIdx.x % kFpXcds) * a.run + turn % a.run;
+  if (id >= total) return;
+  const uint32_t strip = id % a.strips, tile = id / a.strips % a.tiles, f = id / a.strips / a.tiles;
   const uint8_t *rgb_a = a.rgb_a + f * a.rgb_fb;
-  const float *dep_a = a.depth_a ? (const float *)((const uint8_t *)a.depth_a + f * a.depth_fb) : nullptr;
   const uint8_t *rgb_b = kTwo ? a.rgb_b + f * a.rgb_fb : nullptr;
-  const float *dep_b = kTwo ? (const float *)((const uint8_t *)a.depth_b + f * a.depth_fb) : nullptr;
-  uint8_t *yp = a.y + f * a.y_fb;
-  uint8_t *up = a.u + f * a.u_fb;
-  uint8_t *vp = a.v + f * a.v_fb;
+  const uint8_t *dep_a = kTwo ? (const uint8_t *)a.depth_a + f * a.depth_fb : nullptr;
+  const uint8_t *dep_b = kTwo ? (const uint8_t *)a.depth_b + f * a.depth_fb : nullptr;
+  uint8_t *yp = a.y + f * a.y_fb, *up = a.u + f * a.u_fb, *vp = a.v + f * a.v_fb;
 
-  const int ch = a.h >> 1, cw = a.w >> 1;
-  const int k0 = blockIdx.y * kFpCRows;
-  const int k1 = min(k0 + kFpCRows, ch);
-  const int lo = min(a.pos[k0], 2 * k0);
-  const int hi = min(max(a.pos[k1 - 1] + a.taps - 1, 2 * k1 - 1), a.h - 1);
+  const int ch = a.h >> 1;
+  const int k0 = (int)tile * kCRows, k1 = min(k0 + kCRows, ch);
+  const int lo = min(row_pos(a.flt, k0, ch), 2 * k0);
+  const int hi = min(max(row_pos(a.flt, k1 - 1, ch) + a.flt.taps - 1, 2 * k1 - 1), a.h - 1);
   const int nrows = hi - lo + 1;
-  const int q_base = blockIdx.x * kFpQuads;
+  const int lane = (int)(threadIdx.x & 63u);
+  const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // rows are wavefront-uniform
+  const int quad = (int)strip * kFpQuads + lane;
+  // the last quad of a width that is no multiple of 4 overlaps the one before
+  // it (both compute the same values)
+  constexpr bool narrow = kClass == kNarrow, stream = kClass == kBulk;
+  const int x0 = narrow ? 0 : min(4 * quad, a.w - 4);
+  const bool on = 4 * quad < a.w;
 
-  // Phase 1: composite, luma out, chroma intermediates into LDS.
-  for (int it = threadIdx.x; it < nrows * kFpQuads; it += kFpThreads) {
-    const int rr = it / kFpQuads, q = it % kFpQuads;
-    const int r = lo + rr;
-    const int x0 = 4 * (q_base + q);
-    if (x0 >= a.w) continue;
-    const int np = min(4, a.w - x0);  // 4, or 2 at a ragged right edge
-    int px[4][3];
-    const size_t rowp = (size_t)r * a.w + x0;
-    if (kFast) {
-      const uint32_t *ra = (const uint32_t *)(rgb_a + 3 * rowp);
-      uint32_t wa[3] = {ra[0], ra[1], ra[2]};
-      uint32_t wb[3] = {0, 0, 0};
-      float4 da = make_float4(0, 0, 0, 0), db = da;
-      if (kTwo) {
-        const uint32_t *rb = (const uint32_t *)(rgb_b + 3 * rowp);
-        wb[0] = rb[0]; wb[1] = rb[1]; wb[2] = rb[2];
-        da = *(const float4 *)(dep_a + rowp);
-        db = *(const float4 *)(dep_b + rowp);
-      }
-      const float dav[4] = {da.x, da.y, da.z, da.w}, dbv[4] = {db.x, db.y, db.z, db.w};
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const bool useb = kTwo && take_b(dav[p], dbv[p]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const int byte = 3 * p + c;
-          const uint32_t word = useb ? wb[byte >> 2] : wa[byte >> 2];
-          px[p][c] = (word >> (8 * (byte & 3))) & 0xff;
+  const bool edge = k0 < 2 || k1 > ch - 2;
+  if (edge && threadIdx.x < kVClasses * kVTaps)
+    edge_coef[threadIdx.x] = reinterpret_cast<const int16_t *>(a.flt.coef)[threadIdx.x];
+
+  // Phase 1: composite, luma out, chroma intermediates into LDS; one row per
+  // wavefront and iteration.
+  if (on) {
+    auto fetch = [&](int rr) {
+      const size_t at = (size_t)(lo + rr) * a.w + x0;
+      RowIn in;
+      if (narrow) {
+        in.a = load_two_pixels(rgb_a + 3 * at);
+        if (kTwo) {
+          in.b = load_two_pixels(rgb_b + 3 * at);
+          for (int i = 0; i < 2; ++i) {
+            in.da[i] = load_from<Float>(dep_a + 4 * (at + i));
+            in.db[i] = load_from<Float>(dep_b + 4 * (at + i));
+          }
+        }
+      } else {
+        in.a = load_rgb4(rgb_a + 3 * at);
+        if (kTwo) {
+          in.b = load_rgb4(rgb_b + 3 * at);
+          in.da = load_from<Depth4>(dep_a + 4 * at);
+          in.db = load_from<Depth4>(dep_b + 4 * at);
         }
       }
-    } else {
-      for (int p = 0; p < 4; ++p) {
-        if (p >= np) { px[p][0] = px[p][1] = px[p][2] = 0; continue; }
-        const uint8_t *src = rgb_a + 3 * (rowp + p);
-        if (kTwo && take_b(dep_a[rowp + p], dep_b[rowp + p])) src = rgb_b + 3 * (rowp + p);
-        px[p][0] = src[0]; px[p][1] = src[1]; px[p][2] = src[2];
-      }
-    }
-    if (r >= 2 * k0 && r < 2 * k1) {
-      uint8_t *yr = yp + (size_t)r * a.y_stride + x0;
-      if (kFast) {
-        uint32_t packed = 0;
+      return in;
+    };
+    // Every other tile goes from its last row up, so that two neighbours read
+    // the rows they share at about the same time.  The next row's loads are in
+    // flight while this one is converted.
+    const int from = tile & 1 ? nrows - 1 : 0, dir = tile & 1 ? -1 : 1;
+    RowIn next = fetch(from + dir * min(wave, nrows - 1));
+    for (int it = wave; it < nrows; it += kFpWaves) {
+      const RowIn in = next;
+      next = fetch(from + dir * min(it + kFpWaves, nrows - 1));
+      const int rr = from + dir * it, row = lo + rr;
+      Rgb4 p = in.a;
+      if (kTwo) {
+        uint32_t m[4];
 #pragma unroll
-        for (int p = 0; p < 4; ++p) packed |= (uint32_t)y_of(px[p][0], px[p][1], px[p][2]) << (8 * p);
-        *(uint32_t *)yr = packed;
-      } else {
-        for (int p = 0; p < np; ++p) yr[p] = (uint8_t)y_of(px[p][0], px[p][1], px[p][2]);
-      }
-    }
+        for (int i = 0; i < 4; ++i) m[i] = !narrow || i < 2 ? (take_b(in.da[i], in.db[i]) ? ~0u : 0u) : 0u;
+        const uint32_t wm[3] = {(m[0] & 0x00ffffffu) | (m[1] & 0xff000000u),
+                                (m[1] & 0x0000ffffu) | (m[2] & 0xffff0000u),
+                                (m[2] & 0x000000ffu) | (m[3] & 0xffffff00u)};
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      if (2 * e >= np) break;
-      const int rs = px[2 * e][0] + px[2 * e + 1][0];
-      const int gs = px[2 * e][1] + px[2 * e + 1][1];
-      const int bs = px[2 * e][2] + px[2 * e + 1][2];
-      su[rr][2 * q + e] = (int16_t)u15_of(rs, gs, bs);
-      sv[rr][2 * q + e] = (int16_t)v15_of(rs, gs, bs);
+        for (int i = 0; i < 3; ++i) p.w[i] = (in.b.w[i] & wm[i]) | (p.w[i] & ~wm[i]);
+      }
+      // [r0 g0 b0 r1] [g1 b1 r2 g2] [b2 r3 g3 b3]
+      const uint32_t r01 = byte_pair<0, 3>(p.w[1], p.w[0]), g01 = byte_pair<1, 4>(p.w[1], p.w[0]),
+                     b01 = byte_pair<2, 5>(p.w[1], p.w[0]);
+      const uint32_t r23 = byte_pair<2, 5>(p.w[2], p.w[1]), g23 = byte_pair<3, 6>(p.w[2], p.w[1]),
+                     b23 = byte_pair<0, 3>(0u, p.w[2]);
+      if (row >= 2 * k0 && row < 2 * k1) {
+        uint32_t y[4];
+        luma2(r01, g01, b01, y);
+        luma2(r23, g23, b23, y + 2);
+        const uint32_t y01 = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0602u),
+                       y23 = __builtin_amdgcn_perm(y[3], y[2], 0x06020c0cu);
+        uint8_t *yr = yp + (size_t)row * a.y_stride + x0;
+        if (narrow)
+          store_to<stream, Half>(yr, (uint16_t)y01);
+        else
+          store_to<stream, Word>(yr, y01 | y23);
+      }
+      uv[rr][lane] = make_uint2(chroma2(usum(r01, g01, b01), usum(r23, g23, b23)),
+                                chroma2(vsum(r01, g01, b01), vsum(r23, g23, b23)));
     }
   }
   __syncthreads();
+  if (!on) return;
 
-  // Phase 2: vertical chroma filter out of LDS.
-  const int c_base = 2 * q_base;
-  for (int it = threadIdx.x; it < (k1 - k0) * 2 * kFpQuads; it += kFpThreads) {
-    const int k = k0 + it / (2 * kFpQuads);
-    const int cl = it % (2 * kFpQuads);
-    const int c = c_base + cl;
-    if (c >= cw) continue;
-    const int16_t *cf = a.coef + (size_t)k * a.taps;
-    const int p0 = a.pos[k] - lo;
-    const bool x86 = a.mode == NES_SWS_X86 && 2 * k < a.h - 2;
-    int ou, ov;
-    if (x86) {
-      int16_t acu = (int16_t)((64 + 8 * (a.taps - 1)) >> 4), acv = acu;
-      for (int j = 0; j < a.taps; ++j) {
-        const int row = min(p0 + j, nrows - 1);
-        const int cj = cf[j];
-        acu = (int16_t)(acu + (int16_t)((cj * (int)su[row][cl]) >> 16));
-        acv = (int16_t)(acv + (int16_t)((cj * (int)sv[row][cl]) >> 16));
-      }
-      ou = acu >> 3;
-      ov = acv >> 3;
-    } else {
-      int vu = 64 << 12, vv = 64 << 12;
-      for (int j = 0; j < a.taps; ++j) {
-        const int row = min(p0 + j, nrows - 1);
-        vu += cf[j] * (int)su[row][cl];
-        vv += cf[j] * (int)sv[row][cl];
-      }
-      ou = vu >> 19;
-      ov = vv >> 19;
+  // Phase 2: vertical chroma filter out of LDS, one chroma row per wavefront
+  // and iteration, two samples of each plane per lane.  Tiles without the
+  // frame's first or last two chroma rows have one filter row and start at a
+  // fixed offset; in the x86 mode they hold no row of the other rounding.
+  const PlaneRow<kClass> to{up + (x0 >> 1), vp + (x0 >> 1)};
+  if (!edge) {
+    for (int k = k0 + wave; k < k1; k += kFpWaves) {
+      const uint2(*rows)[kFpQuads] = uv + 2 * (k - k0);
+      if (a.mode == NES_SWS_X86)
+        to.store(a, k, filter_row<true>([&](int j) { return rows[j][lane]; }, a.flt.coef[2], kVTaps));
+      else
+        to.store(a, k, filter_row<false>([&](int j) { return rows[j][lane]; }, a.flt.coef[2], kVTaps));
     }
-    up[(size_t)k * a.u_stride + c] = (uint8_t)min(max(ou, 0), 255);
-    vp[(size_t)k * a.v_stride + c] = (uint8_t)min(max(ov, 0), 255);
+  } else {
+    for (int k = k0 + wave; k < k1; k += kFpWaves) {
+      const int c = row_class(k, ch), p0 = row_pos(a.flt, k, ch) - lo;
+      const int16_t *cf = &edge_coef[c * kVTaps];
+      // taps past the filter's own have no weight: any row of the tile will do
+      auto row = [&](int j) { return uv[min(p0 + j, nrows - 1)][lane]; };
+      if (a.mode == NES_SWS_X86 && 2 * k < a.h - 2)
+        to.store(a, k, filter_row<true>(row, cf, a.flt.taps));
+      else
+        to.store(a, k, filter_row<false>(row, cf, a.flt.taps));
+    }
   }
 }
 
@@ -383,13 +496,33 @@ static int frameprep_check(const uint8_t *rgb_a, const float *depth_a, const uin
   return NES_OK;
 }
 
-// The frame-prep launch with the vertical chroma filter `flt` (device table).
-static int launch_frameprep_filter(const uint8_t *rgb_a, const float *depth_a,
-                                   const uint8_t *rgb_b, const float *depth_b, int w, int h,
-                                   int n_frames, size_t rgb_fb, size_t depth_fb, uint8_t *y,
-                                   int y_stride, size_t y_fb, uint8_t *u, int u_stride,
-                                   size_t u_fb, uint8_t *v, int v_stride, size_t v_fb,
-                                   int sws_mode, const DevVFilter &flt, hipStream_t stream);
+// Chroma rows per tile: tall tiles read less halo, but a small batch needs
+// workgroups.  One 720p pair: 4 rows 16.2 us, 8 rows 16.5, 16 rows 18.1; 16
+// of them: 48.9, 48.9, 50.8; 32: 101 us with any.
+static int frameprep_rows(int w, int h, int n_frames) {
+  const size_t strips = ((size_t)w + 255) / 256;
+  auto blocks = [&](int rows) { return strips * (((size_t)h / 2 + rows - 1) / rows) * n_frames; };
+  return blocks(16) >= 2048 ? 16 : blocks(8) >= 1024 ? 8 : 4;
+}
+
+// Inputs beyond this do not stay in the Infinity Cache (256 MB): their planes
+// are stored past the caches (256 720p pairs: 763 -> 743 us).
+constexpr size_t kBulkBytes = (size_t)256 << 20;
+
+constexpr uint32_t kFpRunRows = 6;  // tile rows per run
+
+template <int kCRows, FrameClass kClass>
+static void frameprep_launch(FrameprepArgs &a, bool two, hipStream_t stream) {
+  a.tiles = (uint32_t)((a.h / 2 + kCRows - 1) / kCRows);
+  const uint32_t total = a.strips * a.tiles * a.frames;
+  a.run = std::max(1u, std::min(a.strips * kFpRunRows, (total + kFpXcds - 1) / kFpXcds));
+  const uint32_t turns = (total + a.run * kFpXcds - 1) / (a.run * kFpXcds);
+  const unsigned blocks = turns * a.run * kFpXcds;
+  if (two)
+    frameprep_kernel<true, kCRows, kClass><<<blocks, 64 * kFpWaves, 0, stream>>>(a);
+  else
+    frameprep_kernel<false, kCRows, kClass><<<blocks, 64 * kFpWaves, 0, stream>>>(a);
+}
 
 int launch_frameprep(const uint8_t *rgb_a, const float *depth_a,
                      const uint8_t *rgb_b, const float *depth_b, int w, int h,
@@ -399,42 +532,27 @@ int launch_frameprep(const uint8_t *rgb_a, const float *depth_a,
                      int sws_mode, hipStream_t stream) {
   NES_TRY(frameprep_check(rgb_a, depth_a, rgb_b, depth_b, w, h, n_frames, y, y_stride, u,
                           u_stride, v, v_stride, sws_mode));
-  DevVFilter flt;
-  NES_TRY(get_dev_vfilter(h, &flt));
-  return launch_frameprep_filter(rgb_a, depth_a, rgb_b, depth_b, w, h, n_frames, rgb_fb,
-                                 depth_fb, y, y_stride, y_fb, u, u_stride, u_fb, v, v_stride,
-                                 v_fb, sws_mode, flt, stream);
-}
-
-static int launch_frameprep_filter(const uint8_t *rgb_a, const float *depth_a,
-                                   const uint8_t *rgb_b, const float *depth_b, int w, int h,
-                                   int n_frames, size_t rgb_fb, size_t depth_fb, uint8_t *y,
-                                   int y_stride, size_t y_fb, uint8_t *u, int u_stride,
-                                   size_t u_fb, uint8_t *v, int v_stride, size_t v_fb,
-                                   int sws_mode, const DevVFilter &flt, hipStream_t stream) {
   FrameprepArgs a;
+  NES_TRY(get_vrows(h, &a.flt));
   a.rgb_a = rgb_a; a.depth_a = depth_a; a.rgb_b = rgb_b; a.depth_b = depth_b;
-  a.y = y; a.u = u; a.v = v; a.coef = flt.coef; a.pos = flt.pos;
+  a.y = y; a.u = u; a.v = v;
   a.rgb_fb = rgb_fb; a.depth_fb = depth_fb; a.y_fb = y_fb; a.u_fb = u_fb; a.v_fb = v_fb;
   a.w = w; a.h = h; a.y_stride = y_stride; a.u_stride = u_stride; a.v_stride = v_stride;
-  a.taps = flt.taps; a.mode = sws_mode;
-  auto al = [](const void *p, size_t n) { return ((uintptr_t)p % n) == 0; };
-  bool fast = (w % 4 == 0) && al(rgb_a, 4) && al(y, 4) && (y_stride % 4 == 0) &&
-              (rgb_fb % 4 == 0) && (y_fb % 4 == 0);
-  if (rgb_b) fast = fast && al(rgb_b, 4) && al(depth_a, 16) && al(depth_b, 16) && (depth_fb % 16 == 0);
-  const int ch = h / 2;
-  dim3 grid((unsigned)((w / 4 + kFpQuads - 1) / kFpQuads + ((w % 4) ? 1 : 0)),
-            (unsigned)((ch + kFpCRows - 1) / kFpCRows), (unsigned)n_frames);
-  // quads cover ceil(w/4) columns; the ragged quad (w % 4 == 2) is handled by
-  // the per-pixel path
-  grid.x = (unsigned)(((w + 3) / 4 + kFpQuads - 1) / kFpQuads);
-  if (fast) {
-    if (rgb_b) frameprep_kernel<true, true><<<grid, kFpThreads, 0, stream>>>(a);
-    else frameprep_kernel<true, false><<<grid, kFpThreads, 0, stream>>>(a);
-  } else {
-    if (rgb_b) frameprep_kernel<false, true><<<grid, kFpThreads, 0, stream>>>(a);
-    else frameprep_kernel<false, false><<<grid, kFpThreads, 0, stream>>>(a);
-  }
+  a.mode = sws_mode;
+  a.strips = (uint32_t)(((w + 3) / 4 + kFpQuads - 1) / kFpQuads);
+  a.frames = (uint32_t)n_frames;
+  const bool two = rgb_b != nullptr;
+  const int rows = frameprep_rows(w, h, n_frames);
+  if (w < 4)
+    frameprep_launch<4, kNarrow>(a, two, stream);
+  else if (rows == 4)
+    frameprep_launch<4, kPlain>(a, two, stream);
+  else if (rows == 8)
+    frameprep_launch<8, kPlain>(a, two, stream);
+  else if ((size_t)w * h * n_frames * (two ? 14 : 3) < kBulkBytes)
+    frameprep_launch<16, kPlain>(a, two, stream);
+  else
+    frameprep_launch<16, kBulk>(a, two, stream);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }
@@ -445,44 +563,90 @@ static int launch_frameprep_filter(const uint8_t *rgb_a, const float *depth_a,
 // kDepth: the source is FP32 expected depth, quantised to the GRAY8 depth
 // plane on the fly (depth_gray8, `scale` = 255 / far); that plane is also
 // written to `gray_out` when it is not null.
+// One 4-pixel quad per lane and row (the last one of a width that is no
+// multiple of 4 overlaps its neighbour); the chroma of a row is one value,
+// which depends on the row's filter taps alone (`chroma` per row_class).
+struct GrayArgs {
+  const uint8_t *g;
+  const float *depth;
+  uint8_t *y, *u, *v, *gray_out;
+  int g_stride, w, h, y_stride, u_stride, v_stride;
+  float scale;
+  uint8_t chroma[kVClasses];
+  uint8_t last_chroma;  // of the last chroma row
+};
+
+__device__ __forceinline__ uint32_t gray_luma(uint32_t g) {
+  const int v15 = ((int)(g << 7) * 14071 + 33561947) >> 14;
+  return (uint32_t)min(max((v15 + 64) >> 7, 0), 255);
+}
+
 template <bool kDepth>
-__global__ void gray_kernel(const uint8_t *g, int g_stride, int w, int h,
-                            uint8_t *y, int y_stride, uint8_t *u, int u_stride,
-                            uint8_t *v, int v_stride, const int16_t *coef,
-                            const int32_t *pos, int taps, int mode, const float *depth,
-                            float scale, uint8_t *gray_out) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = blockIdx.y;
-  if (x < w) {
-    int gv;
+__global__ __launch_bounds__(256) void gray_kernel(GrayArgs a) {
+  const int quad = (int)(blockIdx.x * 64 + (threadIdx.x & 63u)), row = (int)(blockIdx.y * 4 + (threadIdx.x >> 6));
+  if (row >= a.h || 4 * quad >= a.w) return;
+  const int x0 = max(min(4 * quad, a.w - 4), 0), n = min(4, a.w);
+  uint32_t g = 0;  // four GRAY8 values
+  if (n == 4) {
     if (kDepth) {
-      gv = depth_gray8(depth[(size_t)r * w + x], scale);
-      if (gray_out) gray_out[(size_t)r * w + x] = (uint8_t)gv;
+      const Depth4 d = *reinterpret_cast<const Depth4 *>(a.depth + (size_t)row * a.w + x0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) g |= (uint32_t)depth_gray8(d[i], a.scale) << (8 * i);
     } else {
-      gv = g[(size_t)r * g_stride + x];
+      g = load_from<Word>(a.g + (size_t)row * a.g_stride + x0);
     }
-    int v15 = gv << 7;
-    v15 = (v15 * 14071 + 33561947) >> 14;
-    y[(size_t)r * y_stride + x] = (uint8_t)min(max((v15 + 64) >> 7, 0), 255);
+  } else {
+    for (int i = 0; i < n; ++i)
+      g |= (uint32_t)(kDepth ? depth_gray8(a.depth[(size_t)row * a.w + i], a.scale)
+                             : a.g[(size_t)row * a.g_stride + i]) << (8 * i);
   }
-  if ((r & 1) == 0 && x < (w >> 1)) {
-    const int k = r >> 1;
-    const int16_t *cf = coef + (size_t)k * taps;
-    int out;
-    if (mode == NES_SWS_X86 && 2 * k < h - 2) {
-      int16_t acc = (int16_t)((64 + 8 * (taps - 1)) >> 4);
-      for (int j = 0; j < taps; ++j) acc = (int16_t)(acc + (int16_t)(((int)cf[j] << 14) >> 16));
-      out = acc >> 3;
-    } else {
-      int val = 64 << 12;
-      for (int j = 0; j < taps; ++j) val += (int)cf[j] << 14;
-      out = val >> 19;
+  uint32_t y = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y |= gray_luma((g >> (8 * i)) & 0xffu) << (8 * i);
+  uint8_t *yr = a.y + (size_t)row * a.y_stride + x0;
+  uint8_t *gr = kDepth && a.gray_out ? a.gray_out + (size_t)row * a.w + x0 : nullptr;
+  const int k = row >> 1, ch = a.h >> 1;
+  const int c = row_class(k, ch);
+  const uint32_t uv = k == ch - 1 ? a.last_chroma
+                      : c == 0 ? a.chroma[0] : c == 1 ? a.chroma[1] : c == 2 ? a.chroma[2] : a.chroma[3];
+  if (n == 4) {
+    store_to<false, Word>(yr, y);
+    if (gr) store_to<false, Word>(gr, g);
+    if (row & 1) return;
+    store_to<false, Half>(a.u + (size_t)k * a.u_stride + (x0 >> 1), (uint16_t)(uv * 0x101u));
+    store_to<false, Half>(a.v + (size_t)k * a.v_stride + (x0 >> 1), (uint16_t)(uv * 0x101u));
+  } else {
+    for (int i = 0; i < n; ++i) {
+      yr[i] = (uint8_t)(y >> (8 * i));
+      if (gr) gr[i] = (uint8_t)(g >> (8 * i));
     }
-    out = min(max(out, 0), 255);
-    u[(size_t)k * u_stride + x] = (uint8_t)out;
-    v[(size_t)k * v_stride + x] = (uint8_t)out;
+    if (row & 1) return;
+    a.u[(size_t)k * a.u_stride] = (uint8_t)uv;
+    a.v[(size_t)k * a.v_stride] = (uint8_t)uv;
   }
-  (void)pos;
+}
+
+// The chroma of a gray source: its planes hold 1 << 14 before the vertical
+// filter, so a row's value is a sum over its taps.
+static uint8_t gray_chroma(const VRows &f, int c, bool x86) {
+  int s = x86 ? (64 + 8 * (f.taps - 1)) >> 4 : 64 << 12;
+  for (int j = 0; j < f.taps; ++j) s += x86 ? ((int)f.coef[c][j] << 14) >> 16 : (int)f.coef[c][j] << 14;
+  return (uint8_t)std::min(std::max(s >> (x86 ? 3 : 19), 0), 255);
+}
+
+static int launch_gray(GrayArgs &a, bool depth, int sws_mode, hipStream_t stream) {
+  VRows f;
+  NES_TRY(get_vrows(a.h, &f));
+  // every chroma row but the last takes the x86 path in that mode
+  for (int c = 0; c < kVClasses; ++c) a.chroma[c] = gray_chroma(f, c, sws_mode == NES_SWS_X86);
+  a.last_chroma = gray_chroma(f, row_class(a.h / 2 - 1, a.h / 2), false);
+  const dim3 grid((unsigned)((a.w + 255) / 256), (unsigned)((a.h + 3) / 4));
+  if (depth)
+    gray_kernel<true><<<grid, 256, 0, stream>>>(a);
+  else
+    gray_kernel<false><<<grid, 256, 0, stream>>>(a);
+  NES_HIP_TRY(hipGetLastError());
+  return NES_OK;
 }
 
 int launch_depth_yuv(const float *depth, int w, int h, float scale, uint8_t *gray, uint8_t *y,
@@ -491,14 +655,11 @@ int launch_depth_yuv(const float *depth, int w, int h, float scale, uint8_t *gra
   if (!depth || !y || !u || !v || w < 2 || h < 2 || (w & 1) || (h & 1)) return NES_EINVAL;
   if (y_stride < w || u_stride < w / 2 || v_stride < w / 2) return NES_EINVAL;
   if (sws_mode != NES_SWS_X86 && sws_mode != NES_SWS_C) return NES_EINVAL;
-  DevVFilter flt;
-  NES_TRY(get_dev_vfilter(h, &flt));
-  dim3 grid((unsigned)((w + 255) / 256), (unsigned)h);
-  gray_kernel<true><<<grid, 256, 0, stream>>>(nullptr, 0, w, h, y, y_stride, u, u_stride, v,
-                                              v_stride, flt.coef, flt.pos, flt.taps, sws_mode,
-                                              depth, scale, gray);
-  NES_HIP_TRY(hipGetLastError());
-  return NES_OK;
+  GrayArgs a{};
+  a.depth = depth; a.scale = scale; a.gray_out = gray;
+  a.y = y; a.u = u; a.v = v;
+  a.w = w; a.h = h; a.y_stride = y_stride; a.u_stride = u_stride; a.v_stride = v_stride;
+  return launch_gray(a, true, sws_mode, stream);
 }
 
 namespace {
@@ -506,61 +667,8 @@ std::mutex g_host_mu;
 DevBuf g_in, g_out;
 }  // namespace
 
-// ------------------------------------------------ allocation-free variant
-// nes_frameprep_device_static keeps its one scratch buffer -- the vertical
-// chroma filter of the frame height (coefficients, then row positions) -- in
-// this fixed device array instead of the per-height device cache, so a call
-// allocates no device memory.  Each GPU holds its own copy until the process
-// ends; the host refers to it only through the address hipGetSymbolAddress
-// returns for the current device.
+// nes_frameprep_device_static's documented height limit.
 constexpr int kStaticMaxHeight = 8192;
-constexpr int kStaticMaxTaps = 16;
-constexpr size_t kStaticCoefBytes = (size_t)(kStaticMaxHeight / 2) * kStaticMaxTaps * sizeof(int16_t);
-constexpr size_t kStaticScratchBytes = kStaticCoefBytes + (size_t)(kStaticMaxHeight / 2) * sizeof(int32_t);
-static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
-
-namespace {
-constexpr int kMaxDevices = 64;
-std::mutex g_static_mu;
-void *g_scratch_dev[kMaxDevices] = {};        // device address of `scratch` per device
-std::map<int, VFilter> g_static_filters;       // host filter tables by height
-}  // namespace
-
-// The current device's address of `scratch`, looked up on the first call on
-// each device with that device current.
-static int static_scratch(void **out) {
-  int dev = 0;
-  NES_HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kMaxDevices) return NES_ENODEV;
-  std::lock_guard<std::mutex> lk(g_static_mu);
-  if (!g_scratch_dev[dev]) {
-    void *p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p) {
-      set_last_error(std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-      return NES_EIO;
-    }
-    g_scratch_dev[dev] = p;
-  }
-  *out = g_scratch_dev[dev];
-  return NES_OK;
-}
-
-// Host filter table of height h (built once per height; host memory only).
-static int static_filter(int h, const VFilter **out) {
-  std::lock_guard<std::mutex> lk(g_static_mu);
-  auto it = g_static_filters.find(h);
-  if (it == g_static_filters.end()) {
-    VFilter f = build_vchroma_filter(h);
-    if (f.taps < 1 || f.taps > kStaticMaxTaps || !filter_fits_tiles(f, h)) {
-      set_last_error("unsupported vertical filter size");
-      return NES_ERANGE;
-    }
-    it = g_static_filters.emplace(h, std::move(f)).first;
-  }
-  *out = &it->second;
-  return NES_OK;
-}
 
 }  // namespace nes
 
@@ -652,29 +760,14 @@ int nes_frameprep_device_static(const uint8_t *rgb_a, const float *depth_a,
   NES_TRY(frameprep_check(rgb_a, depth_a, rgb_b, depth_b, w, h, n_frames, y, y_stride, u,
                           u_stride, v, v_stride, sws_mode));
   if (h > kStaticMaxHeight) {
-    set_last_error("nes_frameprep_device_static: frame height above 8192 (its fixed scratch "
-                   "holds the chroma filter of at most 4096 rows)");
+    set_last_error("nes_frameprep_device_static: frame height above 8192");
     return NES_ERANGE;
   }
-  void *sp = nullptr;
-  NES_TRY(static_scratch(&sp));
-  const VFilter *f = nullptr;
-  NES_TRY(static_filter(h, &f));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  DevVFilter flt;
-  flt.taps = f->taps;
-  flt.coef = static_cast<int16_t *>(sp);
-  flt.pos = reinterpret_cast<int32_t *>(static_cast<uint8_t *>(sp) + kStaticCoefBytes);
-  // the table of this call's height replaces whatever the last call left
-  NES_HIP_TRY(hipMemcpyAsync(flt.coef, f->coef.data(), f->coef.size() * sizeof(int16_t),
-                             hipMemcpyHostToDevice, s));
-  NES_HIP_TRY(hipMemcpyAsync(flt.pos, f->pos.data(), f->pos.size() * sizeof(int32_t),
-                             hipMemcpyHostToDevice, s));
   const size_t px = (size_t)w * h;
-  NES_TRY(launch_frameprep_filter(rgb_a, depth_a, rgb_b, depth_b, w, h, n_frames, 3 * px, 4 * px,
-                                  y, y_stride, (size_t)y_stride * h, u, u_stride,
-                                  (size_t)u_stride * (h / 2), v, v_stride,
-                                  (size_t)v_stride * (h / 2), sws_mode, flt, s));
+  NES_TRY(launch_frameprep(rgb_a, depth_a, rgb_b, depth_b, w, h, n_frames, 3 * px, 4 * px, y, y_stride,
+                           (size_t)y_stride * h, u, u_stride, (size_t)u_stride * (h / 2), v, v_stride,
+                           (size_t)v_stride * (h / 2), sws_mode, s));
   if (!stream) NES_HIP_TRY(hipStreamSynchronize(s));
   return NES_OK;
 }
@@ -687,8 +780,6 @@ int nes_gray8_to_yuv420p(const uint8_t *gray, int w, int h, int g_stride,
   if (sws_mode != NES_SWS_X86 && sws_mode != NES_SWS_C) return NES_EINVAL;
   NES_TRY(ensure_device());
   std::lock_guard<std::mutex> lk(g_host_mu);
-  DevVFilter flt;
-  NES_TRY(get_dev_vfilter(h, &flt));
   const size_t px = (size_t)w * h, cw = (size_t)w / 2, chh = (size_t)h / 2;
   NES_TRY(g_in.reserve(px));
   NES_TRY(g_out.reserve(px + 2 * cw * chh));
@@ -696,11 +787,11 @@ int nes_gray8_to_yuv420p(const uint8_t *gray, int w, int h, int g_stride,
   uint8_t *d_g = g_in.as<uint8_t>();
   uint8_t *d_y = g_out.as<uint8_t>(), *d_u = d_y + px, *d_v = d_u + cw * chh;
   NES_HIP_TRY(hipMemcpy2DAsync(d_g, w, gray, g_stride, w, h, hipMemcpyHostToDevice, s));
-  dim3 grid((unsigned)((w + 255) / 256), (unsigned)h);
-  gray_kernel<false><<<grid, 256, 0, s>>>(d_g, w, w, h, d_y, w, d_u, (int)cw, d_v, (int)cw,
-                                          flt.coef, flt.pos, flt.taps, sws_mode, nullptr, 0.0f,
-                                          nullptr);
-  NES_HIP_TRY(hipGetLastError());
+  GrayArgs ga{};
+  ga.g = d_g; ga.g_stride = w;
+  ga.y = d_y; ga.u = d_u; ga.v = d_v;
+  ga.w = w; ga.h = h; ga.y_stride = w; ga.u_stride = ga.v_stride = (int)cw;
+  NES_TRY(launch_gray(ga, false, sws_mode, s));
   NES_HIP_TRY(hipMemcpy2DAsync(y, y_stride, d_y, w, w, h, hipMemcpyDeviceToHost, s));
   NES_HIP_TRY(hipMemcpy2DAsync(u, u_stride, d_u, cw, cw, chh, hipMemcpyDeviceToHost, s));
   NES_HIP_TRY(hipMemcpy2DAsync(v, v_stride, d_v, cw, cw, chh, hipMemcpyDeviceToHost, s));

@@ -124,13 +124,27 @@ struct VFilter {
 // RGB24 WxH -> YUV420P WxH context (bicubic default scaler).
 VFilter build_vchroma_filter(int h);
 
-// Device copy of a VFilter, cached per frame height.
-struct DevVFilter {
-  int taps = 0;
-  int16_t *coef = nullptr;
-  int32_t *pos = nullptr;
+// The same filter as kernel arguments.  Every even height from 12 on has one
+// 8-tap row for all chroma rows but the first two and the last two, starting
+// at source row 2k - 3; lower heights have at most five chroma rows.  So five
+// rows describe any height: chroma rows 0, 1, the interior, ch - 2, ch - 1
+// (row_class), zero-padded to 8 taps.
+constexpr int kVTaps = 8;
+constexpr int kVClasses = 5;
+struct VRows {
+  int taps = 0;                      // of the filter itself (its rounding term counts them)
+  int16_t coef[kVClasses][kVTaps] = {};
+  int32_t pos[kVClasses] = {};       // first source row (interior: 0, see row_pos)
 };
-int get_dev_vfilter(int h, DevVFilter *out);
+__host__ __device__ inline int row_class(int k, int ch) {
+  return k < 2 ? k : k >= ch - 2 ? kVClasses - (ch - k) : 2;
+}
+__host__ __device__ inline int row_pos(const VRows &f, int k, int ch) {
+  const int c = row_class(k, ch);
+  return c == 2 ? 2 * k - 3 : c == 0 ? f.pos[0] : c == 1 ? f.pos[1] : c == 3 ? f.pos[3] : f.pos[4];
+}
+// NES_ERANGE if the filter of height h does not have this form.
+int get_vrows(int h, VRows *out);
 
 hipStream_t library_stream();
 

@@ -83,3 +83,70 @@ def test_device_batch_bit_exact(nes, oracle):
         assert_planes_equal((y[i], u[i], v[i]), oracle.frameprep(*f, mode=0))
     for buf in bufs + [Y, U, V]:
         buf.free()
+
+
+def _device_planes(nes, bufs, w, h, n, mode, composite, off=0):
+    """nes_frameprep_device over raw device inputs `off` bytes into their
+    buffers, outputs `off` bytes into theirs; returns the planes."""
+    import ctypes as C
+    sizes = (n * w * h, n * (w // 2) * (h // 2), n * (w // 2) * (h // 2))
+    outs = [nes.DeviceBuffer(s + 64) for s in sizes]
+    guard = [np.full(s + 64, 0xA5, np.uint8) for s in sizes]
+    for b, g in zip(outs, guard):
+        b.upload(g)
+    at = lambda b: None if b is None else C.c_void_p(b.ptr.value + off)  # noqa: E731
+    a, da, b, db = bufs if composite else (bufs[0], None, None, None)
+    nes.check(nes.lib().nes_frameprep_device(at(a), at(da), at(b), at(db), w, h, n, at(outs[0]), w,
+                                             at(outs[1]), w // 2, at(outs[2]), w // 2, mode, None),
+              "nes_frameprep_device")
+    got = []
+    for o, g, s in zip(outs, guard, sizes):
+        o.download(g)
+        assert (g[:off] == 0xA5).all() and (g[off + s:] == 0xA5).all()  # nothing beside the planes
+        got.append(g[off:off + s].copy())
+        o.free()
+    return got
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("w,h,n,off", [
+    (2, 2, 3, 0), (2, 40, 1, 0), (4, 24, 1, 0), (6, 12, 2, 0),     # narrow, lowest heights with 8 taps
+    (254, 34, 1, 1), (258, 36, 1, 3), (262, 64, 2, 2),             # ragged strips at odd addresses
+    (640, 480, 1, 0), (642, 360, 8, 0), (514, 482, 16, 0),         # 4, 8 and 16 chroma rows per tile
+    (1282, 722, 21, 0),                                            # more than the Infinity Cache
+])
+def test_tile_shapes_and_alignments_bit_exact(nes, oracle, w, h, n, off, mode):
+    """Every tile height, the last partial strip and tile, widths of 4k + 2 and
+    2, addresses of any alignment and batches beyond the caches against the
+    CPU restatement (of the first, a middle and the last frame)."""
+    rng = np.random.default_rng(w * h + n)
+    host = (rng.integers(0, 256, (n, h, w, 3), dtype=np.uint8),
+            rng.uniform(0.1, 10.0, (n, h, w)).astype(np.float32),
+            rng.integers(0, 256, (n, h, w, 3), dtype=np.uint8),
+            rng.uniform(0.1, 10.0, (n, h, w)).astype(np.float32))
+    host[1][:, ::7, ::3] = np.nan
+    host[3][:, ::5, ::2] = np.nan
+    host[1][:, 1::9, 1::4] = np.inf
+    host[3][:, 2::6, ::5] = host[1][:, 2::6, ::5]
+    bufs = []
+    for x in host:
+        b = nes.DeviceBuffer(x.nbytes + 64)
+        b.upload(np.concatenate([np.zeros(off, np.uint8), x.reshape(-1).view(np.uint8)]))
+        bufs.append(b)
+    for composite in (True, False):
+        y, u, v = _device_planes(nes, bufs, w, h, n, mode, composite, off)
+        for i in sorted({0, n // 2, n - 1}):
+            ref = (oracle.frameprep(host[0][i], host[1][i], host[2][i], host[3][i], mode=mode) if composite
+                   else oracle.frameprep(host[0][i], host[1][i], mode=mode))
+            for g, r in zip((y, u, v), ref):
+                assert np.array_equal(g.reshape(n, *r.shape)[i], r), (composite, i)
+    for b in bufs:
+        b.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("w,h", [(2, 2), (4, 4), (6, 10), (254, 12), (258, 36), (1030, 100)])
+def test_gray_stream_shapes_bit_exact(nes, oracle, w, h, mode):
+    g = np.random.default_rng(w + h).integers(0, 256, (h, w), dtype=np.uint8)
+    for a, b in zip(nes.gray8_to_yuv420p(g, mode), oracle.gray8_to_yuv420p(g, mode)):
+        assert np.array_equal(a, b)
