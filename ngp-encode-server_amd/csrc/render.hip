@@ -12,7 +12,7 @@
 //                 XCD p encode levels p and 15-p, so each XCD's L2 caches two
 //                 levels of the table
 //   MLPs          density + colour MLPs over the dense sample list:
-//                   FP32:  mlp_train<false> (train.hip), FP32 features on
+//                   FP32:  mlp_f32 (train.hip), FP32 features on
 //                          v_mfma_f32_16x16x4_f32
 //                   mixed: mlp_mixed, FP16 features on
 //                          v_mfma_f32_16x16x32_f16, FP32 accumulation
