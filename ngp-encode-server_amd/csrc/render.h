@@ -200,6 +200,8 @@ int render_launch_frame(const SceneDev &scene, RenderWork &w, int precision, hip
 // the counts; updates first_pass_cap for the next frame.
 uint32_t render_frame_max_total(const RenderWork &w);
 FrameCounts render_frame_finish(RenderWork &w);
+// Device time between the frame's begin and end stamps in total_host.
+double frame_ms(const RenderWork &w);
 // Device bytes the sample buffers of `capacity` samples take (all buffers
 // that grow with the sample count).
 size_t sample_buffer_bytes(size_t capacity, int precision);

@@ -1345,11 +1345,10 @@ FrameCounts render_frame_finish(RenderWork &w) {
   return c;
 }
 
-// Single-stage launchers reused by the training step (rays and compositing
-// state already initialised by the caller, one output index per ray slot).
+// Single-stage launchers reused by the training step (rays prepared and the
+// sample cursor cleared by the caller, one output index per ray slot).
 int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStream_t stream) {
   const unsigned blocks = (unsigned)((w.n_slots + 255) / 256);
-  zero_u32<<<1, 64, 0, stream>>>(w.total.as<uint32_t>(), 2);
   march_emit<<<blocks, 256, 0, stream>>>(march_args(w, occ, k0, k1, kMarchPrepared, kMaxSteps));
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
@@ -1446,6 +1445,11 @@ static double tick_ms() {
   return ms;
 }
 
+double frame_ms(const RenderWork &w) {
+  const uint64_t *st = reinterpret_cast<const uint64_t *>(w.total_host + kTotStamps);
+  return st[kStampEnd] > st[kStampBegin] ? (double)(st[kStampEnd] - st[kStampBegin]) * tick_ms() : 0.0;
+}
+
 // Stage times of `passes` passes from the stamps of the last frame_end:
 // t[0..3] += march, encode, MLPs, composite; returns begin to end.
 static double add_stage_times(const RenderWork &w, int first_pass, int passes, double t[4]) {
@@ -1456,7 +1460,7 @@ static double add_stage_times(const RenderWork &w, int first_pass, int passes, d
     const uint64_t next = p + 1 < first_pass + passes ? s[kStampStages] : st[kStampEnd];
     for (int k = 0; k < kStampStages; ++k) t[k] += ms(s[k], k + 1 < kStampStages ? s[k + 1] : next);
   }
-  return ms(st[kStampBegin], st[kStampEnd]);
+  return frame_ms(w);
 }
 
 static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precision,

@@ -468,6 +468,9 @@ struct TrainRayArgs {
   float *target;         // [ray][3]
   const float *ray_o;    // explicit rays (optional)
   const float *ray_d;
+  uint32_t *total;       // RenderWork::total: sample cursor cleared, start stamped
+  uint32_t *buckets;     // kBuckets counters, cleared
+  uint32_t n_buckets;
 };
 
 __device__ __forceinline__ uint64_t mix64_d(uint64_t z) {
@@ -479,6 +482,13 @@ __device__ __forceinline__ uint64_t mix64_d(uint64_t z) {
 
 __global__ void train_rays(TrainRayArgs a) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) {
+      a.total[kTotCursor] = 0u;
+      reinterpret_cast<uint64_t *>(a.total + kTotStamps)[kStampBegin] = wall_clock64();
+    }
+    for (uint32_t b = threadIdx.x; b < a.n_buckets; b += blockDim.x) a.buckets[b] = 0u;
+  }
   if (i >= a.n_rays) return;
   RayData r;
   if (a.ray_o) {
@@ -558,7 +568,9 @@ __global__ __launch_bounds__(kLossThreads) void loss_sum(const float *partial, u
 __global__ __launch_bounds__(256) void train_dcomposite(
     uint32_t n_slots, const RayData *__restrict__ rays, const RayAcc *__restrict__ acc,
     const uint32_t *__restrict__ counts, const uint32_t *__restrict__ offsets,
-    const float4 *__restrict__ sout, const float *__restrict__ dC, float4 *__restrict__ dout) {
+    const float4 *__restrict__ sout, const float *__restrict__ dC, float4 *__restrict__ dout,
+    const uint32_t *__restrict__ n_ptr, uint32_t capacity) {
+  if (*n_ptr > capacity) return;  // overflowed: the host runs the step again
   const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = lane_id();
   const bool valid = slot < n_slots;
@@ -967,7 +979,9 @@ __global__ __launch_bounds__(kSliceThreads) void scatter_slices(
 }
 
 __global__ void adam_kernel(float *p, float *grad, float *m, float *v, size_t n, float lr,
-                            float b1, float b2, float eps, float c1, float c2) {
+                            float b1, float b2, float eps, float c1, float c2,
+                            const uint32_t *n_ptr, uint32_t capacity) {
+  if (*n_ptr > capacity) return;  // overflowed: the host runs the step again
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x) {
     const float gi = grad[i];
@@ -986,9 +1000,61 @@ __global__ void zero_f32(float *p, size_t n) {
     p[i] = 0.0f;
 }
 
+// A table in the device layout (and the weights behind it) into pinned host
+// memory in the packed layout, one level (or the weights) per blockIdx.y, 8
+// bytes per lane: the link takes 0.87 ms for the 48.8 MB; as one runtime copy
+// per level the hand-overs add 0.2 ms.  kClear: zeroes what was read.
+template <bool kClear>
+__global__ __launch_bounds__(256) void store_params(float *__restrict__ src, float2 *__restrict__ table,
+                                                    float *__restrict__ weights) {
+  const uint32_t step = gridDim.x * blockDim.x;
+  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.y == kLevels) {
+    float *w = src + 2 * (size_t)kDevTableEntries;
+    for (; i < (uint32_t)kWeights; i += step) {
+      if (weights) weights[i] = w[i];
+      if (kClear) w[i] = 0.0f;
+    }
+    return;
+  }
+  uint32_t from = 0, to = 0, n = 0;
+#pragma unroll
+  for (int l = 0; l < kLevels; ++l)
+    if ((int)blockIdx.y == l) {
+      from = kDevLevelOffset[l];
+      to = kLevelOffset[l];
+      n = kLevelOffset[l + 1] - kLevelOffset[l];
+    }
+  float2 *s = reinterpret_cast<float2 *>(src) + from;
+  for (; i < n; i += step) {
+    if (table) table[to + i] = s[i];
+    if (kClear) s[i] = make_float2(0.0f, 0.0f);
+  }
+}
+
+// The end of a call's device work: sample count, loss, stamps and (optional)
+// ray colours into pinned host memory.
+__global__ __launch_bounds__(256) void train_end(const uint32_t *total, const float *loss, uint32_t *host,
+                                                 const float *rgb, float *rgb_host, uint32_t n_rgb) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    host[kTotCursor] = total[kTotCursor];
+    host[kTotEvaluated] = __float_as_uint(loss ? *loss : 0.0f);
+    uint64_t *st = reinterpret_cast<uint64_t *>(host + kTotStamps);
+    st[kStampBegin] = reinterpret_cast<const uint64_t *>(total + kTotStamps)[kStampBegin];
+    st[kStampEnd] = wall_clock64();
+  }
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_rgb; i += gridDim.x * blockDim.x)
+    rgb_host[i] = rgb[i];
+}
+
 }  // namespace nes
 
 using namespace nes;
+
+// Explicit rays up to this count are staged in pinned memory and read over the
+// link by the kernels (three runtime copies of pageable memory take 15 us each
+// before the first kernel); more go through copies.
+constexpr uint32_t kStagedRays = 16384;
 
 struct nes_trainer {
   nes_train_config cfg{};
@@ -999,12 +1065,13 @@ struct nes_trainer {
   ViewDesc *poses = nullptr;
   float *targets = nullptr;
   float *target = nullptr, *loss = nullptr, *loss_part = nullptr;
-  DevBuf dout, dfeat, items, xo, xd, dCb;
+  DevBuf dout, dfeat, items, xo, xd, xg, dCb;
   uint32_t *bucket_count = nullptr, *bucket_off = nullptr, *bucket_cursor = nullptr;
   float *dC = nullptr;
   RenderWork work;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  float *rays_host = nullptr;     // pinned staging of explicit rays and their gradients
+  bool grads_dirty = false;       // grads may hold something (they are zero between calls)
   uint64_t step = 0;
   std::mutex mu;
 };
@@ -1034,51 +1101,123 @@ static int trainer_grow(nes_trainer *t, size_t cap) {
   NES_TRY(render_reserve_samples(t->work, NES_PRECISION_FP32, cap));
   NES_TRY(t->dout.reserve(sizeof(float4) * (cap + 1)));
   NES_TRY(t->dfeat.reserve(2 * sizeof(float4) * kParts * (cap + 1)));
-  // a step's samples stay below kMaxBucketSamples (checked in trainer_forward)
+  // a call's samples stay below kMaxBucketSamples (checked in trainer_finish)
   NES_TRY(t->items.reserve(sizeof(uint32_t) * kEntriesPerSample *
                            std::min<size_t>(cap + 1, kMaxBucketSamples)));
   return NES_OK;
 }
 
-// Forward of n_rays prepared by train_rays: samples, features, MLP outputs and
-// per-ray colour.  Re-runs with larger buffers when the samples overflow.
-static int trainer_forward(nes_trainer *t, uint32_t n_rays, const TrainRayArgs &ra) {
+// Every call queues its whole device work for the sample buffers as they are,
+// without a host round trip in between, and reads the sample count at its end.
+// Kernels write nothing beyond the capacity, and nothing that lasts when the
+// count exceeds it: such a call grows the buffers and runs once more.
+
+// Samples a call is expected to have (for launch sizes only).
+static uint32_t expected_samples(const RenderWork &w, uint32_t n_rays) {
+  const size_t last = w.last_total[0];
+  return (uint32_t)std::min<size_t>(std::max<size_t>(last ? last + last / 8 : (size_t)n_rays * 3, n_rays / 2), w.capacity);
+}
+
+// Forward of n_rays from train_rays: samples, features, MLP outputs and
+// per-ray colour.
+static int trainer_forward(nes_trainer *t, uint32_t n_rays, TrainRayArgs ra) {
   RenderWork &w = t->work;
   hipStream_t s = t->stream;
   NES_TRY(trainer_grow(t, std::max<size_t>(w.capacity, (size_t)n_rays * 4)));
+  ra.total = w.total.as<uint32_t>();
+  ra.buckets = t->bucket_count;
+  ra.n_buckets = kBuckets;
+  train_rays<<<(n_rays + 255) / 256, 256, 0, s>>>(ra);
+  NES_HIP_TRY(hipGetLastError());
+  NES_TRY(launch_march_emit(t->occ, w, 0, kMaxSteps, s));
+  NES_TRY(launch_encode_f32(t->params, w, expected_samples(w, n_rays), s));
+  NES_TRY(launch_mlp_f32(t->params + t->n_table, w, w.total.as<uint32_t>(), s));
+  return launch_composite(w, s);
+}
+
+// Waits for the call's device work; *again is set if the samples did not fit
+// and the buffers have been grown for another run.
+static int trainer_finish(nes_trainer *t, bool *again) {
+  RenderWork &w = t->work;
+  NES_HIP_TRY(hipStreamSynchronize(t->stream));
+  const uint32_t n = w.total_host[kTotCursor];
+  w.last_total[0] = n;
+  *again = false;
+  if (n >= kMaxBucketSamples) {
+    set_last_error("training step has " + std::to_string(n) +
+                   " samples, more than the gradient buckets index (" +
+                   std::to_string(kMaxBucketSamples) + ")");
+    return NES_ERANGE;
+  }
+  if (n <= w.capacity) return NES_OK;
+  *again = true;
+  return trainer_grow(t, (size_t)n + n / 8 + 1024);
+}
+
+// Runs `launch` (which ends with train_end) until its samples fit.
+template <class Launch>
+static int trainer_run(nes_trainer *t, Launch &&launch) {
   for (int attempt = 0; attempt < 2; ++attempt) {
-    train_rays<<<(n_rays + 255) / 256, 256, 0, s>>>(ra);
-    NES_HIP_TRY(hipGetLastError());
-    NES_TRY(launch_march_emit(t->occ, w, 0, kMaxSteps, s));
-    NES_HIP_TRY(hipMemcpyAsync(w.total_host, w.total.ptr, 4, hipMemcpyDeviceToHost, s));
-    NES_HIP_TRY(hipStreamSynchronize(s));
-    const uint32_t n = w.total_host[0];
-    if (n >= kMaxBucketSamples) {
-      set_last_error("training step has " + std::to_string(n) +
-                     " samples, more than the gradient buckets index (" +
-                     std::to_string(kMaxBucketSamples) + ")");
-      return NES_ERANGE;
-    }
-    if (n > w.capacity) {
-      NES_TRY(trainer_grow(t, (size_t)n + n / 8 + 1024));
-      continue;
-    }
-    NES_TRY(launch_encode_f32(t->params, w, n, s));
-    NES_TRY(launch_mlp_f32(t->params + t->n_table, w, w.total.as<uint32_t>(), s));
-    NES_TRY(launch_composite(w, s));
-    return NES_OK;
+    bool again = false;
+    int rc = launch();
+    if (rc != NES_OK) hipStreamSynchronize(t->stream);  // what was queued reads the call's staging
+    if (rc == NES_OK) rc = trainer_finish(t, &again);
+    if (rc != NES_OK || !again) return rc;
   }
   set_last_error("training sample buffers could not be grown");
   return NES_ENOMEM;
 }
 
-// Backward from dC (per ray, already on the device) into t->grads.
-static int trainer_backward(nes_trainer *t, uint32_t n_rays) {
+static int launch_train_end(nes_trainer *t, const float *loss, float *rgb_host, uint32_t n_rays) {
+  RenderWork &w = t->work;
+  const float *rgb = reinterpret_cast<const float *>(w.out.as<uint8_t>() + out_layout(w.out_px).rgbf);
+  const uint32_t n = rgb_host ? 3 * n_rays : 0u;
+  train_end<<<std::max(1u, std::min(64u, n / 1024)), 256, 0, t->stream>>>(w.total.as<uint32_t>(), loss, w.total_host, rgb,
+                                                                          rgb_host, n);
+  NES_HIP_TRY(hipGetLastError());
+  return NES_OK;
+}
+
+// The gradients are zero between calls; a call that failed half way leaves
+// that to the next one.
+static int trainer_clean_grads(nes_trainer *t) {
+  if (t->grads_dirty) zero_f32<<<1024, 256, 0, t->stream>>>(t->grads, t->n_params);
+  NES_HIP_TRY(hipGetLastError());
+  t->grads_dirty = true;
+  return NES_OK;
+}
+
+// Gradients to the caller (either may be null) and back to zero.
+static int trainer_take_grads(nes_trainer *t, float *grad_table, float *grad_weights) {
+  hipStream_t s = t->stream;
+  const bool pinned = (!grad_table || device_writable(grad_table, sizeof(float) * 2 * kTableEntries)) &&
+                      (!grad_weights || device_writable(grad_weights, sizeof(float) * kWeights)) &&
+                      (uintptr_t)grad_table % 8 == 0 && (uintptr_t)grad_weights % 4 == 0;
+  if (pinned) {
+    store_params<true><<<dim3(16, kLevels + 1), 256, 0, s>>>(t->grads, reinterpret_cast<float2 *>(grad_table), grad_weights);
+    NES_HIP_TRY(hipGetLastError());
+  } else {
+    if (grad_table)
+      NES_TRY(table_copy(grad_table, false, t->grads, true, sizeof(float), hipMemcpyDeviceToHost, s));
+    if (grad_weights)
+      NES_HIP_TRY(hipMemcpyAsync(grad_weights, t->grads + t->n_table, kWeights * sizeof(float),
+                                 hipMemcpyDeviceToHost, s));
+    zero_f32<<<1024, 256, 0, s>>>(t->grads, t->n_params);
+    NES_HIP_TRY(hipGetLastError());
+  }
+  NES_HIP_TRY(hipStreamSynchronize(s));
+  t->grads_dirty = false;
+  return NES_OK;
+}
+
+// Backward from dC (per ray, readable by the device) into t->grads.
+static int trainer_backward(nes_trainer *t, uint32_t n_rays, const float *dC) {
   RenderWork &w = t->work;
   hipStream_t s = t->stream;
   train_dcomposite<<<(n_rays + 255) / 256, 256, 0, s>>>(
       n_rays, w.rays.as<RayData>(), w.acc.as<RayAcc>(), w.counts.as<uint32_t>(),
-      w.offsets.as<uint32_t>(), w.sample_out.as<float4>(), t->dC, t->dout.as<float4>());
+      w.offsets.as<uint32_t>(), w.sample_out.as<float4>(), dC, t->dout.as<float4>(),
+      w.total.as<uint32_t>(), w.capacity);
   NES_HIP_TRY(hipGetLastError());
   TrainMlpArgs ma{};
   ma.pos = w.sample_pos.as<float4>();
@@ -1092,12 +1231,15 @@ static int trainer_backward(nes_trainer *t, uint32_t n_rays) {
   ma.grad_w = t->grads + t->n_table;
   mlp_train_bwd<<<256, 256, 0, s>>>(ma);
   NES_HIP_TRY(hipGetLastError());
-  zero_f32<<<1, 1024, 0, s>>>(reinterpret_cast<float *>(t->bucket_count), kBuckets);
+  // (the bucket counters were cleared by train_rays; items holds the entries
+  // of fewer than kMaxBucketSamples samples, more than that are refused at the
+  // end of the call)
+  const uint32_t most = std::min(w.capacity, kMaxBucketSamples - 1);
   bucket_count<<<kBucketBlocks, kBucketThreads, 0, s>>>(w.sample_pos.as<float4>(), w.total.as<uint32_t>(),
-                                                        w.capacity, t->bucket_count);
+                                                        most, t->bucket_count);
   bucket_scan<<<1, kBucketScanThreads, 0, s>>>(t->bucket_count, t->bucket_off, t->bucket_cursor);
   bucket_place<<<kBucketBlocks, kBucketThreads, 0, s>>>(w.sample_pos.as<float4>(), w.total.as<uint32_t>(),
-                                                        w.capacity, t->bucket_cursor, t->items.as<uint32_t>());
+                                                        most, t->bucket_cursor, t->items.as<uint32_t>());
   scatter_slices<<<kParts * kSliceTasksPerXcd, kSliceThreads, 0, s>>>(
       t->dfeat.as<float4>(), t->items.as<uint32_t>(), t->bucket_off,
       w.capacity, t->tasks, t->grads);
@@ -1118,11 +1260,12 @@ static TrainRayArgs step_rays(nes_trainer *t, uint64_t step) {
   return ra;
 }
 
-// Loss and gradients of one step's batch into t->grads (zeroed first).
-static int trainer_batch(nes_trainer *t, uint64_t step, float *loss_out) {
+// Loss and gradients of one step's batch into t->grads (launches only).
+static int trainer_batch(nes_trainer *t, uint64_t step) {
   const uint32_t n = t->cfg.rays_per_batch;
   hipStream_t s = t->stream;
   NES_TRY(trainer_prepare(t, n));
+  NES_TRY(trainer_clean_grads(t));
   NES_TRY(trainer_forward(t, n, step_rays(t, step)));
   const OutLayout L = out_layout(t->work.out_px);
   const float *rgbf = reinterpret_cast<const float *>(t->work.out.as<uint8_t>() + L.rgbf);
@@ -1130,12 +1273,13 @@ static int trainer_batch(nes_trainer *t, uint64_t step, float *loss_out) {
   train_loss<<<n_part, kLossThreads, 0, s>>>(rgbf, t->target, n, t->dC, t->loss_part);
   loss_sum<<<1, kLossThreads, 0, s>>>(t->loss_part, n_part, t->loss);
   NES_HIP_TRY(hipGetLastError());
-  NES_TRY(trainer_backward(t, n));
-  if (loss_out) {
-    NES_HIP_TRY(hipMemcpyAsync(loss_out, t->loss, 4, hipMemcpyDeviceToHost, s));
-    NES_HIP_TRY(hipStreamSynchronize(s));
-  }
-  return NES_OK;
+  return trainer_backward(t, n, t->dC);
+}
+
+static float loss_of(const nes_trainer *t) {
+  float l;
+  std::memcpy(&l, &t->work.total_host[kTotEvaluated], sizeof(l));
+  return l;
 }
 
 }  // namespace nes
@@ -1159,8 +1303,7 @@ int nes_trainer_create(const nes_scene_desc *init, const nes_train_config *cfg,
   auto build = [&]() -> int {
     t->n_params = t->n_table + kWeights;
     NES_HIP_TRY(hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking));
-    NES_HIP_TRY(hipEventCreate(&t->ev0));
-    NES_HIP_TRY(hipEventCreate(&t->ev1));
+    NES_HIP_TRY(hipHostMalloc((void **)&t->rays_host, kStagedRays * 9 * sizeof(float)));
     for (float **p : {&t->params, &t->grads, &t->m, &t->v})
       NES_HIP_TRY(hipMalloc(p, t->n_params * sizeof(float)));
     NES_HIP_TRY(hipMalloc(&t->occ, NES_OCC_WORDS * sizeof(uint32_t)));
@@ -1234,9 +1377,9 @@ int nes_trainer_destroy(nes_trainer *t) {
     if (p) hipFree(p);
   t->xo.release();
   t->xd.release();
+  t->xg.release();
   render_work_free(t->work);
-  if (t->ev0) hipEventDestroy(t->ev0);
-  if (t->ev1) hipEventDestroy(t->ev1);
+  if (t->rays_host) hipHostFree(t->rays_host);
   if (t->stream) hipStreamDestroy(t->stream);
   delete t;
   return NES_OK;
@@ -1245,26 +1388,24 @@ int nes_trainer_destroy(nes_trainer *t) {
 int nes_trainer_step(nes_trainer *t, float *loss, nes_train_stats *stats) {
   if (!t || !t->poses) return NES_EINVAL;
   std::lock_guard<std::mutex> lk(t->mu);
-  hipStream_t s = t->stream;
-  NES_HIP_TRY(hipEventRecord(t->ev0, s));
-  float l = 0.0f;
-  NES_TRY(trainer_batch(t, t->step, nullptr));
+  RenderWork &w = t->work;
+  const float c1 = 1.0f - std::pow(t->cfg.beta1, (float)(t->step + 1));
+  const float c2 = 1.0f - std::pow(t->cfg.beta2, (float)(t->step + 1));
+  NES_TRY(trainer_run(t, [&]() -> int {
+    NES_TRY(trainer_batch(t, t->step));
+    adam_kernel<<<4096, 256, 0, t->stream>>>(t->params, t->grads, t->m, t->v, t->n_params, t->cfg.lr,
+                                             t->cfg.beta1, t->cfg.beta2, t->cfg.eps, c1, c2,
+                                             w.total.as<uint32_t>(), w.capacity);
+    NES_HIP_TRY(hipGetLastError());
+    return launch_train_end(t, t->loss, nullptr, 0);
+  }));
+  t->grads_dirty = false;  // Adam leaves them zero
   t->step++;
-  const float c1 = 1.0f - std::pow(t->cfg.beta1, (float)t->step);
-  const float c2 = 1.0f - std::pow(t->cfg.beta2, (float)t->step);
-  adam_kernel<<<4096, 256, 0, s>>>(t->params, t->grads, t->m, t->v, t->n_params, t->cfg.lr,
-                                   t->cfg.beta1, t->cfg.beta2, t->cfg.eps, c1, c2);
-  NES_HIP_TRY(hipGetLastError());
-  NES_HIP_TRY(hipMemcpyAsync(&l, t->loss, 4, hipMemcpyDeviceToHost, s));
-  NES_HIP_TRY(hipEventRecord(t->ev1, s));
-  NES_HIP_TRY(hipEventSynchronize(t->ev1));
-  if (loss) *loss = l;
+  if (loss) *loss = loss_of(t);
   if (stats) {
-    float ms = 0.0f;
-    hipEventElapsedTime(&ms, t->ev0, t->ev1);
-    stats->ms = ms;
+    stats->ms = frame_ms(w);
     stats->rays = t->cfg.rays_per_batch;
-    stats->samples = t->work.total_host[0];
+    stats->samples = w.total_host[kTotCursor];
     stats->step = t->step;
   }
   return NES_OK;
@@ -1274,23 +1415,25 @@ int nes_trainer_batch_grad(nes_trainer *t, uint64_t step, float *loss, float *gr
                            float *grad_weights) {
   if (!t || !t->poses) return NES_EINVAL;
   std::lock_guard<std::mutex> lk(t->mu);
-  hipStream_t s = t->stream;
-  zero_f32<<<1024, 256, 0, s>>>(t->grads, t->n_params);
-  NES_TRY(trainer_batch(t, step, loss));
-  if (grad_table)
-    NES_TRY(table_copy(grad_table, false, t->grads, true, sizeof(float), hipMemcpyDeviceToHost, s));
-  if (grad_weights)
-    NES_HIP_TRY(hipMemcpyAsync(grad_weights, t->grads + t->n_table, kWeights * sizeof(float),
-                               hipMemcpyDeviceToHost, s));
-  zero_f32<<<1024, 256, 0, s>>>(t->grads, t->n_params);
-  NES_HIP_TRY(hipStreamSynchronize(s));
-  return NES_OK;
+  NES_TRY(trainer_run(t, [&]() -> int {
+    NES_TRY(trainer_batch(t, step));
+    return launch_train_end(t, t->loss, nullptr, 0);
+  }));
+  if (loss) *loss = loss_of(t);
+  return trainer_take_grads(t, grad_table, grad_weights);
 }
 
 int nes_trainer_get_params(nes_trainer *t, float *table, float *weights) {
   if (!t) return NES_EINVAL;
   std::lock_guard<std::mutex> lk(t->mu);
   NES_HIP_TRY(hipStreamSynchronize(t->stream));
+  if ((!table || (device_writable(table, sizeof(float) * 2 * kTableEntries) && (uintptr_t)table % 8 == 0)) &&
+      (!weights || (device_writable(weights, sizeof(float) * kWeights) && (uintptr_t)weights % 4 == 0))) {
+    store_params<false><<<dim3(16, kLevels + 1), 256, 0, t->stream>>>(t->params, reinterpret_cast<float2 *>(table), weights);
+    NES_HIP_TRY(hipGetLastError());
+    NES_HIP_TRY(hipStreamSynchronize(t->stream));
+    return NES_OK;
+  }
   if (table) NES_TRY(table_copy(table, false, t->params, true, sizeof(float), hipMemcpyDeviceToHost, nullptr));
   if (weights)
     NES_HIP_TRY(hipMemcpy(weights, t->params + t->n_table, kWeights * sizeof(float), hipMemcpyDeviceToHost));
@@ -1307,36 +1450,48 @@ int nes_trainer_set_params(nes_trainer *t, const float *table, const float *weig
   return NES_OK;
 }
 
-// Forward of explicit rays (n x 3 origins, unit directions) into the work
-// area, leaving their per-ray colour in its outputs.
-static int trainer_forward_rays(nes_trainer *t, const float *ray_o, const float *ray_d,
-                                uint32_t n) {
-  hipStream_t s = t->stream;
+// A caller's n x 3 array as the kernels read it: part `which` of the pinned
+// staging, or a device copy in `buf`.
+static int ray_input(nes_trainer *t, const float *src, uint32_t n, int which, DevBuf &buf, const float **out) {
+  if (n <= kStagedRays) {
+    float *p = t->rays_host + (size_t)which * 3 * kStagedRays;
+    std::memcpy(p, src, 12ull * n);
+    *out = p;
+    return NES_OK;
+  }
+  NES_TRY(buf.reserve(12ull * n));
+  NES_HIP_TRY(hipMemcpyAsync(buf.ptr, src, 12ull * n, hipMemcpyHostToDevice, t->stream));
+  *out = buf.as<float>();
+  return NES_OK;
+}
+
+// Work area and inputs of explicit rays (n x 3 origins, unit directions).
+static int explicit_rays(nes_trainer *t, const float *ray_o, const float *ray_d, uint32_t n, TrainRayArgs *ra) {
   NES_TRY(trainer_prepare(t, n));
-  NES_TRY(t->xo.reserve(12ull * n));
-  NES_TRY(t->xd.reserve(12ull * n));
-  NES_HIP_TRY(hipMemcpyAsync(t->xo.ptr, ray_o, 12ull * n, hipMemcpyHostToDevice, s));
-  NES_HIP_TRY(hipMemcpyAsync(t->xd.ptr, ray_d, 12ull * n, hipMemcpyHostToDevice, s));
-  TrainRayArgs ra{};
-  ra.n_rays = n;
-  ra.rays = t->work.rays.as<RayData>();
-  ra.ray_o = t->xo.as<float>();
-  ra.ray_d = t->xd.as<float>();
-  return trainer_forward(t, n, ra);
+  *ra = TrainRayArgs{};
+  ra->n_rays = n;
+  ra->rays = t->work.rays.as<RayData>();
+  NES_TRY(ray_input(t, ray_o, n, 0, t->xo, &ra->ray_o));
+  return ray_input(t, ray_d, n, 1, t->xd, &ra->ray_d);
 }
 
 int nes_trainer_forward(nes_trainer *t, const float *ray_o, const float *ray_d, uint32_t n,
                         float *rgb) {
   if (!t || !ray_o || !ray_d || !n || n > kMaxSlots) return NES_EINVAL;
   std::lock_guard<std::mutex> lk(t->mu);
-  hipStream_t s = t->stream;
-  NES_TRY(trainer_forward_rays(t, ray_o, ray_d, n));
-  if (rgb) {
+  TrainRayArgs ra;
+  NES_TRY(explicit_rays(t, ray_o, ray_d, n, &ra));
+  float *direct = rgb && device_writable(rgb, 12ull * n) && (uintptr_t)rgb % 4 == 0 ? rgb : nullptr;
+  NES_TRY(trainer_run(t, [&]() -> int {
+    NES_TRY(trainer_forward(t, n, ra));
+    return launch_train_end(t, nullptr, direct, n);
+  }));
+  if (rgb && !direct) {
     const OutLayout L = out_layout(t->work.out_px);
     NES_HIP_TRY(hipMemcpyAsync(rgb, t->work.out.as<uint8_t>() + L.rgbf, 12ull * n,
-                               hipMemcpyDeviceToHost, s));
+                               hipMemcpyDeviceToHost, t->stream));
+    NES_HIP_TRY(hipStreamSynchronize(t->stream));
   }
-  NES_HIP_TRY(hipStreamSynchronize(s));
   return NES_OK;
 }
 
@@ -1348,21 +1503,17 @@ int nes_trainer_backward(nes_trainer *t, const float *ray_o, const float *ray_d,
                          const float *d_rgb, float *grad_table, float *grad_weights) {
   if (!t || !ray_o || !ray_d || !d_rgb || !n || n > kMaxSlots) return NES_EINVAL;
   std::lock_guard<std::mutex> lk(t->mu);
-  hipStream_t s = t->stream;
-  NES_TRY(trainer_forward_rays(t, ray_o, ray_d, n));
-  NES_TRY(t->dCb.reserve(12ull * n));
-  t->dC = t->dCb.as<float>();
-  NES_HIP_TRY(hipMemcpyAsync(t->dC, d_rgb, 12ull * n, hipMemcpyHostToDevice, s));
-  zero_f32<<<1024, 256, 0, s>>>(t->grads, t->n_params);
-  NES_TRY(trainer_backward(t, n));
-  if (grad_table)
-    NES_TRY(table_copy(grad_table, false, t->grads, true, sizeof(float), hipMemcpyDeviceToHost, s));
-  if (grad_weights)
-    NES_HIP_TRY(hipMemcpyAsync(grad_weights, t->grads + t->n_table, kWeights * sizeof(float),
-                               hipMemcpyDeviceToHost, s));
-  zero_f32<<<1024, 256, 0, s>>>(t->grads, t->n_params);
-  NES_HIP_TRY(hipStreamSynchronize(s));
-  return NES_OK;
+  TrainRayArgs ra;
+  const float *g = nullptr;
+  NES_TRY(explicit_rays(t, ray_o, ray_d, n, &ra));
+  NES_TRY(ray_input(t, d_rgb, n, 2, t->xg, &g));
+  NES_TRY(trainer_run(t, [&]() -> int {
+    NES_TRY(trainer_clean_grads(t));
+    NES_TRY(trainer_forward(t, n, ra));
+    NES_TRY(trainer_backward(t, n, g));
+    return launch_train_end(t, nullptr, nullptr, 0);
+  }));
+  return trainer_take_grads(t, grad_table, grad_weights);
 }
 
 // ------------------------------------------------------------ checkpoint
