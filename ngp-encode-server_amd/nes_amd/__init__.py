@@ -15,6 +15,7 @@ there is no fallback path -- a missing or broken library raises.
 """
 import ctypes as C
 import os
+import threading
 
 import numpy as np
 
@@ -248,6 +249,85 @@ def _ptr(a, t):
     return a.ctypes.data_as(C.POINTER(t))
 
 
+# ------------------------------------------------- pinned output arrays
+
+class _PinnedBlock:
+    """One nes_host_alloc allocation; goes back to the pool with the last
+    array that uses it."""
+
+    __slots__ = ("ptr", "size", "pool")
+
+    def __init__(self, pool, ptr, size):
+        self.pool, self.ptr, self.size = pool, ptr, size
+
+    def __del__(self):
+        self.pool.give_back(self.ptr, self.size)
+
+
+class _PinnedPool:
+    """Pinned memory for the arrays that calls return: the library's kernels
+    store results straight into it, where an ordinary array costs a staged
+    copy and the page faults of fresh memory.  At most LIMIT bytes are
+    allocated (further arrays are ordinary ones) and at most KEEP of them stay
+    unused.  Any thread may take and drop arrays."""
+
+    LIMIT = 1 << 30
+    KEEP = 256 << 20
+
+    def __init__(self):
+        self.lock = threading.RLock()  # re-entered when a collection drops a block inside it
+        self.free = {}
+        self.allocated = self.unused = 0
+
+    @staticmethod
+    def size_class(nbytes):
+        """Sizes in steps of an eighth of their power of two, whole pages."""
+        step = max(4096, 1 << max(0, nbytes.bit_length() - 4))
+        return (nbytes + step - 1) // step * step
+
+    def take(self, nbytes):
+        size = self.size_class(nbytes)
+        with self.lock:
+            blocks = self.free.get(size)
+            if blocks:
+                self.unused -= size
+                return _PinnedBlock(self, blocks.pop(), size)
+            if self.allocated + size > self.LIMIT:
+                return None
+            self.allocated += size
+        p = C.c_void_p()
+        if lib().nes_host_alloc(size, C.byref(p)) != NES_OK or not p.value:
+            with self.lock:
+                self.allocated -= size
+            return None
+        return _PinnedBlock(self, p.value, size)
+
+    def give_back(self, ptr, size):
+        with self.lock:
+            if self.unused + size <= self.KEEP:
+                self.unused += size
+                self.free.setdefault(size, []).append(ptr)
+                return
+            self.allocated -= size
+        if _lib is not None:
+            _lib.nes_host_free(ptr)
+
+
+_pinned = _PinnedPool()
+
+
+def _out_array(shape, dtype):
+    """An uninitialised array for a call's results, in pinned memory if there
+    is some."""
+    nbytes = int(np.prod(shape)) * np.dtype(dtype).itemsize
+    block = _pinned.take(nbytes) if nbytes else None
+    if block is None:
+        return np.empty(shape, dtype)
+    buf = (C.c_uint8 * nbytes).from_address(block.ptr)
+    buf.block = block
+    return np.frombuffer(buf, dtype).reshape(shape)
+
+
 # ----------------------------------------------------------------- scene
 
 def scene_synthesize(seed, table_init=0):
@@ -307,11 +387,11 @@ class Context:
         outs = (ViewOut * n)()
         results = []
         for i, c in enumerate(cams):
-            r = {"rgb24": np.empty((c.height, c.width, 3), np.uint8),
-                 "depth": np.empty((c.height, c.width), np.float32),
-                 "rgb": np.empty((c.height, c.width, 3), np.float32),
-                 "n_samples": np.empty((c.height, c.width), np.uint16),
-                 "depth_gray8": np.empty((c.height, c.width), np.uint8)}
+            r = {"rgb24": _out_array((c.height, c.width, 3), np.uint8),
+                 "depth": _out_array((c.height, c.width), np.float32),
+                 "rgb": _out_array((c.height, c.width, 3), np.float32),
+                 "n_samples": _out_array((c.height, c.width), np.uint16),
+                 "depth_gray8": _out_array((c.height, c.width), np.uint8)}
             outs[i] = ViewOut(_ptr(r["rgb24"], C.c_uint8), _ptr(r["depth"], C.c_float),
                               _ptr(r["rgb"], C.c_float), _ptr(r["n_samples"], C.c_uint16),
                               _ptr(r["depth_gray8"], C.c_uint8), depth_far)
@@ -753,15 +833,15 @@ class Trainer:
 
     def batch_grad(self, step):
         loss = C.c_float()
-        gt = np.empty(TABLE_ENTRIES * 2, np.float32)
-        gw = np.empty(MLP_WEIGHTS, np.float32)
+        gt = _out_array((TABLE_ENTRIES * 2,), np.float32)
+        gw = _out_array((MLP_WEIGHTS,), np.float32)
         check(lib().nes_trainer_batch_grad(self.handle, step, C.byref(loss), _ptr(gt, C.c_float),
                                            _ptr(gw, C.c_float)), "nes_trainer_batch_grad")
         return loss.value, gt, gw
 
     def get_params(self):
-        t = np.empty(TABLE_ENTRIES * 2, np.float32)
-        w = np.empty(MLP_WEIGHTS, np.float32)
+        t = _out_array((TABLE_ENTRIES * 2,), np.float32)
+        w = _out_array((MLP_WEIGHTS,), np.float32)
         check(lib().nes_trainer_get_params(self.handle, _ptr(t, C.c_float), _ptr(w, C.c_float)),
               "nes_trainer_get_params")
         return t, w
@@ -775,7 +855,7 @@ class Trainer:
     def forward(self, ray_o, ray_d):
         o = np.ascontiguousarray(ray_o, np.float32)
         d = np.ascontiguousarray(ray_d, np.float32)
-        rgb = np.empty((len(o), 3), np.float32)
+        rgb = _out_array((len(o), 3), np.float32)
         check(lib().nes_trainer_forward(self.handle, _ptr(o, C.c_float), _ptr(d, C.c_float), len(o),
                                         _ptr(rgb, C.c_float)), "nes_trainer_forward")
         return rgb
@@ -788,8 +868,8 @@ class Trainer:
         g = np.ascontiguousarray(d_rgb, np.float32)
         if g.shape != (len(o), 3) or d.shape != o.shape:
             raise ValueError("ray_o, ray_d and d_rgb must be n x 3")
-        gt = np.empty(TABLE_ENTRIES * 2, np.float32)
-        gw = np.empty(MLP_WEIGHTS, np.float32)
+        gt = _out_array((TABLE_ENTRIES * 2,), np.float32)
+        gw = _out_array((MLP_WEIGHTS,), np.float32)
         check(lib().nes_trainer_backward(self.handle, _ptr(o, C.c_float), _ptr(d, C.c_float), len(o),
                                          _ptr(g, C.c_float), _ptr(gt, C.c_float),
                                          _ptr(gw, C.c_float)), "nes_trainer_backward")

@@ -428,3 +428,17 @@ def test_pinned_outputs_of_multi_pass_frames(nes, oracle, prec):
         assert passes > 1
         for k in ALL:
             assert np.array_equal(want[0][k], got[0][k]), k
+
+
+def test_returned_arrays_are_the_callers(nes, gpu_ctx):
+    """Arrays of earlier renders keep their values through later ones (their
+    memory is reused only once they are gone)."""
+    cams = [nes.camera(320, 200, nes.orbit_camera(30.0 * i, 20.0)) for i in range(4)]
+    first = [gpu_ctx.render(c)[0][0] for c in cams]
+    copies = [{k: v.copy() for k, v in r.items()} for r in first]
+    for _ in range(3):
+        for c in cams[::-1]:
+            gpu_ctx.render(c)
+    for r, k in zip(first, copies):
+        for name in k:
+            assert np.array_equal(r[name], k[name]), name
