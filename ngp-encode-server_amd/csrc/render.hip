@@ -446,22 +446,47 @@ __device__ __forceinline__ void store_background(const BackgroundArgs &a, uint32
 // the corner gathers hit in L2 instead of streaming 64-byte lines from the
 // Infinity Cache.  (In FP32 a hashed level alone is 4 MB.)  Features go to
 // feat[p][sample] as {level p f0, f1, level 15-p f0, f1}.
+//
+// Parts 0, 1 and 2 take longer than the others where neighbouring rays lie
+// several cells of the finest levels apart: level 15's four L2 requests per
+// sample fill XCD 0's request rate, while XCD 7 is done in two thirds of the
+// time.  So XCD 7 - p encodes the last share[p] of part p's samples (in 1 /
+// 65536) once its own part is done: in turn, so that its L2 holds two levels
+// at a time.  Stereo 1080p, times of the parts alone, us:
+//   996 951 844 775 779 714 700 659, together 1040; with shares 950
+// (1440x1600 at 75 degrees 1229 -> 1064, 2064x2208 2263 -> 1995).
+constexpr int kHelpedParts = 3;
+struct PartShares {
+  uint32_t share[kHelpedParts];
+};
+
+// Samples of part P beyond its own XCD's share start here (a multiple of the
+// workgroup size, so that a workgroup works on one part at a time).
+__device__ __forceinline__ uint32_t part_end(uint32_t n, uint32_t share) {
+  return (n - (uint32_t)((uint64_t)n * share >> 16)) & ~255u;
+}
+
+// Samples [from + i, to) of part P for i, i + step, ...; returns the first i
+// past them.
 template <class Tab, int P>
-__device__ __forceinline__ void encode_part_loop(const typename PosIn<Tab>::type *__restrict__ pos,
-                                                 uint32_t n, uint32_t stride, const Tab *table,
-                                                 typename PartOut<Tab>::type *__restrict__ feat,
-                                                 uint32_t grp, uint32_t blocks_per_part,
-                                                 uint32_t *xch) {
+__device__ __forceinline__ uint32_t encode_part_loop(const typename PosIn<Tab>::type *__restrict__ pos,
+                                                     uint32_t from, uint32_t to, uint32_t stride,
+                                                     const Tab *table,
+                                                     typename PartOut<Tab>::type *__restrict__ feat,
+                                                     uint32_t i, uint32_t step, uint32_t *xch) {
   constexpr int LA = P, LB = 15 - P;
   const char *base_a = level_base<Tab, LA>(table), *base_b = level_base<Tab, LB>(table);
   typename PartOut<Tab>::type *dst = feat + (size_t)P * stride;
-  for (uint32_t s = grp * blockDim.x + threadIdx.x; s < n; s += blocks_per_part * blockDim.x) {
+  const uint32_t count = to - from;
+  for (; i < count; i += step) {
+    const uint32_t s = from + i;
     float xc[3];
     PosIn<Tab>::get(pos[s], xc);
     float2 fa, fb;
     encode_two<Tab, LA, LB>(base_a, base_b, xc, fa, fb, xch);
     dst[s] = PartOut<Tab>::pack(fa, fb);
   }
+  return i - count;
 }
 
 // Each part is its own instantiation, so level resolutions, offsets and the
@@ -471,8 +496,8 @@ __global__ __launch_bounds__(256) void encode_parts(const typename PosIn<Tab>::t
                                                     const uint32_t *__restrict__ n_ptr,
                                                     uint32_t stride, const Tab *__restrict__ table,
                                                     typename PartOut<Tab>::type *__restrict__ feat,
-                                                    uint32_t blocks_per_part, BackgroundArgs bg,
-                                                    uint64_t *stamp) {
+                                                    uint32_t blocks_per_part, PartShares shares,
+                                                    BackgroundArgs bg, uint64_t *stamp) {
   stamp_start(stamp);
   __shared__ uint32_t xch_all[4][256];  // per-wavefront gather exchange (FP16 hashed levels)
   // the first workgroups (a multiple of kParts of them) store background pixels
@@ -482,17 +507,29 @@ __global__ __launch_bounds__(256) void encode_parts(const typename PosIn<Tab>::t
   }
   uint32_t *xch = xch_all[threadIdx.x >> 6];
   const uint32_t n = min(*n_ptr, stride);
-  const uint32_t grp = (blockIdx.x - bg.groups) / kParts;
+  uint32_t i = (blockIdx.x - bg.groups) / kParts * blockDim.x + threadIdx.x;
+  const uint32_t step = blocks_per_part * blockDim.x;
+#define NES_PART(P, FROM, TO) i = encode_part_loop<Tab, P>(pos, FROM, TO, stride, table, feat, i, step, xch)
   switch (blockIdx.x % kParts) {
-    case 0: encode_part_loop<Tab, 0>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    case 1: encode_part_loop<Tab, 1>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    case 2: encode_part_loop<Tab, 2>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    case 3: encode_part_loop<Tab, 3>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    case 4: encode_part_loop<Tab, 4>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    case 5: encode_part_loop<Tab, 5>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    case 6: encode_part_loop<Tab, 6>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
-    default: encode_part_loop<Tab, 7>(pos, n, stride, table, feat, grp, blocks_per_part, xch); break;
+    case 0: NES_PART(0, 0u, part_end(n, shares.share[0])); break;
+    case 1: NES_PART(1, 0u, part_end(n, shares.share[1])); break;
+    case 2: NES_PART(2, 0u, part_end(n, shares.share[2])); break;
+    case 3: NES_PART(3, 0u, n); break;
+    case 4: NES_PART(4, 0u, n); break;
+    case 5:
+      NES_PART(5, 0u, n);
+      NES_PART(2, part_end(n, shares.share[2]), n);
+      break;
+    case 6:
+      NES_PART(6, 0u, n);
+      NES_PART(1, part_end(n, shares.share[1]), n);
+      break;
+    default:
+      NES_PART(7, 0u, n);
+      NES_PART(0, part_end(n, shares.share[0]), n);
+      break;
   }
+#undef NES_PART
 }
 
 // FP16 MFMA MLPs: lane (g, j) of a 16-sample tile loads parts 2g and 2g+1 of
@@ -1182,6 +1219,20 @@ static size_t expected_samples(const RenderWork &w, int pass) {
   return std::min<size_t>(est, w.capacity);
 }
 
+// Shares of the mixed encode's first parts (see encode_parts): how far apart
+// neighbouring samples are, and with it what part 0 costs above part 7, follows
+// the focal length in pixels: 12 % at 416 (640x480 at 60 degrees), 52 % at 935
+// (1080p), 75 % at 1439 (2064x2208 at 75 degrees).  The shares start at 500
+// and reach 12, 9 and 4 % at 935, 21, 15 and 6 % from 1250 on.  Below 500 they
+// gain nothing; a fifth more or less of them costs 1 to 3 %.
+static PartShares part_shares(const RenderWork &w) {
+  double focal = 0.0;
+  for (uint32_t i = 0; i < w.n_views; ++i)
+    focal += (double)w.host_views[i].focal * w.host_views[i].slot_count / w.n_slots;
+  const double f = std::min(std::max((focal - 500.0) / 600.0, 0.0), 1.25);
+  return PartShares{{(uint32_t)(0.17 * f * 65536), (uint32_t)(0.12 * f * 65536), (uint32_t)(0.05 * f * 65536)}};
+}
+
 int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int k0, int k1,
                        bool first, bool last, hipStream_t stream, uint32_t ray_cap, bool resume) {
   const unsigned blocks = (unsigned)((w.n_slots + 255) / 256);
@@ -1205,13 +1256,14 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
   // grids for the expected samples, with grid-stride loops: the sample count
   // stays on the device
   const size_t expect = expected_samples(w, first ? 0 : 1);
-  const uint32_t bpp = part_blocks(expect);
+  const PartShares shares = f32 ? PartShares{} : part_shares(w);
+  const uint32_t bpp = part_blocks(expect + (expect * shares.share[0] >> 16));
   BackgroundArgs bg = background_args(w);
   if (!first) bg.groups = 0;
   if (f32) {
     encode_parts<float><<<bpp * kParts + bg.groups, 256, 0, stream>>>(w.sample_pos.as<float4>(), cursor, cap,
                                                            scene.table_f32, w.feat.as<float4>(),
-                                                           bpp, bg, stamp + 1);
+                                                           bpp, shares, bg, stamp + 1);
     NES_HIP_TRY(hipGetLastError());
     if (precision == NES_PRECISION_FP32_VALU)
       mlp_fp32_valu<<<256 * 4, 256, 0, stream>>>(w.sample_pos.as<float4>(), w.feat.as<float4>(),
@@ -1223,7 +1275,7 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
   } else {
     encode_parts<_Float16><<<bpp * kParts + bg.groups, 256, 0, stream>>>(w.sample_pos.as<uint2>(), cursor,
                                                               cap, scene.table_f16,
-                                                              w.feat.as<uint2>(), bpp, bg, stamp + 1);
+                                                              w.feat.as<uint2>(), bpp, shares, bg, stamp + 1);
     NES_HIP_TRY(hipGetLastError());
     const unsigned mlp_blocks =
         (unsigned)std::min<size_t>(256 * 8, std::max<size_t>(expect / (16 * kEvalWaves), 64));
@@ -1358,7 +1410,7 @@ int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t
   const uint32_t bpp = part_blocks(n);
   encode_parts<float><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<float4>(),
                                                          w.total.as<uint32_t>(), w.capacity,
-                                                         table, w.feat.as<float4>(), bpp, BackgroundArgs{},
+                                                         table, w.feat.as<float4>(), bpp, PartShares{}, BackgroundArgs{},
                                                          nullptr);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;

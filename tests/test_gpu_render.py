@@ -442,3 +442,20 @@ def test_returned_arrays_are_the_callers(nes, gpu_ctx):
     for r, k in zip(first, copies):
         for name in k:
             assert np.array_equal(r[name], k[name]), name
+
+
+@pytest.mark.parametrize("w,h", [(17, 9), (64, 48), (257, 131)])
+def test_encode_shares_change_no_result(nes, gpu_ctx, w, h):
+    """The XCDs share the encode's parts by the views' mean focal length: a
+    narrow view (shares at their largest) equals the same view in batches whose
+    other views move the shares, down to none."""
+    narrow = [nes.camera(w, h, nes.orbit_camera(50.0 * i, 15.0), fov=f) for i, f in enumerate((0.3, 1.5, 4.0))]
+    wide = nes.camera(320, 200, nes.orbit_camera(10.0, 25.0), fov=80.0)
+    for v in narrow:
+        (alone,), st = gpu_ctx.render(v)
+        assert st.samples > 0
+        for batch in ([v, wide], [wide, wide, wide, v], narrow + [v]):
+            outs, _ = gpu_ctx.render(batch)
+            got = outs[batch.index(v)]
+            for k in alone:
+                assert np.array_equal(alone[k], got[k]), k
