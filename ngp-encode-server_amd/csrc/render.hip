@@ -284,6 +284,208 @@ __global__ __launch_bounds__(256) void march_emit(MarchArgs m) {
 }
 
 
+// The same for few rays, which leave the chip idle while each wavefront works
+// through its chain of steps and samples: one workgroup per tile, four lanes
+// per ray, each testing a quarter of the ray's steps and emitting what it
+// found.  The list is laid out as march_emit lays it out: rank r of ray l at
+// start[r] + |{rays < l with more than r samples}|, from the ranks' ray masks.
+// 64x48: 24.0 -> 11.4 us, 320x240: 24.6 -> 14.5 us, 4096 rays of a batch:
+// 29 -> 14 us.
+__global__ __launch_bounds__(256) void march_emit_split(MarchArgs m) {
+  stamp_start(m.stamp);
+  __shared__ uint32_t ray_n[64];
+  __shared__ uint64_t rank_rays[kMaxSteps];
+  __shared__ uint32_t rank_at[kMaxSteps];
+  __shared__ uint32_t block_base;
+  const int lane = lane_id();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t ray = threadIdx.x >> 2, seg = threadIdx.x & 3u;
+  const uint32_t slot = blockIdx.x * 64 + ray;
+  const bool valid = slot < m.n_slots;
+  RayData r;
+  r.n_steps = 0;
+  uint32_t state = 0;
+  int k = m.k_begin;
+  if (m.mode == kMarchFirst) {
+    const uint32_t tslot = blockIdx.x * 64;
+    const ViewDesc &v = m.views[view_of(m.views, m.n_views, tslot)];
+    const uint32_t tile = (tslot - v.slot_base) >> 6;
+    const uint32_t px0 = (tile % v.tiles_x) * 8, py0 = (tile / v.tiles_x) * 8;
+    const uint32_t px = px0 + (ray & 7), py = py0 + (ray >> 3);
+    if (!tile_misses(v, px0, py0) && px < v.width && py < v.height) {
+      make_ray(v, px, py, r.o, r.d);
+      r.n_steps = ray_box(r.o, r.d, &r.t_start);
+    } else {
+      r.o[0] = r.o[1] = r.o[2] = 0.0f;
+      r.d[0] = r.d[1] = r.d[2] = 0.0f;
+      r.t_start = 0.0f;
+    }
+    if (m.store_rays == 2 && seg == 0) m.rays[slot] = r;
+  } else if (valid) {
+    if (m.mode == kMarchPrepared) {
+      r = load_ray(m.rays, slot);
+    } else {
+      const uint32_t prev = m.counts[slot];
+      state = prev & (kRayState | kRayDone);
+      if (!(prev & kRayDone) && (!m.resume || (prev & kRayState))) r = load_ray(m.rays, slot);
+      if (m.resume) k = max(k, (int)(prev >> 16));
+    }
+  }
+  // this lane's quarter of the ray's steps
+  const int kend = min(m.k_end, (int)r.n_steps);
+  const int quarter = (max(kend - k, 0) + 3) >> 2;
+  const int k0 = k + (int)seg * quarter, k1 = min(k0 + quarter, kend);
+  uint32_t hits = 0;  // occupied steps, from k0 on
+  if (k0 < k1) {
+    float o128[3], d128[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      o128[a] = 128.0f * r.o[a];
+      d128[a] = 128.0f * r.d[a];
+    }
+    for (int g = k0; g < k1; g += kStepUnroll) {
+      uint32_t word[kStepUnroll], cell[kStepUnroll];
+      const float kf = (float)g + 0.5f;
+#pragma unroll
+      for (int u = 0; u < kStepUnroll; ++u) {
+        const float t = fmaf(kf + (float)u, kDelta, r.t_start);
+        float x[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) x[a] = fmaf(t, d128[a], o128[a]);
+        cell[u] = occ_cell(x);
+        word[u] = __ldg(m.occ + (cell[u] >> 5));
+      }
+      uint32_t hit = 0;
+#pragma unroll
+      for (int u = 0; u < kStepUnroll; ++u) hit |= ((word[u] >> (cell[u] & 31u)) & 1u) << u;
+      if (k1 - g < kStepUnroll) hit &= (1u << (k1 - g)) - 1u;
+      hits |= hit << (g - k0);
+    }
+  }
+  // samples of the ray's earlier quarters and of all of them, cut at the cap
+  uint32_t n = (uint32_t)__popc(hits), before = 0, all = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t c = (uint32_t)__shfl((int)n, (lane & ~3) + q);
+    if (q < (int)seg) before += c;
+    all += c;
+  }
+  uint32_t knext = (uint32_t)max(kend, k);
+  if (all >= m.cap) {
+    const uint32_t keep = before < m.cap ? min(n, m.cap - before) : 0u;
+    for (; n > keep; --n) hits &= ~(0x80000000u >> __clz(hits));
+    // one step past the cap-th sample, which one lane of the ray holds
+    uint32_t past = n && before + n == m.cap ? (uint32_t)(k0 + 32 - __clz(hits)) : 0u;
+    past = max(past, (uint32_t)__shfl_xor((int)past, 1));
+    past = max(past, (uint32_t)__shfl_xor((int)past, 2));
+    knext = past;
+    all = m.cap;
+  }
+  if (valid && seg == 0) {
+    m.counts[slot] = all | state | (knext << 16);
+    if (all) {
+      m.t_start[slot] = r.t_start;
+      if (m.store_rays == 1) m.rays[slot] = r;
+    }
+  }
+  if (seg == 0) ray_n[ray] = all;
+  if (m.ray_sh && all) {
+    // the colour MLP's SH input of this ray, a quarter per lane
+    float sh[16];
+    sh4(r.d, sh);
+    uint32_t hw[2] = {0u, 0u};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q == (int)seg)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          half2v h;
+          h[0] = (_Float16)sh[4 * q + 2 * i];
+          h[1] = (_Float16)sh[4 * q + 2 * i + 1];
+          hw[i] = __builtin_bit_cast(uint32_t, h);
+        }
+    m.ray_sh[(size_t)slot * 4 + seg] = make_uint2(hw[0], hw[1]);
+  }
+  __syncthreads();
+  // every wavefront sees the 64 counts; the ranks' masks are dealt to them
+  const uint32_t c = ray_n[lane];
+  const uint32_t mx = wave_max(c);
+  if (wave == 0) {
+    const uint32_t total = wave_sum(c);
+    if (lane == 0) {
+      block_base = total ? atomicAdd(m.cursor, total) : 0u;
+      if (m.mode == kMarchFirst) m.tile_n[blockIdx.x] = total;
+      if (total) m.offsets[blockIdx.x] = block_base;
+    }
+  }
+  if (mx == 0) return;  // the same in every wavefront
+  for (uint32_t i = wave; i < mx; i += 4) {
+    const uint64_t has = __ballot(c > i);
+    if (lane == 0) rank_rays[i] = has;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // exclusive prefix sums of the ranks' sizes, two ranks per lane
+    const uint32_t i0 = 2 * (uint32_t)lane;
+    const uint32_t n0 = i0 < mx ? (uint32_t)__popcll(rank_rays[i0]) : 0u;
+    const uint32_t n1 = i0 + 1 < mx ? (uint32_t)__popcll(rank_rays[i0 + 1]) : 0u;
+    uint32_t inc = n0 + n1;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t o = __shfl_up(inc, d);
+      if (lane >= d) inc += o;
+    }
+    rank_at[i0] = inc - n0 - n1;
+    rank_at[i0 + 1] = inc - n1;
+  }
+  __syncthreads();
+  const uint32_t base = block_base;
+  const uint64_t below = lanes_below((int)ray);
+  const float scale = m.packed ? 2097152.0f : 1.0f;
+  float os[3], ds[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    os[a] = scale * r.o[a];
+    ds[a] = scale * r.d[a];
+  }
+  for (uint32_t rank = before; hits; ++rank) {
+    const int ks = k0 + __builtin_ctz(hits);
+    hits &= hits - 1;
+    const uint32_t at = base + rank_at[rank] + (uint32_t)__popcll(rank_rays[rank] & below);
+    if (at >= m.capacity) continue;
+    const float t = step_t(ks, r.t_start);
+    float x[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) x[a] = fmaf(t, ds[a], os[a]);
+    if (m.packed)
+      reinterpret_cast<uint2 *>(m.pos)[at] = pack_pos21(x);
+    else
+      m.pos[at] = make_float4(fminf(fmaxf(x[0], 0.0f), 1.0f), fminf(fmaxf(x[1], 0.0f), 1.0f),
+                              fminf(fmaxf(x[2], 0.0f), 1.0f), __uint_as_float(slot));
+    m.samples[at] = (slot << 7) | (uint32_t)ks;
+  }
+}
+
+// Ray slots up to which the march runs four lanes per ray.  Past that the chip
+// is full either way and a ray's set-up, done by all four, costs more than the
+// shorter chains give (march_emit -> march_emit_split, us): 173k slots
+// 24.6 -> 16.5, 307k 25.9 -> 24.3, 614k 29.7 -> 29.9, 1.0M 39.6 -> 45.2,
+// 4.1M 73 -> 135.
+constexpr uint32_t kSplitSlots = 1u << 19;
+// The same for a batch of rays, whose tiles all have rays that cross the cube,
+// where a frame's mostly miss it: 16k rays 25.1 -> 14.8, 65k 23.8 -> 25.0,
+// 131k 27 -> 38.
+constexpr uint32_t kSplitBatchRays = 1u << 15;
+
+static int launch_march(const MarchArgs &m, hipStream_t stream) {
+  if (m.n_slots <= (m.mode == kMarchPrepared ? kSplitBatchRays : kSplitSlots))
+    march_emit_split<<<(unsigned)((m.n_slots + 63) / 64), 256, 0, stream>>>(m);
+  else
+    march_emit<<<(unsigned)((m.n_slots + 255) / 256), 256, 0, stream>>>(m);
+  NES_HIP_TRY(hipGetLastError());
+  return NES_OK;
+}
+
 constexpr int kEvalWaves = 4;
 
 // ------------------------------------------------------ FP32 VALU eval
@@ -1252,8 +1454,7 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
   m.store_rays = !first ? 0 : k1 < kMaxSteps ? 2 : !last || f32 ? 1 : 0;
   m.ray_sh = f32 ? nullptr : w.ray_sh.as<uint2>();
   m.stamp = stamp;
-  march_emit<<<blocks, 256, 0, stream>>>(m);
-  NES_HIP_TRY(hipGetLastError());
+  NES_TRY(launch_march(m, stream));
   // grids for the expected samples, with grid-stride loops: the sample count
   // stays on the device
   const size_t expect = expected_samples(w, first ? 0 : 1);
@@ -1401,10 +1602,7 @@ FrameCounts render_frame_finish(RenderWork &w) {
 // Single-stage launchers reused by the training step (rays prepared and the
 // sample cursor cleared by the caller, one output index per ray slot).
 int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStream_t stream) {
-  const unsigned blocks = (unsigned)((w.n_slots + 255) / 256);
-  march_emit<<<blocks, 256, 0, stream>>>(march_args(w, occ, k0, k1, kMarchPrepared, kMaxSteps));
-  NES_HIP_TRY(hipGetLastError());
-  return NES_OK;
+  return launch_march(march_args(w, occ, k0, k1, kMarchPrepared, kMaxSteps), stream);
 }
 
 int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t stream) {

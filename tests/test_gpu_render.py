@@ -459,3 +459,28 @@ def test_encode_shares_change_no_result(nes, gpu_ctx, w, h):
             got = outs[batch.index(v)]
             for k in alone:
                 assert np.array_equal(alone[k], got[k]), k
+
+
+@pytest.mark.parametrize("prec", [FP32, MIXED])
+@pytest.mark.parametrize("sigma", [None, 30.0])
+def test_small_and_large_batches_agree(nes, gpu_ctx, prec, sigma):
+    """Batches below 2^19 ray slots march with four lanes per ray, larger ones
+    with one: small views alone, whole and in windows of steps, equal the same
+    views beside one of 2^20 slots (with sigma = 30, rays that end within the
+    cube, in one pass, in two and in windows)."""
+    views = [nes.camera(w, h, nes.orbit_camera(35.0 * i, 18.0), fov=f)
+             for i, (w, h, f) in enumerate(((1, 1, 5.0), (8, 8, 20.0), (33, 17, 40.0), (130, 67, 60.0)))]
+    large = nes.camera(1024, 1024, nes.orbit_camera(10.0, 25.0), fov=70.0)
+    ctx = nes.Context(*_const_scene(sigma)) if sigma else gpu_ctx
+    try:
+        for windows in (0, 0, 7, 128):
+            ref, _ = ctx.render(views + [large], precision=prec, steps_per_pass=windows)
+            assert sum(int(r["n_samples"].sum()) for r in ref[:-1]) > 0
+            got, _ = ctx.render(views, precision=prec, steps_per_pass=windows)
+            alone = [ctx.render(v, precision=prec, steps_per_pass=windows)[0][0] for v in views]
+            for r, g, a in zip(ref, got, alone):
+                for k in r:
+                    assert np.array_equal(r[k], g[k]) and np.array_equal(r[k], a[k]), (windows, k)
+    finally:
+        if sigma:
+            ctx.close()

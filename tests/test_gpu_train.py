@@ -330,3 +330,15 @@ def test_checkpoint_round_trip(nes, oracle, scene1, tmp_path):
         assert e.value.code == -22
         tc, wc = b.get_params()
         assert np.array_equal(tc, tb4) and np.array_equal(wc, wb4)
+
+
+def test_small_and_large_ray_batches_agree(nes, oracle, scene1):
+    """Up to 2^15 rays march with four lanes per ray, more with one: the
+    colours of a large batch equal those of its parts, whose sizes leave the
+    last tile of 64 rays partly empty."""
+    ro, rd, _, _ = oracle.training_rays(0, 0, 40000)
+    with nes.Trainer(*scene1, rays_per_batch=40000) as tr:
+        whole = tr.forward(ro, rd)
+        assert np.abs(whole).max() > 0
+        for a, b in ((0, 1), (1, 64), (64, 129), (129, 7000), (7000, 39768)):
+            assert np.array_equal(tr.forward(ro[a:b], rd[a:b]), whole[a:b]), (a, b)
