@@ -123,6 +123,41 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
   return v;
 }
 
+// The layout of a tile's part of the sample list, for a workgroup of four
+// wavefronts that works on one tile: rank r's samples are those of the rays in
+// rank_rays[r], in ray order from rank_at[r] on.  c is the count of ray
+// lane_id(), mx the tile's largest.
+__device__ __forceinline__ void index_ranks(uint32_t c, uint32_t mx, uint64_t *rank_rays, uint32_t *rank_at) {
+  const int lane = lane_id();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (uint32_t i = wave; i < mx; i += 4) {
+    const uint64_t has = __ballot(c > i);
+    if (lane == 0) rank_rays[i] = has;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // exclusive prefix sums of the ranks' sizes, two ranks per lane
+    const uint32_t i0 = 2 * (uint32_t)lane;
+    const uint32_t n0 = i0 < mx ? (uint32_t)__popcll(rank_rays[i0]) : 0u;
+    const uint32_t n1 = i0 + 1 < mx ? (uint32_t)__popcll(rank_rays[i0 + 1]) : 0u;
+    uint32_t inc = n0 + n1;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t o = __shfl_up(inc, d);
+      if (lane >= d) inc += o;
+    }
+    rank_at[i0] = inc - n0 - n1;
+    rank_at[i0 + 1] = inc - n1;
+  }
+  __syncthreads();
+}
+
+// Value of lane q of each group of four lanes.
+template <int q>
+__device__ __forceinline__ float quad_value(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), q * 0x55, 0xf, 0xf, true));
+}
+
 
 // --------------------------------------------------------------- encoding
 __device__ __forceinline__ void sh4(const float d[3], float sh[16]) {

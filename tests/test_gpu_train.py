@@ -342,3 +342,36 @@ def test_small_and_large_ray_batches_agree(nes, oracle, scene1):
         assert np.abs(whole).max() > 0
         for a, b in ((0, 1), (1, 64), (64, 129), (129, 7000), (7000, 39768)):
             assert np.array_equal(tr.forward(ro[a:b], rd[a:b]), whole[a:b]), (a, b)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 200])
+def test_backward_of_rays_that_end(nes, oracle, n):
+    """Rays of 1 to 98 samples (the gradient walks them 32 at a time), most of
+    which end (T < 1e-4) before their last, in batches around a tile's 64 rays.
+    Table values are 30 times scene 1's, and the kink margin with them; the
+    forward's tolerance on this scene is five times scene 1's, and so is the
+    gradient's: 5e-4 of the largest."""
+    t, w, _ = oracle.scene(1)
+    t = (t * 30.0).astype(np.float32)
+    w = w.copy()
+    w[2048:2048 + 64] *= 4.0  # densities from ~1e-3 to ~1e3
+    occ = np.full(65536, 0xFFFFFFFF, np.uint32)
+    ro, rd, _, _ = oracle.training_rays(0, 0, 4000)
+    keep = []
+    for i in range(len(ro)):
+        if len(keep) < n and oracle.render_ray(t, w, occ, ro[i], rd[i])[3] > 0 and \
+                oracle.ray_relu_margin(t, w, occ, ro[i], rd[i]) > 30 * KINK_MARGIN:
+            keep.append(i)
+    assert len(keep) == n
+    ro, rd = ro[keep], rd[keep]
+    if n >= 63:
+        there = np.array([oracle.render_ray(t, 0 * w, occ, ro[i], rd[i])[3] for i in range(n)])
+        used = np.array([oracle.render_ray(t, w, occ, ro[i], rd[i])[3] for i in range(n)])
+        assert there.max() > 64 and (used < there).sum() > n // 4
+    target = np.random.default_rng(n).uniform(0, 1, (n, 3)).astype(np.float32)
+    _, gt_ref, gw_ref = oracle.loss_grad(t, w, occ, ro, rd, target)
+    with nes.Trainer(t, w, occ, rays_per_batch=256) as tr:
+        rgb = tr.forward(ro, rd)
+        gt, gw = tr.backward(ro, rd, 2.0 * (rgb - target) / (3 * n))
+    assert np.abs(gw - gw_ref).max() <= 5e-4 * np.abs(gw_ref).max()
+    assert np.abs(gt - gt_ref).max() <= 5e-4 * np.abs(gt_ref).max()
