@@ -219,17 +219,18 @@ int render_launch_bounded(const SceneDev &scene, RenderWork &w, int precision, h
 // (about one sample per thread) 2.20 ms.  An empty workgroup costs 0.2 ns of
 // dispatch (393216 of them 83 us, 32768 7 us), so the grid follows the
 // expected samples and not the capacity of the buffers.
+constexpr uint32_t kMaxPartBlocks = 49152;
 inline uint32_t part_blocks(size_t samples) {
   const size_t b = (samples + 255) / 256;
-  return (uint32_t)(b < 16 ? 16 : b > 49152 ? 49152 : b);
+  return (uint32_t)(b < 16 ? 16 : b > kMaxPartBlocks ? kMaxPartBlocks : b);
 }
 
 // Single-stage launchers (training step): march_emit over prepared rays,
 // FP32 encode_parts, composite (which stores the final state of rays that have
 // samples in work.acc for the backward; ray slot i is output i).
 int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStream_t stream);
-// (n: the host's sample count, for the launch size.)
-int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t stream);
+// (n: the host's sample count, for the launch size; scattered: rays in no order.)
+int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, bool scattered, hipStream_t stream);
 int launch_mlp_f32(const float *weights, RenderWork &w, const uint32_t *n_ptr, hipStream_t stream,
                    uint64_t *stamp = nullptr);
 int launch_composite(RenderWork &w, hipStream_t stream);

@@ -637,10 +637,12 @@ __device__ __forceinline__ void store_background(const BackgroundArgs &a, uint32
 // 65536) once its own part is done: in turn, so that its L2 holds two levels
 // at a time.  Stereo 1080p, times of the parts alone, us:
 //   996 951 844 775 779 714 700 659, together 1040; with shares 950
-// (1440x1600 at 75 degrees 1229 -> 1064, 2064x2208 2263 -> 1995).
+// (1440x1600 at 75 degrees 1229 -> 1064, 2064x2208 2263 -> 1995).  A batch of
+// random rays in FP32 is the other way round (see kScatteredShare).
 constexpr int kHelpedParts = 3;
 struct PartShares {
   uint32_t share[kHelpedParts];
+  uint32_t reverse;  // parts 7, 6, 5 are helped by XCDs 0, 1, 2 instead (FP32 only)
 };
 
 // Samples of part P beyond its own XCD's share start here (a multiple of the
@@ -693,25 +695,25 @@ __global__ __launch_bounds__(256) void encode_parts(const typename PosIn<Tab>::t
   uint32_t i = (blockIdx.x - bg.groups) / kParts * blockDim.x + threadIdx.x;
   const uint32_t step = blocks_per_part * blockDim.x;
 #define NES_PART(P, FROM, TO) i = encode_part_loop<Tab, P>(pos, FROM, TO, stride, table, feat, i, step, xch)
+  // part P and its helper's turn at part 7 - P, or the other way round
+  const bool rev = sizeof(Tab) == 4 && shares.reverse;
+#define NES_PART_PAIR(P)                                                \
+  case P:                                                               \
+    NES_PART(P, 0u, rev ? n : part_end(n, shares.share[P]));            \
+    if (rev) NES_PART(7 - P, part_end(n, shares.share[P]), n);          \
+    break;                                                              \
+  case 7 - P:                                                           \
+    NES_PART(7 - P, 0u, rev ? part_end(n, shares.share[P]) : n);        \
+    if (!rev) NES_PART(P, part_end(n, shares.share[P]), n);             \
+    break;
   switch (blockIdx.x % kParts) {
-    case 0: NES_PART(0, 0u, part_end(n, shares.share[0])); break;
-    case 1: NES_PART(1, 0u, part_end(n, shares.share[1])); break;
-    case 2: NES_PART(2, 0u, part_end(n, shares.share[2])); break;
+    NES_PART_PAIR(0)
+    NES_PART_PAIR(1)
+    NES_PART_PAIR(2)
     case 3: NES_PART(3, 0u, n); break;
-    case 4: NES_PART(4, 0u, n); break;
-    case 5:
-      NES_PART(5, 0u, n);
-      NES_PART(2, part_end(n, shares.share[2]), n);
-      break;
-    case 6:
-      NES_PART(6, 0u, n);
-      NES_PART(1, part_end(n, shares.share[1]), n);
-      break;
-    default:
-      NES_PART(7, 0u, n);
-      NES_PART(0, part_end(n, shares.share[0]), n);
-      break;
+    default: NES_PART(4, 0u, n); break;
   }
+#undef NES_PART_PAIR
 #undef NES_PART
 }
 
@@ -1562,13 +1564,32 @@ static size_t expected_samples(const RenderWork &w, int pass) {
 // and reach 12, 9 and 4 % at 935, 21, 15 and 6 % from 1250 on.  Below 500 they
 // gain nothing.  One of them a fifth smaller or larger moves the encode by 2 %
 // at most; all three a fifth larger cost 1 to 5 %.
-static PartShares part_shares(const RenderWork &w) {
+//
+// In FP32 a hashed level fills an XCD's L2 by itself, part 0 is ahead of part 7
+// already at 416 and the shares are constant from 480 on, us, tables not in the
+// Infinity Cache: 640x480 stereo 382 -> 365, 720p stereo 753 -> 681, 1080p
+// stereo 1480 -> 1312; none up to 280 (640x480 at 75 degrees 225 -> 230).
+// Between limits: of 1 M samples the helpers' extra 4 MB of table cost more
+// than they take off part 0 (640x480: 201 -> 204, the frame 535 -> 546); and
+// where the samples are more than twice the grid's threads its passes mix the
+// parts' turns and four such levels take turns in one L2 (26.7 M samples
+// 2690 -> 3100, 50.8 M 4280 -> 5460).
+constexpr size_t kF32ShareMin = 3u << 19, kF32ShareMax = 2 * 256 * (size_t)kMaxPartBlocks;
+
+static PartShares part_shares(const RenderWork &w, bool f32, size_t expect) {
   double focal = 0.0;
   for (uint32_t i = 0; i < w.n_views; ++i)
     focal += (double)w.host_views[i].focal * w.host_views[i].slot_count / w.n_slots;
+  const auto q = [](double v) { return (uint32_t)(std::max(v, 0.0) * 65536); };
+  if (f32) {
+    if (expect < kF32ShareMin || expect > kF32ShareMax) return PartShares{};
+    const double s = 0.15 * std::min((focal - 280.0) / 200.0, 1.0);
+    return PartShares{{q(s), q(s - 0.05), q(s - 0.10)}, 0u};
+  }
   const double f = std::min(std::max((focal - 500.0) / 600.0, 0.0), 1.25);
-  return PartShares{{(uint32_t)(0.17 * f * 65536), (uint32_t)(0.12 * f * 65536), (uint32_t)(0.05 * f * 65536)}};
+  return PartShares{{q(0.17 * f), q(0.12 * f), q(0.05 * f)}, 0u};
 }
+
 
 int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int k0, int k1,
                        bool first, bool last, hipStream_t stream, uint32_t ray_cap, bool resume) {
@@ -1592,7 +1613,7 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
   // grids for the expected samples, with grid-stride loops: the sample count
   // stays on the device
   const size_t expect = expected_samples(w, first ? 0 : 1);
-  const PartShares shares = f32 ? PartShares{} : part_shares(w);
+  const PartShares shares = part_shares(w, f32, expect);
   const uint32_t bpp = part_blocks(expect + (expect * shares.share[0] >> 16));
   BackgroundArgs bg = background_args(w);
   if (!first) bg.groups = 0;
@@ -1735,11 +1756,21 @@ int launch_march_emit(const uint32_t *occ, RenderWork &w, int k0, int k1, hipStr
   return launch_march(march_args(w, occ, k0, k1, kMarchPrepared, kMaxSteps), stream);
 }
 
-int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, hipStream_t stream) {
-  const uint32_t bpp = part_blocks(n);
+// Rays drawn at random share no cells, and an XCD's time goes with its hashed
+// levels' L2 lines (four to five per sample and level): parts 7, 6 and 5 have
+// two such levels, parts 0, 1 and 2 one.  Helping the former takes a 2^18-ray
+// batch's encode from 424 to 329 us (65536 rays 112 -> 88, 16384 33 -> 28); 20
+// or 30 % instead of 25 gained less.  A caller's own rays may be in any order
+// and are not shared.
+constexpr uint32_t kScatteredShare = 65536 / 4;
+
+int launch_encode_f32(const float *table, RenderWork &w, uint32_t n, bool scattered, hipStream_t stream) {
+  PartShares shares{};
+  if (scattered) shares = PartShares{{kScatteredShare, kScatteredShare, kScatteredShare}, 1u};
+  const uint32_t bpp = part_blocks(n + ((uint64_t)n * shares.share[0] >> 16));
   encode_parts<float><<<bpp * kParts, 256, 0, stream>>>(w.sample_pos.as<float4>(),
                                                          w.total.as<uint32_t>(), w.capacity,
-                                                         table, w.feat.as<float4>(), bpp, PartShares{}, BackgroundArgs{},
+                                                         table, w.feat.as<float4>(), bpp, shares, BackgroundArgs{},
                                                          nullptr);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;

@@ -1187,7 +1187,7 @@ static int trainer_forward(nes_trainer *t, uint32_t n_rays, TrainRayArgs ra) {
   train_rays<<<(n_rays + 255) / 256, 256, 0, s>>>(ra);
   NES_HIP_TRY(hipGetLastError());
   NES_TRY(launch_march_emit(t->occ, w, 0, kMaxSteps, s));
-  NES_TRY(launch_encode_f32(t->params, w, expected_samples(w, n_rays), s));
+  NES_TRY(launch_encode_f32(t->params, w, expected_samples(w, n_rays), !ra.ray_o, s));
   NES_TRY(launch_mlp_f32(t->params + t->n_table, w, w.total.as<uint32_t>(), s));
   return launch_composite(w, s);
 }

@@ -484,3 +484,21 @@ def test_small_and_large_batches_agree(nes, gpu_ctx, prec, sigma):
     finally:
         if sigma:
             ctx.close()
+
+
+@pytest.mark.parametrize("w,h", [(1100, 701), (1024, 1024)])
+def test_fp32_encode_shares_change_no_result(nes, gpu_ctx, w, h):
+    """As the mixed path's, on the FP32 path's own line: shares of 1.6 to 25
+    million samples, from a mean focal length of 280 pixels on.  The view alone
+    has them at their largest, beside wide ones smaller or none."""
+    v = nes.camera(w, h, nes.orbit_camera(25.0, 15.0), fov=35.0)
+    wide = nes.camera(w, h, nes.orbit_camera(10.0, 25.0), fov=140.0)
+    for _ in range(2):  # the first frame's launch size is a guess
+        (alone,), st = gpu_ctx.render(v, precision=FP32)
+    assert 1.6e6 < st.samples < 22e6
+    for batch in ([wide, v], [wide, wide, wide, v]):
+        for _ in range(2):
+            outs, st = gpu_ctx.render(batch, precision=FP32)
+        assert 1.6e6 < st.samples < 22e6
+        for k in alone:
+            assert np.array_equal(alone[k], outs[-1][k]), k
