@@ -90,6 +90,14 @@ static_assert(kW2 - kW1 == 64 * 32 && kW3 - kW2 == 16 * 64 && kW4 - kW3 == 64 * 
                   kW5 - kW4 == 64 * 64 && kWeights - kW5 == 3 * 64,
               "weight matrix shapes");
 
+// One wavefront per SIMD: the 40 weight-gradient blocks and the tile's
+// activations and deltas take 256 vector and 221 accumulation registers.  What
+// bounds it is that this wavefront's LDS reads, transposes and register moves
+// do not overlap with its products (448 of 32 cycles a tile, about half of the
+// time).  Every product therefore goes to another accumulator than the one
+// before, and a weight gradient reads each operand once: 2^18 rays 630 -> 593
+// us, 16384 73 -> 65.  (Loading the next tile's samples ahead spills and gains
+// nothing more.)
 __global__ __launch_bounds__(256) void mlp_train_bwd(TrainMlpArgs a) {
   constexpr int kS1 = WL::S1, kS2 = WL::S2, kS3 = WL::S3, kS4 = WL::S4, kS5 = WL::S5;
   constexpr int kP1 = WL::P1, kP2 = WL::P2, kP3 = WL::P3, kP4 = WL::P4, kP5 = WL::P5;
@@ -136,74 +144,66 @@ __global__ __launch_bounds__(256) void mlp_train_bwd(TrainMlpArgs a) {
         if (g == c) v = shv[4 * c + r];
       shq[r] = v;
     }
-    float4v d1[4], d3[4], d4[4], d2 = zero;
+    float4v d1[4] = {zero, zero, zero, zero}, d3[4] = {zero, zero, zero, zero}, d4[4] = {zero, zero, zero, zero},
+            d2 = zero;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      float4v acc = zero;
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc = mfma32(W[kP1 + (16 * m + j) * kS1 + w1_col(16 * b + 4 * g + r)], xf[b][r], acc);
-      d1[m] = acc;
-    }
+        for (int m = 0; m < 4; ++m)
+          d1[m] = mfma32(W[kP1 + (16 * m + j) * kS1 + w1_col(16 * b + 4 * g + r)], xf[b][r], d1[m]);
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         d2 = mfma32(W[kP2 + j * kS2 + 16 * m + 4 * g + r], fmaxf(d1[m][r], 0.0f), d2);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      float4v acc = zero;
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int r = 0; r < 4; ++r) {
+        const int col = w3_col(16 * b + 4 * g + r);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int col = w3_col(16 * b + 4 * g + r);
+        for (int m = 0; m < 4; ++m) {
           const float wv = col < 0 ? 0.0f : W[kP3 + (16 * m + j) * kS3 + col];
-          acc = mfma32(wv, b == 0 ? d2[r] : shq[r], acc);
+          d3[m] = mfma32(wv, b == 0 ? d2[r] : shq[r], d3[m]);
         }
-      d3[m] = acc;
-    }
+      }
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      float4v acc = zero;
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc = mfma32(W[kP4 + (16 * m + j) * kS4 + 16 * b + 4 * g + r], fmaxf(d3[b][r], 0.0f), acc);
-      d4[m] = acc;
-    }
+        for (int m = 0; m < 4; ++m)
+          d4[m] = mfma32(W[kP4 + (16 * m + j) * kS4 + 16 * b + 4 * g + r], fmaxf(d3[b][r], 0.0f), d4[m]);
     // ---------------- backward
     float4 go = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (g == 0 && valid) go = a.dout[s];
     const float4v e5 = {go.y, go.z, go.w, 0.0f};  // rows 0..2 of block 0 (g == 0)
-    float4v e4[4], e3[4], e1[4], e2 = zero;
+    float4v e4[4] = {zero, zero, zero, zero}, e3[4] = {zero, zero, zero, zero}, e1[4] = {zero, zero, zero, zero},
+            e2 = zero;
+    auto relu_back = [](float4v(&e)[4], const float4v(&d)[4]) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      float4v acc = zero;
+      for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < 4; ++r) e[m][r] = d[m][r] > 0.0f ? e[m][r] : 0.0f;
+    };
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
         const int o = 4 * g + r;
-        acc = mfma32(o < 3 ? W[kP5 + o * kS5 + 16 * m + j] : 0.0f, e5[r], acc);
+        e4[m] = mfma32(o < 3 ? W[kP5 + o * kS5 + 16 * m + j] : 0.0f, e5[r], e4[m]);
       }
+    relu_back(e4, d4);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = d4[m][r] > 0.0f ? acc[r] : 0.0f;
-      e4[m] = acc;
-    }
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      float4v acc = zero;
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc = mfma32(W[kP4 + (16 * b + 4 * g + r) * kS4 + 16 * m + j], e4[b][r], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = d3[m][r] > 0.0f ? acc[r] : 0.0f;
-      e3[m] = acc;
-    }
+        for (int m = 0; m < 4; ++m)
+          e3[m] = mfma32(W[kP4 + (16 * b + 4 * g + r) * kS4 + 16 * m + j], e4[b][r], e3[m]);
+    relu_back(e3, d3);
     {
       const int col = w3_col(j);  // row j of the out2 block
 #pragma unroll
@@ -214,14 +214,10 @@ __global__ __launch_bounds__(256) void mlp_train_bwd(TrainMlpArgs a) {
       if (g == 0) e2[0] = go.x;  // log-sigma row
     }
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      float4v acc = zero;
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc = mfma32(W[kP2 + (4 * g + r) * kS2 + 16 * m + j], e2[r], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = d1[m][r] > 0.0f ? acc[r] : 0.0f;
-      e1[m] = acc;
-    }
+      for (int m = 0; m < 4; ++m) e1[m] = mfma32(W[kP2 + (4 * g + r) * kS2 + 16 * m + j], e2[r], e1[m]);
+    relu_back(e1, d1);
 #pragma unroll
     for (int bq = 0; bq < 2; ++bq) {
       float4v acc = zero;
@@ -251,14 +247,18 @@ __global__ __launch_bounds__(256) void mlp_train_bwd(TrainMlpArgs a) {
       constexpr int OB = decltype(ob)::value, IB = decltype(ib)::value, BASE = decltype(base)::value;
       wave_lds_fence();
 #pragma unroll
-      for (int mo = 0; mo < OB; ++mo)
+      for (int t = 0; t < 4; ++t) {
+        float dv[OB], xv[IB];
 #pragma unroll
-        for (int mk = 0; mk < IB; ++mk) {
-          float4v acc = wacc[BASE + mo * IB + mk];
+        for (int mo = 0; mo < OB; ++mo) dv[mo] = td[16 * mo + j][4 * t + g];
 #pragma unroll
-          for (int t = 0; t < 4; ++t) acc = mfma32(td[16 * mo + j][4 * t + g], tx[16 * mk + j][4 * t + g], acc);
-          wacc[BASE + mo * IB + mk] = acc;
-        }
+        for (int mk = 0; mk < IB; ++mk) xv[mk] = tx[16 * mk + j][4 * t + g];
+#pragma unroll
+        for (int mo = 0; mo < OB; ++mo)
+#pragma unroll
+          for (int mk = 0; mk < IB; ++mk)
+            wacc[BASE + mo * IB + mk] = mfma32(dv[mo], xv[mk], wacc[BASE + mo * IB + mk]);
+      }
       wave_lds_fence();
     };
     // layer 5: delta rows 0..2, x = h4
