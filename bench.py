@@ -178,11 +178,12 @@ def ceilings_leg(N, samples, ms_encode, l2_req_per_launch, l1_acc_per_launch=Non
         out["encode_l1_accesses_frac"] = round(l1_acc_per_launch / (ms_encode * 1e-3) / l1, 4)
     if l2_req_per_launch:
         rate = l2_req_per_launch / (ms_encode * 1e-3)
+        # level 15 on XCD 0: no reuse between samples, so 4 L2 requests (one
+        # per y/z corner pair) per sample, of the 87.7 % that it encodes itself
+        # at this focal length (935 pixels)
+        xcd0 = 4 * 0.877 * samples / (ms_encode * 1e-3)
         out.update({"encode_l2_requests_per_s": rate, "encode_l2_frac": round(rate / l2, 4),
-                    # level 15 on XCD 0: no reuse between samples, so 4 L2
-                    # requests (one per y/z corner pair) per sample
-                    "xcd0_l2_requests_per_s": 4 * samples / (ms_encode * 1e-3),
-                    "xcd0_l2_frac": round(4 * samples / (ms_encode * 1e-3) / (l2 / 8), 4)})
+                    "xcd0_l2_requests_per_s": xcd0, "xcd0_l2_frac": round(xcd0 / (l2 / 8), 4)})
     return out
 
 
