@@ -71,8 +71,9 @@ constexpr int kTotWords = kTotTermBase + kTotTermSlots * kTotTermStride;
 constexpr size_t kTotBytes = sizeof(uint32_t) * kTotWords;
 
 // One output array on its way to pinned host memory: src (device, 16-byte
-// aligned) to dst, `bytes` long, bpp bytes per pixel of view `view`.  With a
-// gray_scale the source is FP32 depth, stored as the GRAY8 plane.
+// aligned) to dst, `bytes` long, bpp bytes per pixel of view `view`.  The array
+// of one byte per pixel is the GRAY8 plane, whose source is FP32 depth times
+// gray_scale.
 struct HostArray {
   const uint8_t *src;
   uint8_t *dst;

@@ -1150,7 +1150,7 @@ __global__ __launch_bounds__(kFrameThreads) void frame_begin(uint32_t *total, Ar
 template <class T>
 __device__ __forceinline__ void store_unit(const HostArray &h, uint32_t at) {
   T v;
-  if (h.gray_scale != 0.0f) {
+  if (h.bpp == 1) {  // (the scale may have any value: 0 for an infinite far distance)
     uint8_t g[sizeof(T)];
 #pragma unroll
     for (int i = 0; i < (int)sizeof(T); ++i)

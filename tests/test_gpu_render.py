@@ -430,6 +430,20 @@ def test_pinned_outputs_of_multi_pass_frames(nes, oracle, prec):
             assert np.array_equal(want[0][k], got[0][k]), k
 
 
+@pytest.mark.parametrize("far", [float("inf"), 3e38, 1e-42, float("nan"), -1.0])
+@pytest.mark.parametrize("w,h,offset", [(640, 480, 0), (31, 17, 0), (31, 17, 1)])
+def test_gray8_of_any_far_distance(nes, oracle, gpu_ctx, w, h, offset, far):
+    """The GRAY8 plane stored into pinned memory is the quantised depth for far
+    distances whose scale 255 / far is 0, infinite or the default's as well."""
+    v = nes.camera(w, h, nes.orbit_camera(30.0, 20.0), fov=40.0)
+    (got,), _ = _pinned_render(nes, gpu_ctx, [v], MIXED, ("depth", "depth_gray8"), offset, far)
+    assert got["depth"].max() > 0
+    want = oracle.depth_gray8(got["depth"], far if far > 0 else nes.DEPTH_FAR_DEFAULT)
+    assert np.array_equal(got["depth_gray8"], want)
+    (o,), _ = gpu_ctx.render(v, precision=MIXED, depth_far=far)  # the binding's own arrays
+    assert np.array_equal(o["depth_gray8"], want)
+
+
 def test_returned_arrays_are_the_callers(nes, gpu_ctx):
     """Arrays of earlier renders keep their values through later ones (their
     memory is reused only once they are gone)."""
