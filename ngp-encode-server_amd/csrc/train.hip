@@ -1135,6 +1135,12 @@ struct nes_trainer {
 
 namespace nes {
 
+// Samples the buffers are sized for when `samples` are wanted.  Never as many
+// as a call is refused for: the count of a refused call then exceeds the
+// capacity as well, and what lasts (the update above all) is left out on the
+// device before the host has seen the count.
+static size_t sample_room(size_t samples) { return std::min<size_t>(samples, kMaxBucketSamples - 1); }
+
 static int trainer_prepare(nes_trainer *t, uint32_t n_rays) {
   RenderWork &w = t->work;
   w.n_slots = n_rays;
@@ -1149,25 +1155,26 @@ static int trainer_prepare(nes_trainer *t, uint32_t n_rays) {
   NES_TRY(w.total.reserve(kTotBytes));
   NES_TRY(w.views.reserve(sizeof(ViewDesc)));
   if (!w.total_host) NES_HIP_TRY(hipHostMalloc((void **)&w.total_host, kTotBytes));
-  if (w.capacity < (size_t)n_rays * 4 || w.capacity_precision != NES_PRECISION_FP32)
-    NES_TRY(render_reserve_samples(w, NES_PRECISION_FP32, std::max<size_t>(w.capacity, (size_t)n_rays * 4)));
+  const size_t room = sample_room(std::max<size_t>(w.capacity, (size_t)n_rays * 4));
+  if (w.capacity < room || w.capacity_precision != NES_PRECISION_FP32)
+    NES_TRY(render_reserve_samples(w, NES_PRECISION_FP32, room));
   return NES_OK;
 }
 
-static int trainer_grow(nes_trainer *t, size_t cap) {
+static int trainer_grow(nes_trainer *t, size_t samples) {
+  const size_t cap = sample_room(samples);
   NES_TRY(render_reserve_samples(t->work, NES_PRECISION_FP32, cap));
   NES_TRY(t->dout.reserve(sizeof(float4) * (cap + 1)));
   NES_TRY(t->dfeat.reserve(2 * sizeof(float4) * kParts * (cap + 1)));
-  // a call's samples stay below kMaxBucketSamples (checked in trainer_finish)
-  NES_TRY(t->items.reserve(sizeof(uint32_t) * kEntriesPerSample *
-                           std::min<size_t>(cap + 1, kMaxBucketSamples)));
+  NES_TRY(t->items.reserve(sizeof(uint32_t) * kEntriesPerSample * (cap + 1)));
   return NES_OK;
 }
 
 // Every call queues its whole device work for the sample buffers as they are,
 // without a host round trip in between, and reads the sample count at its end.
 // Kernels write nothing beyond the capacity, and nothing that lasts when the
-// count exceeds it: such a call grows the buffers and runs once more.
+// count exceeds it: such a call grows the buffers and runs once more, or is
+// refused (kMaxBucketSamples, sample_room).
 
 // Samples a call is expected to have (for launch sizes only).
 static uint32_t expected_samples(const RenderWork &w, uint32_t n_rays) {
@@ -1288,15 +1295,12 @@ static int trainer_backward(nes_trainer *t, uint32_t n_rays, const float *dC) {
   ma.grad_w = t->grads + t->n_table;
   mlp_train_bwd<<<256, 256, 0, s>>>(ma);
   NES_HIP_TRY(hipGetLastError());
-  // (the bucket counters were cleared by train_rays; items holds the entries
-  // of fewer than kMaxBucketSamples samples, more than that are refused at the
-  // end of the call)
-  const uint32_t most = std::min(w.capacity, kMaxBucketSamples - 1);
+  // (the bucket counters were cleared by train_rays)
   bucket_count<<<kBucketBlocks, kBucketThreads, 0, s>>>(w.sample_pos.as<float4>(), w.total.as<uint32_t>(),
-                                                        most, t->bucket_count);
+                                                        w.capacity, t->bucket_count);
   bucket_scan<<<1, kBucketScanThreads, 0, s>>>(t->bucket_count, t->bucket_off, t->bucket_cursor);
   bucket_place<<<kBucketBlocks, kBucketThreads, 0, s>>>(w.sample_pos.as<float4>(), w.total.as<uint32_t>(),
-                                                        most, t->bucket_cursor, t->items.as<uint32_t>());
+                                                        w.capacity, t->bucket_cursor, t->items.as<uint32_t>());
   scatter_slices<<<kParts * kSliceTasksPerXcd, kSliceThreads, 0, s>>>(
       t->dfeat.as<float4>(), t->items.as<uint32_t>(), t->bucket_off,
       w.capacity, t->tasks, t->grads);

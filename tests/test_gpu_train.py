@@ -332,6 +332,28 @@ def test_checkpoint_round_trip(nes, oracle, scene1, tmp_path):
         assert np.array_equal(tc, tb4) and np.array_equal(wc, wb4)
 
 
+def test_refused_step_changes_nothing(nes, oracle, scene1, tmp_path):
+    """A step of 2^25 rays has more samples (about 110 million) than the
+    gradient buckets index (79.5 million): it is refused, twice alike, and
+    parameters, moments and step count stay as they were, bit for bit."""
+    poses = np.stack([oracle.training_pose(0, i) for i in range(16)])
+    targets = np.zeros((16, 48, 64, 3), np.float32)
+    files = [str(tmp_path / f"{i}.bin") for i in range(3)]
+    ro, rd, _, _ = oracle.training_rays(0, 0, 500)
+    with nes.Trainer(*scene1, poses=poses, targets=targets, width=64, height=48,
+                     rays_per_batch=1 << 25, seed=0) as tr:
+        rgb = tr.forward(ro, rd)
+        tr.save(files[0])
+        for f in files[1:]:
+            with pytest.raises(nes.NesError) as e:
+                tr.step()
+            assert e.value.code == -34 and "samples" in str(e.value)
+            tr.save(f)
+        assert np.array_equal(tr.forward(ro, rd), rgb)
+    saved = [np.fromfile(f, np.uint8) for f in files]
+    assert np.array_equal(saved[0], saved[1]) and np.array_equal(saved[0], saved[2])
+
+
 def test_small_and_large_ray_batches_agree(nes, oracle, scene1):
     """Up to 2^15 rays march with four lanes per ray, more with one: the
     colours of a large batch equal those of its parts, whose sizes leave the
