@@ -354,8 +354,8 @@ __global__ __launch_bounds__(64 * kFpWaves) void frameprep_kernel(FrameprepArgs 
   __shared__ int16_t edge_coef[kVClasses * kVTaps];
   const uint32_t total = a.strips * a.tiles * a.frames;
   // runs of a.run tiles, dealt to the XCDs in turn
-  const uint32_t turn = blockIdx.x / kFpXcds;
-  const uint32_t id = (turn / a.run * kFpXcds + blockIdx.x % kFpXcds) * a.run + turn % a.run;
+  const uint32_t block = blockIdx.y * gridDim.x + blockIdx.x, turn = block / kFpXcds;
+  const uint32_t id = (turn / a.run * kFpXcds + block % kFpXcds) * a.run + turn % a.run;
   if (id >= total) return;
   const uint32_t strip = id % a.strips, tile = id / a.strips % a.tiles, f = id / a.strips / a.tiles;
   const uint8_t *rgb_a = a.rgb_a + f * a.rgb_fb;
@@ -511,17 +511,23 @@ constexpr size_t kBulkBytes = (size_t)256 << 20;
 
 constexpr uint32_t kFpRunRows = 6;  // tile rows per run
 
+// Workgroups in a row of the grid.  One dimension of a launch holds fewer than
+// 2^32 threads; tens of thousands of narrow frames have more tiles than that.
+constexpr uint32_t kFpGridRow = 1u << 23;
+static_assert(kFpGridRow % kFpXcds == 0, "a row starts on XCD 0");
+
 template <int kCRows, FrameClass kClass>
 static void frameprep_launch(FrameprepArgs &a, bool two, hipStream_t stream) {
   a.tiles = (uint32_t)((a.h / 2 + kCRows - 1) / kCRows);
   const uint32_t total = a.strips * a.tiles * a.frames;
   a.run = std::max(1u, std::min(a.strips * kFpRunRows, (total + kFpXcds - 1) / kFpXcds));
   const uint32_t turns = (total + a.run * kFpXcds - 1) / (a.run * kFpXcds);
-  const unsigned blocks = turns * a.run * kFpXcds;
+  const uint32_t blocks = turns * a.run * kFpXcds;
+  const dim3 grid(std::min(blocks, kFpGridRow), (blocks + kFpGridRow - 1) / kFpGridRow);
   if (two)
-    frameprep_kernel<true, kCRows, kClass><<<blocks, 64 * kFpWaves, 0, stream>>>(a);
+    frameprep_kernel<true, kCRows, kClass><<<grid, 64 * kFpWaves, 0, stream>>>(a);
   else
-    frameprep_kernel<false, kCRows, kClass><<<blocks, 64 * kFpWaves, 0, stream>>>(a);
+    frameprep_kernel<false, kCRows, kClass><<<grid, 64 * kFpWaves, 0, stream>>>(a);
 }
 
 int launch_frameprep(const uint8_t *rgb_a, const float *depth_a,

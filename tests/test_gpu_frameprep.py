@@ -150,3 +150,25 @@ def test_gray_stream_shapes_bit_exact(nes, oracle, w, h, mode):
     g = np.random.default_rng(w + h).integers(0, 256, (h, w), dtype=np.uint8)
     for a, b in zip(nes.gray8_to_yuv420p(g, mode), oracle.gray8_to_yuv420p(g, mode)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("static", [False, True])
+def test_more_tiles_than_one_grid_dimension(nes, oracle, static):
+    """16400 frames of 2 x 8192 pixels, 4 chroma rows to a tile: 2^24 + 16384
+    workgroups of 256 threads, more than one dimension of a launch takes.
+    Every frame equals the oracle's."""
+    w, h, n = 2, 8192, 16400
+    src = np.random.default_rng(9).integers(0, 256, (3, h, w, 3), dtype=np.uint8)
+    ref = [oracle.rgb24_to_yuv420p(x, 0) for x in src]
+    which = np.arange(n) % 3
+    rgb, sizes = nes.DeviceBuffer(n * h * w * 3), (h * w, h // 2, h // 2)
+    out = [nes.DeviceBuffer(n * s) for s in sizes]
+    rgb.upload(src[which])
+    call = nes.frameprep_device_static if static else nes.frameprep_device
+    call(rgb, None, None, None, w, h, n, *out)
+    for k, (buf, s) in enumerate(zip(out, sizes)):
+        got = buf.download(np.empty((n, s), np.uint8))
+        for i in range(3):
+            assert (got[which == i] == ref[i][k].reshape(-1)).all(), (k, i)
+    for buf in [rgb] + out:
+        buf.free()
