@@ -14,6 +14,7 @@ Errors surface as :class:`NesError` carrying the library's negative errno code;
 there is no fallback path -- a missing or broken library raises.
 """
 import ctypes as C
+import mmap
 import os
 import threading
 
@@ -269,15 +270,20 @@ class _PinnedPool:
     store results straight into it, where an ordinary array costs a staged
     copy and the page faults of fresh memory.  At most LIMIT bytes are
     allocated (further arrays are ordinary ones) and at most KEEP of them stay
-    unused.  Any thread may take and drop arrays."""
+    unused.  Any thread may take and drop arrays.
+
+    A forked child does not inherit pinned memory, so os.fork (multiprocessing,
+    a data loader's workers) gives it private copies at the same addresses: the
+    arrays stay what ordinary ones would be.  The child takes no pinned memory."""
 
     LIMIT = 1 << 30
     KEEP = 256 << 20
 
     def __init__(self):
         self.lock = threading.RLock()  # re-entered when a collection drops a block inside it
-        self.free = {}
+        self.free, self.live = {}, {}  # unused blocks by size; size of each used one
         self.allocated = self.unused = 0
+        self.pid, self.copies = os.getpid(), []
 
     @staticmethod
     def size_class(nbytes):
@@ -291,7 +297,7 @@ class _PinnedPool:
             blocks = self.free.get(size)
             if blocks:
                 self.unused -= size
-                return _PinnedBlock(self, blocks.pop(), size)
+                return self.use(blocks.pop(), size)
             if self.allocated + size > self.LIMIT:
                 return None
             self.allocated += size
@@ -300,10 +306,20 @@ class _PinnedPool:
             with self.lock:
                 self.allocated -= size
             return None
-        return _PinnedBlock(self, p.value, size)
+        with self.lock:
+            return self.use(p.value, size)
+
+    def use(self, ptr, size):
+        self.live[ptr] = size
+        return _PinnedBlock(self, ptr, size)
 
     def give_back(self, ptr, size):
+        if os.getpid() != self.pid:  # a forked child's copy
+            if self.copies is None:
+                _libc().munmap(ptr, size)
+            return
         with self.lock:
+            del self.live[ptr]
             if self.unused + size <= self.KEEP:
                 self.unused += size
                 self.free.setdefault(size, []).append(ptr)
@@ -312,8 +328,46 @@ class _PinnedPool:
         if _lib is not None:
             _lib.nes_host_free(ptr)
 
+    def before_fork(self):
+        self.lock.acquire()  # the state below is whole in the child
+        if os.getpid() == self.pid:
+            self.copies = [(ptr, C.string_at(ptr, size)) for ptr, size in self.live.items()]
+
+    def after_fork_parent(self):
+        if os.getpid() == self.pid:
+            self.copies = []
+        self.lock.release()
+
+    def after_fork_child(self):
+        for ptr, data in self.copies or ():
+            _map_private(ptr, data)
+        self.lock, self.free, self.live, self.copies = threading.RLock(), {}, {}, None
+        self.allocated = self.unused = self.LIMIT = 0
+
+
+def _libc():
+    c = C.CDLL(None, use_errno=True)
+    c.mmap.restype = C.c_void_p
+    c.mmap.argtypes = [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_long]
+    c.munmap.argtypes = [C.c_void_p, C.c_size_t]
+    return c
+
+
+def _map_private(ptr, data):
+    """Ordinary memory holding `data` at address ptr, in place of what was
+    mapped there."""
+    map_fixed = 0x10
+    at = _libc().mmap(ptr, len(data), mmap.PROT_READ | mmap.PROT_WRITE,
+                      mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS | map_fixed, -1, 0)
+    if at != ptr:
+        raise OSError(C.get_errno(), "mmap of a forked child's array")
+    C.memmove(ptr, data, len(data))
+
 
 _pinned = _PinnedPool()
+os.register_at_fork(before=lambda: _pinned.before_fork(),
+                    after_in_parent=lambda: _pinned.after_fork_parent(),
+                    after_in_child=lambda: _pinned.after_fork_child())
 
 
 def _out_array(shape, dtype):

@@ -458,6 +458,28 @@ def test_returned_arrays_are_the_callers(nes, gpu_ctx):
             assert np.array_equal(r[name], k[name]), name
 
 
+def test_returned_arrays_in_a_forked_child(nes, gpu_ctx):
+    """A child forked after a render (which uses no GPU) reads the returned
+    arrays; the parent's stay as they are and it renders on."""
+    import os
+    cam = nes.camera(320, 200, nes.orbit_camera(30.0, 20.0))
+    got = gpu_ctx.render(cam)[0][0]
+    want = {k: np.array(v) for k, v in got.items()}
+    pid = os.fork()
+    if pid == 0:
+        code = 1
+        try:
+            code = 0 if all(np.array_equal(got[k], want[k]) for k in want) else 2
+            for v in got.values():
+                v[...] = 0
+        finally:
+            os._exit(code)
+    assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
+    again = gpu_ctx.render(cam)[0][0]
+    for k in want:
+        assert np.array_equal(got[k], want[k]) and np.array_equal(again[k], want[k]), k
+
+
 @pytest.mark.parametrize("w,h", [(17, 9), (64, 48), (257, 131)])
 def test_encode_shares_change_no_result(nes, gpu_ctx, w, h):
     """The XCDs share the encode's parts by the views' mean focal length: a

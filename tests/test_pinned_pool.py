@@ -97,3 +97,62 @@ def test_threads(pool):
     [t.join() for t in ts]
     gc.collect()
     assert not bad and p.unused == p.allocated <= p.KEEP
+
+
+class DontForkLib(FakeLib):
+    """Memory that a forked child does not inherit, as pinned memory is."""
+
+    def nes_host_alloc(self, n, out):
+        import mmap
+        m = mmap.mmap(-1, n)
+        m.madvise(mmap.MADV_DONTFORK)
+        out._obj.value = C.addressof(C.c_char.from_buffer(m))
+        self.live[out._obj.value] = m
+        return 0
+
+
+def in_child(f):
+    """Exit code (or minus the signal) of a forked child that runs f."""
+    import os
+    pid = os.fork()
+    if pid == 0:
+        code = 1
+        try:
+            code = 0 if f() else 2
+        finally:
+            os._exit(code)
+    return os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1])
+
+
+def test_forked_children_keep_their_arrays(pool, monkeypatch):
+    """A child forked between calls reads the values that arrays had at the
+    fork, may write and drop them and take more, and forks in turn; nothing of
+    it reaches the parent's arrays or its pool."""
+    N, p, _ = pool
+    monkeypatch.setattr(N, "_lib", DontForkLib())
+    arrays = [N._out_array((n, 3), np.float32) for n in (1, 1000, 70000)]
+    for i, a in enumerate(arrays):
+        a[:] = i + 1.5
+    part = arrays[1][5:9]
+    dropped = N._out_array((50,), np.int32)
+    del dropped                       # a free block stays the parent's
+    gc.collect()
+
+    def child():
+        ok = all((a == i + 1.5).all() for i, a in enumerate(arrays))
+        arrays[0][:] = 9.0
+        more = N._out_array((50,), np.int32)
+        more[:] = 7
+        ok = ok and in_child(lambda: (arrays[0] == 9.0).all() and (arrays[2] == 3.5).all()) == 0
+        arrays.clear()
+        gc.collect()
+        return ok and (part == 2.5).all() and (more == 7).all()
+
+    allocated = p.allocated
+    for _ in range(2):
+        assert in_child(child) == 0
+    assert all((a == i + 1.5).all() for i, a in enumerate(arrays)) and (part == 2.5).all()
+    assert p.allocated == allocated and p.unused == 4096 and len(p.live) == 3
+    again = N._out_array((50,), np.int32)
+    assert p.unused == 0 and len(p.live) == 4
+    del again
