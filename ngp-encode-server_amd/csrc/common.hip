@@ -74,6 +74,7 @@ int DevBuf::reserve(size_t need) {
   size_t cap = need + need / 8 + 256;
   hipError_t e = hipMalloc(&ptr, cap);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here, not by the next launch
     ptr = nullptr;
     bytes = 0;
     set_last_error(std::string("hipMalloc: ") + hipGetErrorString(e));

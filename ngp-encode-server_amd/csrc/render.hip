@@ -686,8 +686,9 @@ __global__ __launch_bounds__(256) void encode_parts(const typename PosIn<Tab>::t
   stamp_start(stamp);
   __shared__ uint32_t xch_all[4][256];  // per-wavefront gather exchange (FP16 hashed levels)
   // the first workgroups (a multiple of kParts of them) store background pixels
+  // (nothing of a pass that overflowed: the host may not be able to run it again)
   if (blockIdx.x < bg.groups) {
-    store_background(bg, blockIdx.x);
+    if (*n_ptr <= stride) store_background(bg, blockIdx.x);
     return;
   }
   uint32_t *xch = xch_all[threadIdx.x >> 6];
@@ -1190,15 +1191,17 @@ __device__ __forceinline__ void store_outputs(const HostArray &h, const Backgrou
   }
 }
 
-// The end of a frame: the counters and stamps and the output arrays into
-// pinned host memory.
-__global__ __launch_bounds__(256) void frame_end(const uint32_t *total, uint32_t *host, BackgroundArgs a) {
+// The end of a frame: the counters and stamps and, if its samples fitted, the
+// output arrays into pinned host memory.
+__global__ __launch_bounds__(256) void frame_end(const uint32_t *total, uint32_t *host, BackgroundArgs a,
+                                                 uint32_t capacity) {
   constexpr int kEnd = kTotStamps + 2 * kStampEnd;
   if (blockIdx.x == 0 && blockIdx.y == 0) {
     for (int i = (int)threadIdx.x; i < kTotWords; i += (int)blockDim.x)
       if (i != kEnd && i != kEnd + 1) host[i] = total[i];
     if (threadIdx.x == 0) reinterpret_cast<uint64_t *>(host + kTotStamps)[kStampEnd] = wall_clock64();
   }
+  if (max(total[kTotCursor], total[kTotCursorLater]) > capacity) return;  // the host re-renders
   if (blockIdx.y < a.n_arrays) store_outputs(a.arrays[blockIdx.y], a.groups ? &a : nullptr);
 }
 
@@ -1417,6 +1420,7 @@ int render_work_reserve(RenderWork &w, uint64_t max_slots, uint64_t max_px, uint
 int render_reserve_samples(RenderWork &w, int precision, size_t capacity) {
   if (capacity > 0xffffffffull) capacity = 0xffffffffull;
   const size_t fbytes = precision != NES_PRECISION_MIXED ? sizeof(float4) : sizeof(uint2);
+  w.capacity = 0;  // a buffer that cannot be had leaves the work area without any
   NES_TRY(w.samples.reserve(sizeof(uint32_t) * (capacity + 1)));
   NES_TRY(w.sample_out.reserve(sizeof(float4) * (capacity + 1)));
   NES_TRY(w.sample_pos.reserve(sizeof(float4) * (capacity + 1)));
@@ -1497,7 +1501,7 @@ int render_end(RenderWork &w, hipStream_t stream) {
   uint64_t most = 0;
   for (uint32_t i = 0; i < w.n_host_out; ++i) most = std::max(most, w.host_out[i].bytes);
   frame_end<<<dim3(store_blocks(most), std::max(w.n_host_out, 1u)), 256, 0, stream>>>(
-      w.total.as<uint32_t>(), w.total_host, background_args(w));
+      w.total.as<uint32_t>(), w.total_host, background_args(w), w.capacity);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }
@@ -1901,12 +1905,15 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
         set_last_error("sample capacity still exceeded after regrowth");
         return NES_ENOMEM;
       }
-      // grow when the budget allows it, else render within the buffers
-      const size_t want = (size_t)n + n / 8 + 1024;
-      if (render_growth_fits(w, precision, want))
-        NES_TRY(render_reserve_samples(w, precision, want));
-      else
+      // grow when the budget and the device allow it, else render within the
+      // buffers (the first of two passes has stored background already: the
+      // frame is not given up here)
+      const size_t want = (size_t)n + n / 8 + 1024, had = w.capacity;
+      bounded = !render_growth_fits(w, precision, want);
+      if (!bounded && render_reserve_samples(w, precision, want) != NES_OK) {
+        NES_TRY(render_reserve_samples(w, precision, had));
         bounded = true;
+      }
     }
     if (bounded) {
       double unused[4] = {0, 0, 0, 0};

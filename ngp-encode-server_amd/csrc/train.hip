@@ -1089,10 +1089,11 @@ __global__ __launch_bounds__(256) void store_params(float *__restrict__ src, flo
   }
 }
 
-// The end of a call's device work: sample count, loss, stamps and (optional)
-// ray colours into pinned host memory.
+// The end of a call's device work: sample count, loss, stamps and (optional,
+// if the samples fitted) ray colours into pinned host memory.
 __global__ __launch_bounds__(256) void train_end(const uint32_t *total, const float *loss, uint32_t *host,
-                                                 const float *rgb, float *rgb_host, uint32_t n_rgb) {
+                                                 const float *rgb, float *rgb_host, uint32_t n_rgb,
+                                                 uint32_t capacity) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     host[kTotCursor] = total[kTotCursor];
     host[kTotEvaluated] = __float_as_uint(loss ? *loss : 0.0f);
@@ -1100,6 +1101,7 @@ __global__ __launch_bounds__(256) void train_end(const uint32_t *total, const fl
     st[kStampBegin] = reinterpret_cast<const uint64_t *>(total + kTotStamps)[kStampBegin];
     st[kStampEnd] = wall_clock64();
   }
+  if (total[kTotCursor] > capacity) return;  // overflowed: the host runs the call again or refuses it
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_rgb; i += gridDim.x * blockDim.x)
     rgb_host[i] = rgb[i];
 }
@@ -1237,7 +1239,7 @@ static int launch_train_end(nes_trainer *t, const float *loss, float *rgb_host, 
   const float *rgb = reinterpret_cast<const float *>(w.out.as<uint8_t>() + out_layout(w.out_px).rgbf);
   const uint32_t n = rgb_host ? 3 * n_rays : 0u;
   train_end<<<std::max(1u, std::min(64u, n / 1024)), 256, 0, t->stream>>>(w.total.as<uint32_t>(), loss, w.total_host, rgb,
-                                                                          rgb_host, n);
+                                                                          rgb_host, n, w.capacity);
   NES_HIP_TRY(hipGetLastError());
   return NES_OK;
 }

@@ -354,6 +354,36 @@ def test_refused_step_changes_nothing(nes, oracle, scene1, tmp_path):
     assert np.array_equal(saved[0], saved[1]) and np.array_equal(saved[0], saved[2])
 
 
+def test_refused_forward_writes_nothing(nes, oracle, scene1):
+    """A forward with more samples than a call may have is refused and leaves
+    the caller's (pinned) colour array alone; so does the call's first run
+    where the samples outgrow the buffers, which ends with the right colours."""
+    import ctypes as C
+    t, w, _ = scene1
+    occ = np.full(nes.OCC_WORDS, 0xffffffff, np.uint32)
+    ro, rd, _, _ = oracle.training_rays(0, 0, 4096)
+    mid = 0.5 - ro                     # through the cube's centre: about 100 samples
+    rd = (mid / np.linalg.norm(mid, axis=1, keepdims=True)).astype(np.float32)
+    n = 1 << 20
+    p = C.c_void_p()
+    nes.check(nes.lib().nes_host_alloc(12 * n, C.byref(p)), "nes_host_alloc")
+    f32p = C.POINTER(C.c_float)
+    rgb = np.ctypeslib.as_array(C.cast(p, f32p), (n, 3))
+    with nes.Trainer(t, w, occ, rays_per_batch=4096) as tr:
+        def forward(o, d):
+            o, d = np.ascontiguousarray(o), np.ascontiguousarray(d)
+            return nes.lib().nes_trainer_forward(tr.handle, o.ctypes.data_as(f32p), d.ctypes.data_as(f32p),
+                                                 len(o), C.cast(p, f32p))
+        rgb[:] = 0.25
+        assert forward(ro, rd) == 0
+        assert np.array_equal(rgb[:4096], tr.forward(ro, rd)) and (rgb[4096:] == 0.25).all()
+        rgb[:] = 0.25
+        k = n // 4096
+        assert forward(np.tile(ro, (k, 1)), np.tile(rd, (k, 1))) == -34
+        assert (rgb == 0.25).all()
+    nes.check(nes.lib().nes_host_free(p), "nes_host_free")
+
+
 def test_small_and_large_ray_batches_agree(nes, oracle, scene1):
     """Up to 2^15 rays march with four lanes per ray, more with one: the
     colours of a large batch equal those of its parts, whose sizes leave the
