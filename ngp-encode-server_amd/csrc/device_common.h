@@ -160,7 +160,11 @@ __device__ __forceinline__ float quad_value(float v) {
 
 
 // --------------------------------------------------------------- encoding
+// The fused multiply-adds are written out: left to the compiler, which ones
+// are fused depends on the code around them, and a ray's values with it (a
+// batch's size decides which march kernel computes them).
 __device__ __forceinline__ void sh4(const float d[3], float sh[16]) {
+#pragma clang fp contract(off)
   const float x = d[0], y = d[1], z = d[2];
   const float xx = x * x, yy = y * y, zz = z * z;
   sh[0] = 0.28209479177387814f;
@@ -169,16 +173,16 @@ __device__ __forceinline__ void sh4(const float d[3], float sh[16]) {
   sh[3] = -0.48860251190291987f * x;
   sh[4] = 1.0925484305920792f * x * y;
   sh[5] = -1.0925484305920792f * y * z;
-  sh[6] = 0.94617469575755997f * zz - 0.31539156525251999f;
+  sh[6] = fmaf(0.94617469575755997f, zz, -0.31539156525251999f);
   sh[7] = -1.0925484305920792f * x * z;
-  sh[8] = 0.54627421529603959f * xx - 0.54627421529603959f * yy;
-  sh[9] = 0.59004358992664352f * y * (-3.0f * xx + yy);
+  sh[8] = fmaf(0.54627421529603959f, xx, -(0.54627421529603959f * yy));
+  sh[9] = 0.59004358992664352f * y * fmaf(-3.0f, xx, yy);
   sh[10] = 2.8906114426405538f * x * y * z;
-  sh[11] = 0.45704579946446572f * y * (1.0f - 5.0f * zz);
-  sh[12] = 0.3731763325901154f * z * (5.0f * zz - 3.0f);
-  sh[13] = 0.45704579946446572f * x * (1.0f - 5.0f * zz);
-  sh[14] = 1.4453057213202769f * z * (xx - yy);
-  sh[15] = 0.59004358992664352f * x * (-xx + 3.0f * yy);
+  sh[11] = 0.45704579946446572f * y * fmaf(-5.0f, zz, 1.0f);
+  sh[12] = 0.3731763325901154f * z * fmaf(5.0f, zz, -3.0f);
+  sh[13] = 0.45704579946446572f * x * fmaf(-5.0f, zz, 1.0f);
+  sh[14] = 1.4453057213202769f * z * fmaf(x, x, -yy);
+  sh[15] = 0.59004358992664352f * x * fmaf(3.0f, yy, -xx);
 }
 
 // One table entry (2 features) as stored: a float2, or two FP16 in a word.

@@ -522,6 +522,20 @@ def test_small_and_large_batches_agree(nes, gpu_ctx, prec, sigma):
             ctx.close()
 
 
+@pytest.mark.parametrize("prec", [FP32, MIXED])
+@pytest.mark.parametrize("w,h", [(641, 481), (320, 200), (721, 700)])
+def test_a_view_alone_and_in_a_batch_agree(nes, gpu_ctx, prec, w, h):
+    """Every output of a view, the FP32 colours among them, is the same alone
+    and in a batch large enough for the other march and composite kernels."""
+    views = [nes.camera(w, h, nes.orbit_camera(30.0 + 70.0 * i, 20.0), fov=25.0) for i in range(2)]
+    large = nes.camera(1024, 1024, nes.orbit_camera(10.0, 25.0), fov=70.0)
+    batch, _ = gpu_ctx.render(views + [large], precision=prec)
+    for v, b in zip(views, batch):
+        a = gpu_ctx.render(v, precision=prec)[0][0]
+        for k in a:
+            assert np.array_equal(a[k], b[k]), (k, int((a[k] != b[k]).sum()))
+
+
 @pytest.mark.parametrize("w,h", [(1100, 701), (1024, 1024)])
 def test_fp32_encode_shares_change_no_result(nes, gpu_ctx, w, h):
     """As the mixed path's, on the FP32 path's own line: shares of 1.6 to 25
