@@ -79,7 +79,7 @@ struct HostArray {
   uint8_t *dst;
   uint64_t bytes;
   uint32_t bpp, view;
-  uint32_t unit;  // bytes per store: 16, 4 or 1, what dst is aligned to
+  uint32_t head;  // bytes in front of dst's first multiple of 16
   float gray_scale;
 };
 constexpr uint32_t kHostArrays = 40;  // carried to the device as kernel arguments

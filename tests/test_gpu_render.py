@@ -430,6 +430,36 @@ def test_pinned_outputs_of_multi_pass_frames(nes, oracle, prec):
             assert np.array_equal(want[0][k], got[0][k]), k
 
 
+@pytest.mark.parametrize("w,h", [(1, 1), (2, 3), (5, 1), (17, 3), (641, 481)])
+@pytest.mark.parametrize("offset", [0, 1, 2, 7, 12, 15])
+def test_pinned_outputs_at_any_address(nes, gpu_ctx, w, h, offset):
+    """Arrays shorter than the bytes in front of their first 16-byte unit, of
+    no whole unit, and large ones (background stored during the encode) at
+    odd addresses: equal to the ones copied, and nothing beside them written."""
+    views = [nes.camera(w, h, nes.orbit_camera(30.0, 20.0, 2.0, e), fov=25.0) for e in (-0.032, 0.032)]
+    want = [{k: _render_pageable(nes, gpu_ctx, v, k) for k in ALL} for v in views]
+    got, _ = _pinned_render(nes, gpu_ctx, views, MIXED, ALL, offset)
+    assert all(a["depth"].max() > 0 for a in want)
+    for a, b in zip(want, got):
+        for k in ALL:
+            assert np.array_equal(a[k], b[k]), k
+
+
+def _render_pageable(nes, ctx, view, name):
+    """One array of a render into ordinary memory (copied by the runtime)."""
+    import ctypes as C
+    ch, dt, t, field = {"rgb24": (3, np.uint8, C.c_uint8, "rgb24"), "depth": (1, np.float32, C.c_float, "depth"),
+                        "rgb": (3, np.float32, C.c_float, "rgb_f32"),
+                        "n_samples": (1, np.uint16, C.c_uint16, "n_samples"),
+                        "depth_gray8": (1, np.uint8, C.c_uint8, "depth_gray8")}[name]
+    a = np.empty((view.height, view.width) + ((3,) if ch == 3 else ()), dt)
+    out = nes.ViewOut()
+    out.depth_far = 2.5
+    setattr(out, field, a.ctypes.data_as(C.POINTER(t)))
+    nes.check(nes.lib().nes_render(ctx.handle, MIXED, C.byref(view), 1, C.byref(out), 0, None), "nes_render")
+    return a
+
+
 @pytest.mark.parametrize("far", [float("inf"), 3e38, 1e-42, float("nan"), -1.0])
 @pytest.mark.parametrize("w,h,offset", [(640, 480, 0), (31, 17, 0), (31, 17, 1)])
 def test_gray8_of_any_far_distance(nes, oracle, gpu_ctx, w, h, offset, far):
