@@ -1568,43 +1568,59 @@ static size_t expected_samples(const RenderWork &w, int pass) {
   return std::min<size_t>(est, w.capacity);
 }
 
-// Shares of the mixed encode's first parts (see encode_parts): how far apart
-// neighbouring samples are, and with it what part 0 costs above part 7, follows
-// the focal length in pixels: 12 % at 416 (640x480 at 60 degrees), 52 % at 935
-// (1080p), 75 % at 1439 (2064x2208 at 75 degrees).  The shares start at 500
-// and reach 12, 9 and 4 % at 935, 21, 15 and 6 % from 1250 on.  Below 500 they
-// gain nothing.  One of them a fifth smaller or larger moves the encode by 2 %
-// at most; all three a fifth larger cost 1 to 5 %.
+// Shares of the encode's first parts (see encode_parts) by how far apart
+// neighbouring samples lie: distance over focal length, written as the focal
+// length in pixels of a view with the same spacing from 2 units off the cube's
+// centre.  (From inside, a ray's samples are 0.3 away in the mean.)  Encode
+// times below: two eyes (views of up to 10 degrees one), without shares -> with
+// them, us, frame after frame.
 //
-// In FP32 a hashed level fills an XCD's L2 by itself, part 0 is ahead of part 7
-// already at 416 and the shares are constant from 480 on, us, tables not in the
-// Infinity Cache: 640x480 stereo 382 -> 365, 720p stereo 753 -> 681, 1080p
-// stereo 1480 -> 1312; none up to 280 (640x480 at 75 degrees 225 -> 230).
+// Mixed: part 0 costs 12 % more than part 7 at 416 (640x480 at 60 degrees), 52 %
+// at 935 (1080p) and 75 % at 1439 (2064x2208 at 75 degrees), until neighbours
+// share the finest level's cells too.  The shares start at 500 (720p at 620:
+// 619 -> 610; 1440x1600 from 6 off at 348: 213 without, 240 with the shares of
+// 2 off), reach 12, 9 and 4 % at 935 (1293 -> 1234), stay at 21, 15 and 6 % from
+// 1250 to 3600 (1440x1600 from 1 off 7200 -> 5700, 2064x2208 from 0.8 off 18900 ->
+// 15600) and end at 9600 (2064x2208 from 0.6 off, 4797: 31700 -> 27600; 1080p
+// from 0.3 off, 6233: 15900 -> 14000, with 21 % 15300; 640x480 at 5 degrees
+// from 0.6 off, 18300: 1080, with 21 % 1200).
+//
+// FP32: a hashed level fills an XCD's L2 by itself; shares of 15, 10 and 5 %
+// gain from 485 on (at 425 1800x1700 loses, 433 -> 456; 900x800 at 521 632 ->
+// 618, 720p 879 -> 818, 1080p 1857 -> 1680, 640x480 of one eye from 0.3 off,
+// 2773, 1964 -> 1650), up to about 5000 (640x480 at 10 degrees: 3918 2020 -> 2009,
+// 5486 1690, with 15 % 1733, 9143 1396 -> 1666).
 // Between limits: of 1 M samples the helpers' extra 4 MB of table cost more
 // than they take off part 0 (640x480: 201 -> 204, the frame 535 -> 546); and
 // where the samples are more than twice the grid's threads its passes mix the
 // parts' turns and four such levels take turns in one L2 (26.7 M samples
 // 2690 -> 3100, 50.8 M 4280 -> 5460).
 constexpr size_t kF32ShareMin = 3u << 19, kF32ShareMax = 2 * 256 * (size_t)kMaxPartBlocks;
+constexpr double kShareEnd = 9600.0;
+
+static double spacing_focal(const ViewDesc &v) {
+  double d2 = 0.0;
+  for (int i = 0; i < 3; ++i) d2 += ((double)v.c2w[4 * i + 3] - 0.5) * ((double)v.c2w[4 * i + 3] - 0.5);
+  return 2.0 * v.focal / std::max(std::sqrt(d2), 0.3);
+}
 
 static PartShares part_shares(const RenderWork &w, bool f32, size_t expect) {
   double focal = 0.0;
   for (uint32_t i = 0; i < w.n_views; ++i)
-    focal += (double)w.host_views[i].focal * w.host_views[i].slot_count / w.n_slots;
+    focal += spacing_focal(w.host_views[i]) * w.host_views[i].slot_count / w.n_slots;
+  if (!(focal < kShareEnd)) return PartShares{};  // (nor for a camera that is not finite)
   const auto q = [](double v) { return (uint32_t)(std::max(v, 0.0) * 65536); };
   if (f32) {
     if (expect < kF32ShareMin || expect > kF32ShareMax) return PartShares{};
-    const double s = 0.15 * std::min((focal - 280.0) / 200.0, 1.0);
+    const double s = 0.15 * std::min({(focal - 470.0) / 130.0, (6000.0 - focal) / 2000.0, 1.0});
     return PartShares{{q(s), q(s - 0.05), q(s - 0.10)}, 0u};
   }
-  const double f = std::min(std::max((focal - 500.0) / 600.0, 0.0), 1.25);
+  const double f = std::min({std::max((focal - 500.0) / 600.0, 0.0), (kShareEnd - focal) / 4800.0, 1.25});
   return PartShares{{q(0.17 * f), q(0.12 * f), q(0.05 * f)}, 0u};
 }
 
-
 int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int k0, int k1,
                        bool first, bool last, hipStream_t stream, uint32_t ray_cap, bool resume) {
-  const unsigned blocks = (unsigned)((w.n_slots + 255) / 256);
   uint32_t *const total = w.total.as<uint32_t>();
   uint32_t *cursor = total + (first ? kTotCursor : kTotCursorLater);
   const uint32_t cap = w.capacity;

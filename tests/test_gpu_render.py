@@ -528,6 +528,24 @@ def test_encode_shares_change_no_result(nes, gpu_ctx, w, h):
 
 
 @pytest.mark.parametrize("prec", [FP32, MIXED])
+@pytest.mark.parametrize("radius", [0.0, 0.2, 0.45, 0.9, 6.0, 1e6, float("nan"), float("inf")])
+def test_encode_shares_of_any_eye(nes, gpu_ctx, prec, radius):
+    """The shares follow the eye's distance as well: a view beside one from
+    inside the cube, close to it, far off or from nowhere equals the same view
+    alone, and so does the other."""
+    v = nes.camera(643, 481, nes.orbit_camera(25.0, 15.0), fov=40.0)
+    c2w = np.array(nes.orbit_camera(60.0, 10.0), np.float32)
+    eye = c2w[3::4] - 0.5
+    c2w[3::4] = 0.5 + eye / np.linalg.norm(eye) * np.float32(radius)
+    other = nes.camera(320, 200, c2w, fov=50.0)
+    outs, _ = gpu_ctx.render([v, other], precision=prec)
+    for got, cam in zip(outs, (v, other)):
+        alone = gpu_ctx.render(cam, precision=prec)[0][0]
+        for k in alone:
+            assert np.array_equal(alone[k], got[k], equal_nan=alone[k].dtype.kind == "f"), k
+
+
+@pytest.mark.parametrize("prec", [FP32, MIXED])
 @pytest.mark.parametrize("sigma", [None, 30.0])
 def test_small_and_large_batches_agree(nes, gpu_ctx, prec, sigma):
     """Batches below 2^19 ray slots march with four lanes per ray, larger ones
