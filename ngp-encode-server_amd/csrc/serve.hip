@@ -144,6 +144,13 @@ static nes_frame_planes padded_planes(uint8_t *p, const nes_camera &c) {
   return f;
 }
 
+// Bytes of device staging per ray slot and stream, in sixteenths: YUV420P is
+// 24, and rows of 16 bytes take up to 27 of most views (1548 wide: 24.1) but
+// 64 of views 8 wide.
+constexpr size_t kStaging16 = 27;
+static size_t staging_bytes(uint64_t ray_slots) { return (size_t)(ray_slots * kStaging16 / 16); }
+static uint64_t view_slots(const nes_camera &c) { return (uint64_t)((c.width + 7) / 8) * ((c.height + 7) / 8) * 64; }
+
 // Tight YUV420P planes of a w x h frame starting at p.
 static nes_frame_planes tight_planes(uint8_t *p, const nes_camera &c) {
   nes_frame_planes f;
@@ -222,6 +229,19 @@ static size_t slot_bytes(uint32_t max_rays, int precision, bool depth) {
                          (depth ? 4 : 2);
   const size_t per_sample = 4 + sizeof(float4) + sizeof(float4) + feat * 8;  // 8 XCD part planes
   return (r * per_ray + cap * per_sample) / 8 * 9 + ((size_t)1 << 20);
+}
+
+// How a view's planes are staged: caller planes with padded rows where that
+// fits the view's part of the staging reserved for every slot (a buffer that
+// grew while serving would stall the device), tight otherwise.
+static bool staged_padded(const Request &rq, const nes_camera &c) {
+  return rq.caller && padded_bytes(c) <= staging_bytes(view_slots(c));
+}
+static size_t staged_bytes(const Request &rq, const nes_camera &c) {
+  return staged_padded(rq, c) ? padded_bytes(c) : yuv_bytes(c);
+}
+static nes_frame_planes staged_planes(const Request &rq, uint8_t *p, const nes_camera &c) {
+  return staged_padded(rq, c) ? padded_planes(p, c) : tight_planes(p, c);
 }
 
 // Device-to-host copy of one view's staged YUV420P planes into the request's
@@ -329,12 +349,12 @@ static int launch_output(nes_server *s, Slot &sl) {
   RenderWork &w = sl.work;
   const OutLayout L = out_layout(w.out_px);
   const bool depth = s->cfg.depth_stream != 0;
-  // where each request's staged planes start: tight, as its own planes are
-  // laid out, or with padded rows for caller planes
+  // A request's planes start on 16 bytes; they follow each other as its own
+  // planes do, or each view of caller planes starts on 16 bytes again.
   size_t yuv_total = 0;
   for (auto &rq : sl.reqs)
     for (int v = 0; v < rq->n_views; ++v)
-      yuv_total = pitch16(yuv_total) + (rq->caller ? padded_bytes(rq->views[v]) : yuv_bytes(rq->views[v])) * (depth ? 2 : 1);
+      yuv_total = pitch16(yuv_total) + staged_bytes(*rq, rq->views[v]) * (depth ? 2 : 1);
   NES_TRY(sl.yuv.reserve(yuv_total + 256));
   if (s->cfg.font && s->cfg.overlay_flags) {
     // the strings of every view, stamped by one launch before frame prep
@@ -364,7 +384,7 @@ static int launch_output(nes_server *s, Slot &sl) {
       const uint8_t *rgb = w.out.as<uint8_t>() + L.rgb24 + 3 * (size_t)vd.px_base;
       if (rq->caller || v == 0) off = pitch16(off);
       for (int st = 0; st < (depth ? 2 : 1); ++st) {
-        const nes_frame_planes d = rq->caller ? padded_planes(yuv + off, c) : tight_planes(yuv + off, c);
+        const nes_frame_planes d = staged_planes(*rq, yuv + off, c);
         if (st == 0)
           NES_TRY(launch_frameprep(rgb, nullptr, nullptr, nullptr, cw, ch, 1, 0, 0, d.data[0],
                                    d.linesize[0], 0, d.data[1], d.linesize[1], 0, d.data[2],
@@ -373,7 +393,7 @@ static int launch_output(nes_server *s, Slot &sl) {
           NES_TRY(launch_depth_yuv(reinterpret_cast<const float *>(w.out.as<uint8_t>() + L.depth) + vd.px_base,
                                    cw, ch, scale, nullptr, d.data[0], d.linesize[0], d.data[1],
                                    d.linesize[1], d.data[2], d.linesize[2], s->cfg.sws_mode, sl.stream));
-        off += rq->caller ? padded_bytes(c) : yuv_bytes(c);
+        off += staged_bytes(*rq, c);
       }
     }
   }
@@ -383,8 +403,8 @@ static int launch_output(nes_server *s, Slot &sl) {
   off = 0;
   std::vector<RowCopy> rows;
   for (auto &rq : sl.reqs) {
-    off = pitch16(off);
     if (!rq->caller) {
+      off = pitch16(off);
       size_t bytes = 0;
       for (int v = 0; v < rq->n_views; ++v) bytes += yuv_bytes(rq->views[v]) * (depth ? 2 : 1);
       NES_HIP_TRY(hipMemcpyAsync(rq->yuv.ptr, yuv + off, bytes, hipMemcpyDeviceToHost, sl.stream));
@@ -393,8 +413,9 @@ static int launch_output(nes_server *s, Slot &sl) {
     }
     for (int v = 0; v < rq->n_views; ++v) {
       const nes_camera &c = rq->views[v];
+      off = pitch16(off);
       for (int st = 0; st < (depth ? 2 : 1); ++st) {
-        const nes_frame_planes src = padded_planes(yuv + off, c);
+        const nes_frame_planes src = staged_planes(*rq, yuv + off, c);
         const nes_frame_planes &dst = st ? rq->dplanes[v] : rq->planes[v];
         if (rq->row_kernel)
           for (int p = 0; p < 3; ++p)
@@ -403,7 +424,7 @@ static int launch_output(nes_server *s, Slot &sl) {
                                     p ? c.height / 2 : c.height));
         else
           NES_TRY(copy_planes(dst, src, c, sl.stream));
-        off += padded_bytes(c);
+        off += staged_bytes(*rq, c);
       }
     }
   }
@@ -743,8 +764,7 @@ int nes_server_create(nes_ctx *ctx, const nes_server_config *cfg, nes_server **o
       if (per_slot <= sl.work.budget) {
         NES_TRY(render_work_reserve(sl.work, s->cfg.max_batch_rays, s->cfg.max_batch_rays,
                                     kPinnedViews, s->cfg.precision));
-        // YUV420P is 1.5 bytes per pixel, twice with the depth stream
-        NES_TRY(sl.yuv.reserve((size_t)s->cfg.max_batch_rays * 3 / 2 * (depth ? 2 : 1) + 256));
+        NES_TRY(sl.yuv.reserve(staging_bytes(s->cfg.max_batch_rays) * (depth ? 2 : 1) + 256));
       }
     }
     return NES_OK;

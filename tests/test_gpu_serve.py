@@ -286,3 +286,68 @@ def test_caller_planes_of_any_alignment_match_server_planes(nes, gpu_ctx, w, h, 
             assert got.padding_intact()
         for p in planes + dplanes:
             p.free()
+
+
+@pytest.mark.parametrize("depth", [False, True])
+def test_staging_of_a_full_batch_is_reserved(nes, gpu_ctx, depth):
+    """A full batch of views 8 pixels wide, whose rows padded to 16 bytes would
+    take 2.7 times their size: no device memory is allocated while serving."""
+    import ctypes as C
+
+    def free_bytes():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert nes.lib().hipMemGetInfo(C.byref(a), C.byref(b)) == 0  # (of the library's runtime)
+        return a.value
+
+    n = 16  # stereo requests of 2 x 131072 ray slots
+    with nes.Server(gpu_ctx, max_batch_rays=n << 18, max_inflight=1, depth_stream=depth) as srv:
+        kw = dict(depth=True) if depth else {}
+        # (170 degrees: the cube covers a few hundred of the 16384 rows)
+        views = [[nes.camera(8, 16384, nes.orbit_camera(20.0 * i, 15.0, 2.0, e), fov=170.0, index=i,
+                             is_left=int(e < 0)) for e in (-0.03, 0.03)] for i in range(n)]
+        frames = lambda: [nes.HostPlanes(8, 16384, 32) for _ in range(2)]  # noqa: E731
+        planes, dplanes = [frames() for _ in range(n)], [frames() if depth else None for _ in range(n)]
+        want = srv.wait(srv.submit(0, views[3]), **kw)
+        assert want[0] == 0
+        before = free_bytes()
+        srv.hold(True)
+        tickets = [srv.submit_into(i, views[i], planes[i], dplanes[i]) for i in range(n)]
+        srv.hold(False)
+        for t in tickets:
+            assert srv.wait(t, **kw)[0] == 0
+        assert srv.stats().batches == 2
+        assert before - free_bytes() < 1 << 20
+        for got, ref in zip(planes[3] + (dplanes[3] or []), list(want[1]) + (list(want[2]) if depth else [])):
+            for g, r in zip(got.yuv(), ref):
+                assert np.array_equal(g, r)
+            assert got.padding_intact()
+        for f in sum(planes + [d for d in dplanes if d], []):
+            f.free()
+
+
+@pytest.mark.parametrize("pageable", [False, True])
+def test_caller_planes_of_mixed_widths_in_one_batch(nes, gpu_ctx, pageable):
+    """Views staged with padded rows and with tight ones (narrow ones), of
+    requests with the server's planes and with the caller's, side by side."""
+    sizes = [(2, 2), (98, 34), (8, 16), (258, 66), (40, 24), (774, 50), (6, 8), (106, 18)]
+    make = (lambda w, h: _Pageable(nes, w, h, 32)) if pageable else (lambda w, h: nes.HostPlanes(w, h, 32))
+    with nes.Server(gpu_ctx, max_batch_rays=1 << 20, depth_stream=True) as srv:
+        views = [stereo(nes, w, h, 30.0 * i, index=i) for i, (w, h) in enumerate(sizes)]
+        want = [srv.wait(srv.submit(i, v), depth=True) for i, v in enumerate(views)]
+        planes = [[make(*s) for _ in range(2)] for s in sizes]
+        dplanes = [[make(*s) for _ in range(2)] for s in sizes]
+        srv.hold(True)
+        into = [srv.submit_into(2 * i, v, planes[i], dplanes[i]) for i, v in enumerate(views)]
+        own = [srv.submit(2 * i + 1, v) for i, v in enumerate(views)]
+        srv.hold(False)
+        for i in range(len(sizes)):
+            assert srv.wait(into[i], depth=True)[0] == 0
+            rc, y, d, _ = srv.wait(own[i], depth=True)
+            assert rc == 0
+            got = [p.yuv() for p in planes[i] + dplanes[i]]
+            for a, b, c in zip(got, list(y) + list(d), list(want[i][1]) + list(want[i][2])):
+                for p, q, r in zip(a, b, c):
+                    assert np.array_equal(p, r) and np.array_equal(q, r), sizes[i]
+            assert all(p.padding_intact() for p in planes[i] + dplanes[i])
+        for p in sum(planes + dplanes, []):
+            p.free()
