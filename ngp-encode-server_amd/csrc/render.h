@@ -119,8 +119,9 @@ struct RenderWork {
   // samples the first pass gives each ray (kMaxSteps = one single pass).
   uint32_t first_pass_cap = kMaxSteps;
   uint32_t frame_passes = 1;      // passes the last frame launched
-  // Samples of the work area's last frame, first and later pass (0: none yet):
-  // sizes the launches of the next one, whose own count stays on the device.
+  bool whole_frame = false;       // its first pass walked all steps without a capacity's limit
+  // Samples of the work area's last whole frame, first and later pass (0: none
+  // yet): sizes the launches of the next one, whose own count stays on the device.
   uint32_t last_total[2] = {0, 0};
 };
 

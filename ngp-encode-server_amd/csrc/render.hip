@@ -1682,6 +1682,7 @@ int render_launch_pass(const SceneDev &scene, RenderWork &w, int precision, int 
 }
 
 int render_launch_frame(const SceneDev &scene, RenderWork &w, int precision, hipStream_t stream) {
+  w.whole_frame = true;
   NES_TRY(render_begin(w, stream));
   const uint32_t cap1 = w.first_pass_cap;
   if (cap1 >= (uint32_t)kMaxSteps) {
@@ -1719,6 +1720,7 @@ int render_launch_bounded(const SceneDev &scene, RenderWork &w, int precision,
                                           kMaxSteps);
   const int passes = (int)((kMaxSteps + cap - 1) / cap);
   w.frame_passes = (uint32_t)passes;
+  w.whole_frame = false;
   NES_TRY(render_begin(w, stream));
   for (int p = 0; p < passes; ++p) {
     if (p > 1) NES_TRY(clear_later_cursor(w, stream));
@@ -1751,9 +1753,9 @@ size_t sample_buffer_bytes(size_t capacity, int precision) {
 FrameCounts render_frame_finish(RenderWork &w) {
   FrameCounts c;
   c.passes = w.frame_passes;
-  // frames in more passes (bounded, windows) say nothing about a whole one
-  w.last_total[0] = c.passes <= 2 ? w.total_host[kTotCursor] : 0u;
-  w.last_total[1] = c.passes == 2 ? w.total_host[kTotCursorLater] : 0u;
+  // the passes of other frames (bounded, windows) say nothing about a whole one
+  w.last_total[0] = w.whole_frame ? w.total_host[kTotCursor] : 0u;
+  w.last_total[1] = w.whole_frame && c.passes == 2 ? w.total_host[kTotCursorLater] : 0u;
   c.evaluated = w.total_host[2];
   for (int s = 0; s < kTotTermSlots; ++s) {
     const uint32_t *t = w.total_host + kTotTermBase + kTotTermStride * s;
@@ -1950,6 +1952,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
     const int spp = steps_per_pass;
     const int passes = (kMaxSteps + spp - 1) / spp;
     w.frame_passes = 1;
+    w.whole_frame = false;
     for (int p = 0; p < passes; ++p) {
       const int k0 = p * spp, k1 = std::min(kMaxSteps, k0 + spp);
       uint32_t n = 0;
