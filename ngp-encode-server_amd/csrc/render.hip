@@ -1910,7 +1910,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
   NES_TRY(render_prepare_capacity(w, precision));
   NES_TRY(check_budget(w));
   double t[4] = {0, 0, 0, 0};  // march, encode, MLPs, composite
-  double total = 0;
+  double total = 0, lost = 0;  // (lost: launches that overflowed)
   FrameCounts fc;
   if (steps_per_pass == 0 || steps_per_pass >= kMaxSteps) {
     // whole frame: one pass, or two when the previous frame of this work area
@@ -1930,6 +1930,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
         set_last_error("sample capacity still exceeded after regrowth");
         return NES_ENOMEM;
       }
+      lost += frame_ms(w);
       // grow when the budget and the device allow it, else render within the
       // buffers (the first of two passes has stored background already: the
       // frame is not given up here)
@@ -1970,6 +1971,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
           set_last_error("sample capacity still exceeded after regrowth");
           return NES_ENOMEM;
         }
+        if (p == 0) lost += frame_ms(w);  // (later passes run on the first one's clock)
         const size_t want = (size_t)n + n / 8 + 1024;
         if (!render_growth_fits(w, precision, want)) {
           set_last_error("a pass's samples exceed the context's HBM budget");
@@ -1986,7 +1988,7 @@ static int render_enqueue_inner(const SceneDev &scene, RenderWork &w, int precis
   if (stats) {
     stats->rays = w.pixels;
     stats->samples = fc.evaluated;
-    stats->ms_total = total;
+    stats->ms_total = total + lost;
     stats->ms_march = t[0];
     stats->ms_encode = t[1];
     stats->ms_mlp = t[2];

@@ -474,6 +474,22 @@ def test_gray8_of_any_far_distance(nes, oracle, gpu_ctx, w, h, offset, far):
     assert np.array_equal(o["depth_gray8"], want)
 
 
+@pytest.mark.parametrize("windows", [0, 64])
+def test_ms_total_holds_launches_that_overflowed(nes, scene1, windows):
+    """ms_total is the device time of the whole render: of a frame that
+    outgrows its buffers (about 15 samples per ray slot for 4 of capacity) also
+    the launch that was run again, which the stage times leave out."""
+    t, w, _ = scene1
+    occ = np.full(nes.OCC_WORDS, 0xffffffff, np.uint32)
+    cam = nes.camera(1024, 1024, nes.orbit_camera(30.0, 20.0), fov=60.0)
+    with nes.Context(t, w, occ) as ctx:
+        first, later = [ctx.render_device(cam, MIXED, windows) for _ in range(2)]
+    stages = [x.ms_march + x.ms_encode + x.ms_mlp + x.ms_composite for x in (first, later)]
+    assert first.samples == later.samples > 8 << 20
+    assert first.ms_total > 1.15 * stages[0]
+    assert windows or later.ms_total < 1.1 * stages[1]
+
+
 def test_returned_arrays_are_the_callers(nes, gpu_ctx):
     """Arrays of earlier renders keep their values through later ones (their
     memory is reused only once they are gone)."""
