@@ -74,14 +74,6 @@ __device__ __forceinline__ uint32_t occ_cell(const float x128[3]) {
 }
 static_assert(kOccRes == 1 << 7, "cell index");
 
-__device__ __forceinline__ void step_pos(const RayData &r, int k, float x[3],
-                                         float *t) {
-  const float tt = step_t(k, r.t_start);
-#pragma unroll
-  for (int a = 0; a < 3; ++a) x[a] = fmaf(tt, r.d[a], r.o[a]);
-  *t = tt;
-}
-
 __device__ __forceinline__ RayData load_ray(const RayData *rays, uint32_t slot) {
   const float4 *p = reinterpret_cast<const float4 *>(rays + slot);
   const float4 a = p[0], b = p[1];
@@ -96,17 +88,18 @@ __device__ __forceinline__ RayData load_ray(const RayData *rays, uint32_t slot) 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 
 // ------------------------------------------------- rank-major sample list
-// The samples of one wavefront's 64 ray slots (one 8x8 pixel tile) occupy
-// one contiguous range of the sample list, reserved with a single atomic.
+// The samples of a tile's 64 ray slots (8x8 pixels) occupy one contiguous
+// range of the sample list, reserved with one atomic per workgroup.
 // Inside it they are ordered by rank: first the first occupied sample of
 // every ray that has one (in lane order), then every second sample, and so
 // on.  Rank i of lane l sits at
 //   base + sum_{r<i} |{lanes with count > r}| + |{lanes < l with count > i}|.
 // Neighbouring lanes of the encode and MLP kernels thus see samples of
 // neighbouring pixels at similar depths (their table gathers share cache
-// lines), and a ray's samples are still visited in march order.  Every
-// kernel that walks the list by ray runs one lane per slot with
-// slot = 64 * wavefront + lane and keeps all 64 lanes in the loop.
+// lines), and a ray's samples are still visited in march order.  Kernels that
+// walk the list by ray run one lane per slot with slot = 64 * wavefront + lane
+// and keep all 64 lanes in the loop, or a workgroup of four wavefronts per
+// tile with four lanes per ray (index_ranks).
 __device__ __forceinline__ uint64_t lanes_below(int lane) {
   return lane ? (~0ull >> (64 - lane)) : 0ull;
 }

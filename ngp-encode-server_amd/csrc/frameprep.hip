@@ -159,7 +159,8 @@ VFilter build_vchroma_filter(int h) {
 
 namespace {
 std::mutex g_filter_mu;
-std::map<int, VRows> g_filters;  // by frame height (at most 8192 of them)
+std::map<int, VRows> g_filters;  // by frame height
+constexpr size_t kMaxFilters = 8192;
 }  // namespace
 
 int get_vrows(int h, VRows *out) {
@@ -186,6 +187,7 @@ int get_vrows(int h, VRows *out) {
       set_last_error("unsupported vertical filter size");
       return NES_ERANGE;
     }
+    if (g_filters.size() >= kMaxFilters) g_filters.clear();
     it = g_filters.emplace(h, r).first;
   }
   *out = it->second;

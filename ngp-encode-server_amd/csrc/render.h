@@ -165,11 +165,13 @@ OutLayout out_layout(size_t px);
 // Stages of one render:
 //   render_setup            views -> ray-slot layout, ray buffers, view upload
 //   render_prepare_capacity sample buffers for the expected sample count
+//   render_begin            counters cleared, views uploaded
 //   render_launch_pass      march_emit, encode, MLP, composite for march steps
-//                           [k0, k1), then an async copy of the pass's sample
-//                           total into work.total_host[0].  A total above
-//                           work.capacity means the pass was dropped: grow with
-//                           render_reserve_samples and launch the pass again.
+//                           [k0, k1)
+//   render_end              counters and outputs stored on the host's side.  A
+//                           pass's total above work.capacity means the pass was
+//                           dropped: grow with render_reserve_samples and
+//                           launch it again.
 int render_setup(RenderWork &w, const nes_camera *views, int n_views, hipStream_t stream);
 int render_prepare_capacity(RenderWork &w, int precision);
 int render_reserve_samples(RenderWork &w, int precision, size_t capacity);

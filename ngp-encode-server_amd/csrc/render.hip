@@ -5,9 +5,10 @@
 //
 // Pipeline per pass (a pass covers a window of march steps; one pass of 128
 // steps is the default):
-//   march_emit    one thread per ray slot: camera ray, box clip, occupied
-//                 steps; a wave scan + one atomic per wavefront reserves a
-//                 contiguous segment of the sample list on the device
+//   march_emit    one thread per ray slot (march_emit_split: four, for few
+//                 rays): camera ray, box clip, occupied steps; one atomic per
+//                 workgroup reserves a contiguous segment of the sample list
+//                 on the device, one part per wavefront's tile
 //   encode_parts  16-level hash-grid encoding, XCD-partitioned: workgroups on
 //                 XCD p encode levels p and 15-p, so each XCD's L2 caches two
 //                 levels of the table
@@ -16,8 +17,11 @@
 //                          v_mfma_f32_16x16x4_f32
 //                   mixed: mlp_mixed, FP16 features on
 //                          v_mfma_f32_16x16x32_f16, FP32 accumulation
-//   composite     one thread per ray: front-to-back alpha compositing in FP32,
-//                 stops at T < 1e-4, writes RGB24 / depth / float RGB
+//   composite     one thread per ray (composite_split: four, for few rays):
+//                 front-to-back alpha compositing in FP32, stops at T < 1e-4,
+//                 writes RGB24 / depth / float RGB
+// frame_begin clears the frame's counters, frame_end stores them, and outputs
+// wanted in pinned memory, on the host's side.
 // Both precisions share every kernel except the table type in encode_parts,
 // the MLP kernel and the width of the MLP output, so their throughput ratio
 // isolates those; both MLPs run on matrix cores.  The sample
