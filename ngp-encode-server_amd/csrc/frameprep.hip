@@ -198,6 +198,10 @@ int get_vrows(int h, VRows *out) {
 constexpr int kFpQuads = 64;    // 4-pixel quads per tile row, one per lane
 constexpr int kFpWaves = 4;
 constexpr int kFpXcds = 8;      // workgroup b runs on XCD b % 8
+// Workgroups in a row of the grid.  One dimension of a launch holds fewer than
+// 2^32 threads; tens of thousands of narrow frames have more tiles than that.
+constexpr uint32_t kFpGridRow = 1u << 23;
+static_assert(kFpGridRow % kFpXcds == 0, "a row starts on XCD 0");
 
 struct FrameprepArgs {
   const uint8_t *rgb_a;
@@ -356,7 +360,7 @@ __global__ __launch_bounds__(64 * kFpWaves) void frameprep_kernel(FrameprepArgs 
   __shared__ int16_t edge_coef[kVClasses * kVTaps];
   const uint32_t total = a.strips * a.tiles * a.frames;
   // runs of a.run tiles, dealt to the XCDs in turn
-  const uint32_t block = blockIdx.y * gridDim.x + blockIdx.x, turn = block / kFpXcds;
+  const uint32_t block = blockIdx.y * kFpGridRow + blockIdx.x, turn = block / kFpXcds;
   const uint32_t id = (turn / a.run * kFpXcds + block % kFpXcds) * a.run + turn % a.run;
   if (id >= total) return;
   const uint32_t strip = id % a.strips, tile = id / a.strips % a.tiles, f = id / a.strips / a.tiles;
@@ -512,11 +516,6 @@ static int frameprep_rows(int w, int h, int n_frames) {
 constexpr size_t kBulkBytes = (size_t)256 << 20;
 
 constexpr uint32_t kFpRunRows = 6;  // tile rows per run
-
-// Workgroups in a row of the grid.  One dimension of a launch holds fewer than
-// 2^32 threads; tens of thousands of narrow frames have more tiles than that.
-constexpr uint32_t kFpGridRow = 1u << 23;
-static_assert(kFpGridRow % kFpXcds == 0, "a row starts on XCD 0");
 
 template <int kCRows, FrameClass kClass>
 static void frameprep_launch(FrameprepArgs &a, bool two, hipStream_t stream) {
