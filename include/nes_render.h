@@ -107,7 +107,9 @@ int nes_ctx_update_scene(nes_ctx *ctx, const nes_scene_desc *scene);
  * carries (proto/nes.proto:24, consumed as AV_PIX_FMT_GRAY8 at
  * src/server.cpp:193-194): g = clamp(floor(fma(d, 255 / depth_far, 0.5)), 0,
  * 255) in FP32, NaN -> 0, computed on the device; depth_far <= 0 selects
- * NES_DEPTH_FAR_DEFAULT. */
+ * NES_DEPTH_FAR_DEFAULT.  Arrays in pinned memory (nes_host_alloc), at any
+ * address, are stored by the render itself while it runs; others are copied
+ * after it. */
 #define NES_DEPTH_FAR_DEFAULT 4.0f
 typedef struct nes_view_out {
   uint8_t *rgb24;
@@ -363,8 +365,9 @@ typedef struct nes_server_config {
 /* Caller-owned YUV420P planes of one frame: an encoder frame's data[0..2]
  * and linesize[0..2] (e.g. an AVFrame from av_image_alloc with align 32,
  * src/base/video/type_managers.cc:116-141).  The server copies the device
- * planes straight into them (no staging copy); memory from nes_host_alloc is
- * pinned, so those copies are DMA transfers. */
+ * planes straight into them (no staging copy on the host); into pinned memory
+ * (nes_host_alloc) by DMA, or by stores of the GPU where the planes' rows are no
+ * whole words. */
 typedef struct nes_frame_planes {
   uint8_t *data[3];
   int32_t linesize[3];
